@@ -388,7 +388,7 @@ static void balanced_ranges(const std::vector<int64_t> &w, const std::vector<int
 Batch::~Batch() {
     drop_graph();
     for (auto e : ev_pool_) (void)hipEventDestroy(e);
-    d_bd_.release(); d_tiles_.release(); d_order_.release();
+    d_bd_.release(); d_runs_.release(); d_order_.release();
     for (auto &c : d_conv_) c.release();
     d_red_.release(); d_list_.release(); d_bw_.release();
     d_tmp_tiles_.release(); d_tmp_list_.release(); d_ranges_.release();
@@ -442,7 +442,7 @@ hm_status Batch::build_tables() {
         if (!used_[i] || !q.active) continue;
         q.d.tile_begin = (int32_t)tiles.size();
         for (int t = 0; t < q.d.ntiles; ++t) tiles.push_back((int32_t)i);
-        if ((q.d.flags & kPhysMask) != kStdFlags) std_only_ = false;
+        if ((q.d.flags & kPhysMask) != kStdFlags || q.d.nbins < 2) std_only_ = false;
         if (q.d.flags & F_WAKE) pass_lds_ = std::max(pass_lds_, (size_t)pass_lds_bytes(q.d));
         // the whole bin phase in one workgroup (k_bin_whole) for a small bunch
         // without interpolation sums; the other bunches take a launch per phase
@@ -531,15 +531,36 @@ hm_status Batch::build_tables() {
     balanced_ranges(winterp, nullptr, tiles, interp_grid_, ranges);
     deal_tiles(tiles, ranges.data(), pass_grid_, order);
     deal_tiles(tiles, ranges.data() + pass_grid_ + 1, interp_grid_, order);
+    // each workgroup's entries as runs of one bunch, a bunch with the deposit
+    // at most cic_tiles at a time; then `ranges` counts runs instead of tiles
+    std::vector<RunDev> runs;
+    auto find_runs = [&](size_t r0, int grid, size_t base) {
+        for (int g = 0; g <= grid; ++g) {
+            const int32_t e0 = g < grid ? ranges[r0 + (size_t)g] : 0;
+            const int32_t e1 = g < grid ? ranges[r0 + (size_t)g + 1] : 0;
+            ranges[r0 + (size_t)g] = (int32_t)runs.size();
+            for (int32_t e = e0; e < e1;) {
+                const int32_t b = tiles[(size_t)order[base + (size_t)e]];
+                const BunchDev &d = rb_[(size_t)b].d;
+                const int32_t em = (d.flags & F_CIC) ? e + std::min(e1 - e, d.cic_tiles) : e1;
+                int32_t ee = e + 1;
+                while (ee < em && tiles[(size_t)order[base + (size_t)ee]] == b) ++ee;
+                runs.push_back({b, (int32_t)base + e, ee - e});
+                e = ee;
+            }
+        }
+    };
+    if (pass_grid_ > 0) find_runs(0, pass_grid_, 0);
+    if (interp_grid_ > 0) find_runs((size_t)pass_grid_ + 1, interp_grid_, (size_t)ntiles_);
     // one staging round for every table and the descriptors
     size_t bytes = stage_size(ranges.size() * 4) + stage_size(list.size() * 4) +
                    stage_size(bw.size() * 4) +
-                   stage_size(red.size() * 4) + stage_size(tiles.size() * 4) +
+                   stage_size(red.size() * 4) + stage_size(runs.size() * sizeof(RunDev)) +
                    stage_size(order.size() * 4) +
                    stage_size(rb_.size() * sizeof(BunchDev));
     for (int k = 0; k < kConvKinds; ++k) bytes += stage_size(conv[k].size() * 4);
     HM_TRY(d_ranges_.ensure(std::max<size_t>(ranges.size(), 1)));
-    HM_TRY(d_tiles_.ensure(std::max<size_t>(tiles.size(), 1)));
+    HM_TRY(d_runs_.ensure(std::max<size_t>(runs.size(), 1)));
     HM_TRY(d_order_.ensure(std::max<size_t>(order.size(), 1)));
     HM_TRY(d_red_.ensure(std::max<size_t>(red.size(), 2)));
     HM_TRY(d_list_.ensure(std::max<size_t>(list.size(), 1)));
@@ -555,7 +576,7 @@ hm_status Batch::build_tables() {
     HM_TRY(stage_copy(ctx_, d_red_.p, red.data(), red.size() * 4));
     for (int k = 0; k < kConvKinds; ++k)
         HM_TRY(stage_copy(ctx_, d_conv_[k].p, conv[k].data(), conv[k].size() * 4));
-    HM_TRY(stage_copy(ctx_, d_tiles_.p, tiles.data(), tiles.size() * 4));
+    HM_TRY(stage_copy(ctx_, d_runs_.p, runs.data(), runs.size() * sizeof(RunDev)));
     HM_TRY(stage_copy(ctx_, d_order_.p, order.data(), order.size() * 4));
     HM_TRY(stage_descriptors());
     HM_TRY(stage_end(ctx_));
@@ -851,7 +872,8 @@ hm_status Batch::add_slots(const std::vector<RunBunch> &specs, std::vector<int32
         // sums' second read of z.  The counters hold any bunch of fewer than
         // 2^32 particles; a single bin has no cells.
         d.flags &= ~F_CIC;
-        if ((d.flags & F_E0) && !(d.flags & F_GHIST) && nb >= 2 && d.n < ((int64_t)1 << 32) &&
+        d.cic_tiles = (int32_t)(kCicRunPairs / d.pairs_per_tile);
+        if ((d.flags & F_E0) && d.cic_tiles >= 1 && !(d.flags & F_GHIST) && nb >= 2 && d.n < ((int64_t)1 << 32) &&
             (int64_t)pass_hist_bytes(d) + 8 * nb + cic_bytes((int)nb) <=
                 (int64_t)ctx_->lds_max - 1024)
             d.flags |= F_CIC;
@@ -948,7 +970,7 @@ hm_status Batch::one_turn() {
         ev_used_ += 3;
         HIP_TRY(hipEventRecord(e0, s));
     }
-    HIP_TRY(launch_turn_pass(d_bd_.p, d_tiles_.p, d_order_.p, d_ranges_.p, pass_grid_, pass_lds_,
+    HIP_TRY(launch_turn_pass(d_bd_.p, d_order_.p, d_runs_.p, d_ranges_.p, pass_grid_, pass_lds_,
                              std_only_ ? 1 : 0, s));
     if (timing_) HIP_TRY(hipEventRecord(e1, s));
     HIP_TRY(launch_bin_whole(d_bd_.p, d_bw_.p, nbw_, bw_lds_, s));
@@ -966,9 +988,8 @@ hm_status Batch::one_turn() {
     }
     if (timing_) HIP_TRY(hipEventRecord(e2, s));
     if (any_wake_e0_)   // two workgroups per CU when both windows fit the LDS
-        HIP_TRY(launch_interp_sum(d_bd_.p, d_tiles_.p, d_order_.p + ntiles_, d_ranges_.p + pass_grid_ + 1,
-                                  interp_grid_,
-                                  interp_lds_, interp_deep_, s));
+        HIP_TRY(launch_interp_sum(d_bd_.p, d_order_.p, d_runs_.p, d_ranges_.p + pass_grid_ + 1,
+                                  interp_grid_, interp_lds_, interp_deep_, s));
     HIP_TRY(whole ? launch_finalize_whole(d_bd_.p, d_list_.p, nlist_, s)
                   : launch_finalize(d_bd_.p, d_red_.p, nred_, s));
     return HM_OK;

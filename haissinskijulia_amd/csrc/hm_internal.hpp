@@ -232,9 +232,11 @@ class Batch {
     std::vector<RunBunch> rb_;
     std::vector<bool> used_;
     DevBuf<BunchDev> d_bd_;
-    DevBuf<int32_t> d_tiles_, d_order_, d_tmp_tiles_, d_tmp_list_;
-    // per-workgroup tile ranges of the pass and the interpolation sums,
-    // [pass_grid_ + 1] then [interp_grid_ + 1] entries, balanced by pairs
+    DevBuf<int32_t> d_order_, d_tmp_tiles_, d_tmp_list_;
+    // the runs of the pass's and the interpolation sums' workgroups, balanced
+    // by pairs, and each workgroup's first run, [pass_grid_ + 1] then
+    // [interp_grid_ + 1] entries
+    DevBuf<RunDev> d_runs_;
     DevBuf<int32_t> d_ranges_;
     int pass_grid_ = 0, interp_grid_ = 0;
     bool interp_deep_ = false;   // one interpolation workgroup per CU: deeper rings

@@ -112,7 +112,9 @@ struct Flags {
 };
 
 // Philox4x32-10 (Salmon et al., SC'11); the 32x32 -> 64 products give the
-// high and low words in one multiply
+// high and low words in one multiply.  Forced inline: with constant or
+// wave-uniform counter words the first rounds' products are scalar or leave
+// the loop.
 __device__ __forceinline__ void philox4x32_10(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3,
                                               uint32_t k0, uint32_t k1, uint32_t x[4]) {
 #pragma unroll
@@ -152,13 +154,25 @@ __device__ __forceinline__ double bm_radius(double x) {
 
 // Box-Muller (1958) on one Philox block: u1 in (0,1], u2 in [0,1), 53 bits each
 __device__ __forceinline__ void box_muller(const uint32_t x[4], double &n0, double &n1) {
-    const double u1 = ((double)(x[0] >> 5) * 67108864.0 + (double)(x[1] >> 6) + 1.0) * 0x1p-53;
-    const double u2 = ((double)(x[2] >> 5) * 67108864.0 + (double)(x[3] >> 6)) * 0x1p-53;
+    // (a 2^26 + b + 1) 2^-53 and (a 2^26 + b) 2^-53, every step exact
+    const double u1 = __builtin_fma((double)(x[0] >> 5), 0x1p-27,
+                                    __builtin_fma((double)(x[1] >> 6), 0x1p-53, 0x1p-53));
+    const double u2 = __builtin_fma((double)(x[2] >> 5), 0x1p-27, (double)(x[3] >> 6) * 0x1p-53);
     const double r = bm_radius(-2.0 * fm::log_pos<DevOps>(u1));
     double s, c;
     fm::sincos_reduced(kTwoPi * u2, s, c);
     n0 = r * c;
     n1 = r * s;
+}
+
+// QE normals of particle pair p < 2^32 at absolute turn t (a bunch has fewer
+// than 2^31 pairs): the counter's second word is the constant 0, which makes
+// one product of the second round uniform too
+__device__ __forceinline__ void qe_pair_normals32(uint64_t seed, uint32_t p, uint32_t t, double &n0,
+                                                  double &n1) {
+    uint32_t x[4];
+    philox4x32_10(p, 0u, t, 0u, (uint32_t)seed, (uint32_t)(seed >> 32), x);
+    box_muller(x, n0, n1);
 }
 
 // QE normals of particle pair p at absolute turn t
@@ -189,10 +203,11 @@ __device__ __forceinline__ void qe_pair_normals(uint64_t seed, uint64_t p, uint3
 // cloud-in-cell deposit counts a NaN z apart).
 __device__ __forceinline__ void interp_index_pass(double z, double c0, double u1, double inv,
                                                   int nb, int &k, double &w) {
-    const double u = __builtin_fmin(__builtin_fmax((z - c0) * inv, 0.0), u1);
-    const double fu = floor(u);
-    k = min((int)fu, nb - 2);
-    w = u - fu;
+    const double v = __builtin_fmax((z - c0) * inv, 0.0);
+    double u;   // fmin without a canonicalised copy of u1 (v is an arithmetic result, u1 finite)
+    asm("v_min_f64 %0, %1, %2" : "=v"(u) : "v"(v), "s"(u1));
+    k = min((int)u, nb - 2);           // truncation: u >= 0
+    w = __builtin_amdgcn_fract(u);     // u - floor(u), exact
 }
 __device__ __forceinline__ void interp_index(double z, double c0, double c1, double inv, int nb,
                                              int &k, double &w) {
@@ -532,6 +547,7 @@ typedef double f64x2 __attribute__((ext_vector_type(2)));
 typedef __attribute__((address_space(1))) double g_f64;
 typedef __attribute__((address_space(1))) f64x2 g_f64x2;
 typedef __attribute__((address_space(1))) uint32_t g_u32;
+typedef __attribute__((address_space(1))) uint8_t g_u8;
 typedef __attribute__((address_space(1))) unsigned long long g_u64;
 
 __device__ __forceinline__ double2 ld2(const g_f64x2 *a) {
@@ -567,12 +583,14 @@ __device__ __forceinline__ uint8_t *pass_lds() {
     return s_lds;
 }
 
-// LH: the histogram is in LDS (else straight to global memory)
-template <bool LH>
-__device__ __forceinline__ void bin_and_sum(const PassCtx &c, g_u32 *ghist, double z,
+// LH: the histogram is in LDS (else straight to global memory).  v[3] counts
+// the particles that are not binned (a branch most waves skip), n_bad (CIC
+// only) the NaN positions among them, one atomic each.
+template <bool LH, bool CIC>
+__device__ __forceinline__ void bin_and_sum(const PassCtx &c, g_u32 *ghist, g_u32 *n_bad, double z,
                                             double (&v)[4]) {
     v[0] += z;
-    v[1] += z * z;
+    v[1] = __builtin_fma(z, z, v[1]);
     // hist_bin with its range test as the branch: in range, u = (z - e0) * inv
     // is >= 0, and its conversion to int (truncation) is floor(u)
     if ((z >= c.e0) & (z <= c.e1)) {
@@ -581,7 +599,10 @@ __device__ __forceinline__ void bin_and_sum(const PassCtx &c, g_u32 *ghist, doub
             atomicAdd(reinterpret_cast<uint32_t *>(pass_lds()) + b, 1u);
         else
             __hip_atomic_fetch_add(ghist + b, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    } else {
         v[3] += 1.0;
+        if (CIC && z != z)
+            __hip_atomic_fetch_add(n_bad, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
 
@@ -589,45 +610,51 @@ __device__ __forceinline__ void bin_and_sum(const PassCtx &c, g_u32 *ghist, doub
 // at byte offset cb: the cell and weight the next pass's kick takes for it
 // (interp_index_pass).  round(w 2^51) is the low 52 bits of the double
 // 2^52 + w 2^51, formed by one fused multiply-add (one rounding; w in [0, 1),
-// so the sum stays below 2^53).  A NaN z or a non-finite weight is counted in
-// n[nb] instead.
+// so the sum stays below 2^53).  A NaN z lands in cell 0; bin_and_sum counts
+// it, which makes the sum NaN.
 __device__ __forceinline__ void cic_deposit(const PassCtx &c, int cb, double z) {
     int k;
     double w;
     interp_index_pass(z, c.c0, c.u1, c.inv_s, c.nb, k, w);
-    unsigned long long *sH = reinterpret_cast<unsigned long long *>(pass_lds() + cb);
-    unsigned long long *sL = sH + c.nb;
-    uint32_t *sN = reinterpret_cast<uint32_t *>(sL + c.nb);
-    if ((z == z) & (w == w)) {
-        const double y = __builtin_fma(w, kCicScale, 2.0 * kCicScale);
-        const unsigned long long W =
-            (unsigned long long)__double_as_longlong(y) & ((1ull << 52) - 1);   // <= 2^51
-        atomicAdd(sN + k, 1u);
-        atomicAdd(sH + k, W >> kCicLoBits);
-        atomicAdd(sL + k, W & ((1ull << kCicLoBits) - 1));
-    } else {
-        atomicAdd(sN + c.nb, 1u);
-    }
+    unsigned long long *cell = reinterpret_cast<unsigned long long *>(pass_lds() + cb) + 2 * k;
+    const unsigned long long y = (unsigned long long)__double_as_longlong(
+        __builtin_fma(w, kCicScale, 2.0 * kCicScale));
+    atomicAdd(cell, (1ull << kCicCountBit) | ((unsigned)(y >> 32) & 0xfffffu));   // W >> 32 <= 2^19
+    atomicAdd(cell + 1, y & 0xffffffffull);
 }
+
+// A value that every lane holds, as a scalar: the turn scalars are read through
+// a pointer that the kernel also writes near, so the compiler keeps them in
+// vector registers and takes the branches on them lane by lane.
+__device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
 // The fused pass over a run of tiles.  FX = kStdFlags is the common configuration
 // with the flags folded at compile time; FX = 0 handles any other.  Both
 // evaluate the same expressions, so a bunch gets the same bits from either.
 // LH: histogram in LDS at offset 0; the window of P follows at byte hb.
 //
-// One call covers the run of tiles [lt0, lt1) of bunch B that this workgroup
-// owns.  Tiles are whole multiples of the block size, so thread t's pairs in
-// tile lt are lt*ppt + t + k*kPassThreads in ascending k, exactly as for a
-// tile taken alone: the loop keeps its one-pair prefetch running across the
-// tile boundaries and writes each tile's per-wave sums at the tile's end.
-// The run's tiles are run[0..cnt) (indices into the tile table, in ascending
-// order but not necessarily adjacent: a bunch shared by several workgroups
-// has its tiles dealt to them in turn).
+// One call covers the run's tiles run[0..cnt) of bunch B (indices into the
+// tile table, in ascending order but not necessarily adjacent: a bunch shared
+// by several workgroups has its tiles dealt to them in turn).  Tiles are whole
+// multiples of the block size, so thread t's pairs in tile lt are
+// lt*ppt + t + k*kPassThreads in ascending k, exactly as for a tile taken
+// alone.  The loop over them is uniform: one chunk of kPassThreads pairs per
+// step, its addresses a scalar base plus the thread's constant offset, the
+// next chunk (the next tile's first at a tile's end) prefetched; only the last
+// chunk of a bunch may be shorter, and its lanes past the end re-read its last
+// pair and skip the rest.  Each tile's per-wave sums are written at its end.
+// The pass is bound by vector instructions below about 1e8 particles: with
+// per-thread 64-bit positions and bounds the same loop spent 16 of them per
+// pair on addresses, and 130 per tile on spilled scalars (a turn of a scan of 28
+// bunches, most tiles of one to four pairs per thread: 240 -> 213 us; 24 served
+// jobs 33.0 -> 30.3 ms; 1e7 particles 124 -> 121 us a turn).
 // KM, how the kick reads P: kFullWindow (the LDS window holds the whole table:
 // no global gathers), kGatherFirst or kPrefetchFirst (a partial window, the
 // particles outside it gather from global memory; see the loop body).
 // CIC: the bunch's post-drift z are also deposited (cic_deposit) into the LDS
 // counters at byte cb.
+// With FX = kStdFlags the kick is applied from the first turn on: P is zero
+// before it, and subtracting 0 changes nothing.
 enum KickMode { kFullWindow = 0, kGatherFirst = 1, kPrefetchFirst = 2 };
 template <uint32_t FX, bool LH, int KM, bool CIC>
 __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *__restrict__ run,
@@ -638,76 +665,73 @@ __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *
     const bool wake = fl.has(F_WAKE);
     const TurnScalars &sc = *B.sc;
     const int64_t n = B.n;
-    const int64_t ppt = B.pairs_per_tile;
-    const int64_t full = n >> 1;                    // pairs with two particles
+    // pair indices are unsigned 32-bit: a bunch has at most 2^31 pairs
+    const unsigned ppt = (unsigned)B.pairs_per_tile;
+    const unsigned full = (unsigned)(n >> 1);       // pairs with two particles
     const int tb = B.tile_begin;
-    const uint32_t tabs = (uint32_t)(B.turn_offset + sc.turn);
+    const uint32_t tabs = (uint32_t)uni((int)(uint32_t)(B.turn_offset + sc.turn));
     const bool inj = fl.has(F_INJ);
     const bool qe = fl.has(F_QE);
     const g_f64 *nrm = inj ? (const g_f64 *)(B.normals + sc.turn * n) : nullptr;
     const uint64_t seed = B.seed;
-    const bool kick2 = c.pending_kick && c.nb >= 2;
-    const int wlo = window_lo(sc.centre_bin, B.win, c.nb);
+    const bool kick = FX ? true : uni(c.pending_kick) != 0;
+    const bool kick2 = kick && (FX ? true : c.nb >= 2);
+    const bool rec = uni(c.pending_m) != 0;
+    const int wlo = KM == kFullWindow ? 0 : uni(window_lo(sc.centre_bin, B.win, c.nb));
     const unsigned wpairs = (unsigned)max(B.win - 1, 0);   // pair starts inside the window
     const double *sP = reinterpret_cast<const double *>(pass_lds() + hb);
     const g_f64x2 *P2 = (const g_f64x2 *)B.P2;
     g_f64 *zp = (g_f64 *)B.z;
     g_f64 *ep = (g_f64 *)B.dE;
     g_u32 *ghist = (g_u32 *)hist_of(B, sc.turn);
+    g_u32 *n_bad = CIC ? (g_u32 *)(B.cic + 2 * (int64_t)c.nb) + c.nb : nullptr;
+    const unsigned tid = threadIdx.x;
+    const int wave = uni((int)(tid >> 6));
+    constexpr unsigned step = kPassThreads;
 
-    double2 zn = make_double2(0.0, 0.0), en = make_double2(0.0, 0.0);
-    // The pair stride is the block size, as the compile-time constant: read
-    // from the dispatch packet, blockDim.x was reloaded per tile with a vector
-    // load and a full wait (1e8 pass +2%).
-    const int64_t step = kPassThreads;
+    // pair `base` + (byte offset / 16) of the z or dE array
+    auto at = [](g_f64 *a, unsigned base, unsigned off) -> g_f64x2 * {
+        return (g_f64x2 *)((g_u8 *)a + (int64_t)base * 16 + off);
+    };
     // per-wave partial sums of a tile: no workgroup barrier per tile, so a wave
     // never waits for the others of its workgroup between tiles
     auto flush = [&](const double (&v)[4], int lt) {
         const double tot = wave_total4(v);
-        const int lane = (int)threadIdx.x & 63;
-        if (lane >= 60)
-            B.part[4 * ((int64_t)lt * kTileWaves + (threadIdx.x >> 6)) + (lane - 60)] = tot;
+        const int lane = (int)tid & 63;
+        g_f64 *o = (g_f64 *)B.part + 4 * ((int64_t)lt * kTileWaves + wave);
+        if (lane >= 60) o[lane - 60] = tot;
     };
     // the single particle of an odd bunch sits in the bunch's last tile, the
     // last of this run if the run has it: that tile is flushed after the loop
     const int lt_last = run[cnt - 1] - tb;
-    const bool odd_tile = (n & 1) && full >= (int64_t)lt_last * ppt &&
-                          full < min((int64_t)(lt_last + 1) * ppt, B.npairs);
-    double v[4];   // sum z, sum z^2, sum (dE'-dE_init), in-range count
-    bool reload = true;   // this tile's first pair was not prefetched
+    const bool odd_tile = (n & 1) && (int64_t)full >= (int64_t)lt_last * ppt &&
+                          (int64_t)full < min((int64_t)(lt_last + 1) * ppt, B.npairs);
+    double v[4] = {0.0, 0.0, 0.0, 0.0};   // sum z, sum z^2, sum (dE'-dE_init), not binned
+    // a chunk's byte offset for this thread; lanes past the end take its last pair
+    auto offset = [&](unsigned lim) -> unsigned { return min(tid, lim - 1) * 16u; };
+    double2 zn = make_double2(0.0, 0.0), en = make_double2(0.0, 0.0);
+    int lt = run[0] - tb;
+    {
+        const unsigned b0 = (unsigned)lt * ppt, lim = min(full - b0, step);   // b0 <= full
+        if (lim > 0) {
+            const unsigned off = offset(lim);
+            zn = ldnt(at(zp, b0, off));
+            en = ldnt(at(ep, b0, off));
+        }
+    }
+    // the first chunk completes here (s_waitcnt vmcnt(0)), so that in the loop
+    // the pair in hand is never taken for an outstanding load and the waits
+    // there count only the loads issued in the loop
+    __builtin_amdgcn_s_waitcnt(0x0F70);
     for (int t = 0; t < cnt; ++t) {
-        const int lt = run[t] - tb;
-        const int64_t p0 = (int64_t)lt * ppt;
-        const int64_t p1 = min(p0 + ppt, B.npairs);
-        const int64_t pf = min(p1, full);
-        if (reload) {
-            const int64_t p = p0 + threadIdx.x;
-            if (p < pf) {
-                zn = ldnt((const g_f64x2 *)(zp + 2 * p));
-                en = ldnt((const g_f64x2 *)(ep + 2 * p));
-            }
-            // the tile's first pair completes here (s_waitcnt vmcnt(0)), so that
-            // in the loop the pair in hand is never taken for an outstanding
-            // load and the waits there count only the loads issued in the loop
-            __builtin_amdgcn_s_waitcnt(0x0F70);
-        }
-        // where the prefetch goes after this tile's last pair: the next tile's
-        // first pair of this thread when every thread has one there; else this
-        // tile's first pair, read again and not used (and the next tile, the
-        // bunch's short last one, loads its first pair itself)
-        int64_t nxt = p0;
-        reload = false;
-        if (t + 1 < cnt) {
-            const int64_t q0 = (int64_t)(run[t + 1] - tb) * ppt;
-            if (min(q0 + ppt, full) - q0 >= step)
-                nxt = q0;
-            else
-                reload = true;
-        }
+        const unsigned p0 = (unsigned)lt * ppt;
+        const unsigned p1 = min(p0 + ppt, full);
+        const int ltn = t + 1 < cnt ? run[t + 1] - tb : lt;
 #pragma unroll
         for (int k = 0; k < 4; ++k) v[k] = 0.0;
-        for (int64_t p = p0 + threadIdx.x; p < pf; p += step) {
+        for (unsigned base = p0; base < p1; base += step) {
             const double2 zz = zn, ee = en;
+            const unsigned lim = min(p1 - base, step);
             // The previous turn's potential at (P[k], P[k+1]): read from the LDS
             // window (clamped index, always valid), replaced by one 16-byte
             // global gather for the particles outside a partial window.  With
@@ -717,14 +741,16 @@ __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *
             // first.  The order of the loads changes no result.
             constexpr bool gather = KM != kFullWindow;
             constexpr bool gather_first = KM == kGatherFirst;
-            const int64_t pn = p + step;
-            // the next pair (the next tile's first at a tile end); past the end
-            // of the run a pair of this tile is read again and not used, so the
-            // load is unconditional and zn, en need no copy of their old value
+            // the next chunk (the next tile's first at a tile's end); past the
+            // end of the run, or where that tile has no pair of two particles,
+            // this chunk is read again and not used, so the load is
+            // unconditional and zn, en need no copy of their old value
             auto prefetch = [&]() {
-                const int64_t pq = pn < pf ? pn : nxt + threadIdx.x;
-                zn = ldnt((const g_f64x2 *)(zp + 2 * pq));
-                en = ldnt((const g_f64x2 *)(ep + 2 * pq));
+                unsigned bn = base + step < p1 ? base + step : (unsigned)ltn * ppt;
+                if (bn >= full) bn = base;
+                const unsigned off = offset(min(full - bn, step));
+                zn = ldnt(at(zp, bn, off));
+                en = ldnt(at(ep, bn, off));
             };
             if (!gather_first) prefetch();
             // set and read only when kick2 (no per-pair clearing)
@@ -734,16 +760,18 @@ __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *
                 int k0, k1;
                 interp_index_pass(zz.x, c.c0, c.u1, c.inv_s, c.nb, k0, w0);
                 interp_index_pass(zz.y, c.c0, c.u1, c.inv_s, c.nb, k1, w1);
-                const unsigned j0 = (unsigned)(k0 - wlo), j1 = (unsigned)(k1 - wlo);
-                // a full window, and any window of the all-flags pass (its
-                // histogram is in LDS, so its window has at least two entries),
-                // has wpairs >= 1
-                if (KM == kFullWindow || FX != 0 || wpairs) {
-                    const unsigned i0 = min(j0, wpairs - 1), i1 = min(j1, wpairs - 1);
-                    q0 = make_double2(sP[i0], sP[i0 + 1]);
-                    q1 = make_double2(sP[i1], sP[i1 + 1]);
-                }
-                if (gather) {
+                if (!gather) {
+                    q0 = make_double2(sP[k0], sP[k0 + 1]);
+                    q1 = make_double2(sP[k1], sP[k1 + 1]);
+                } else {
+                    const unsigned j0 = (unsigned)(k0 - wlo), j1 = (unsigned)(k1 - wlo);
+                    // any window of the all-flags pass (its histogram is in LDS,
+                    // so its window has at least two entries) has wpairs >= 1
+                    if (FX != 0 || wpairs) {
+                        const unsigned i0 = min(j0, wpairs - 1), i1 = min(j1, wpairs - 1);
+                        q0 = make_double2(sP[i0], sP[i0 + 1]);
+                        q1 = make_double2(sP[i1], sP[i1 + 1]);
+                    }
                     if (j0 >= wpairs) q0 = ld2(P2 + k0);
                     if (j1 >= wpairs) q1 = ld2(P2 + k1);
                 }
@@ -757,26 +785,28 @@ __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *
             double r0 = 0.0, r1 = 0.0;
             if (qe) {
                 if (inj) {   // turn rows of an odd bunch are only 8-byte aligned
+                    const int64_t p = (int64_t)base + min(tid, lim - 1);
                     r0 = nrm[2 * p];
                     r1 = nrm[2 * p + 1];
                 } else {
-                    qe_pair_normals(seed, (uint64_t)p, tabs, r0, r1);
+                    qe_pair_normals32(seed, base + tid, tabs, r0, r1);
                 }
             }
             double z0 = zz.x, z1 = zz.y, e0 = ee.x, e1 = ee.y;
-            if (c.pending_kick) {
+            if (kick) {
                 if (kick2) {
                     e0 = e0 - (q0.x * (1.0 - w0) + q0.y * w0);
                     e1 = e1 - (q1.x * (1.0 - w1) + q1.y * w1);
                 } else {
-                    e0 = e0 - c.P[0];
-                    e1 = e1 - c.P[0];
+                    const double pc = ((const g_f64 *)c.P)[0];
+                    e0 = e0 - pc;
+                    e1 = e1 - pc;
                 }
             }
             // with update_E0 every turn but the first has a re-centre pending,
             // and m_prev is 0 when none is: the all-flags pass subtracts it
             // without a select
-            if (fl.has(F_E0) || c.pending_m) {
+            if (fl.has(F_E0) || rec) {
                 e0 = e0 - c.m_prev;
                 e1 = e1 - c.m_prev;
             }
@@ -788,27 +818,30 @@ __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *
                 advance(c, fl, z0, e0, r0, d0);
                 advance(c, fl, z1, e1, r1, d1);
             }
-            if (wake) {
-                bin_and_sum<LH>(c, ghist, z0, v);
-                bin_and_sum<LH>(c, ghist, z1, v);
-            }
-            if (CIC) {
-                cic_deposit(c, cb, z0);
-                cic_deposit(c, cb, z1);
-            }
-            v[2] += d0;
-            v[2] += d1;
             // The prefetched pair is complete before this pair's stores are
             // issued: a wait for a load behind a store would wait for the store.
             __builtin_amdgcn_s_waitcnt(0x0F70);
-            // streaming stores: the bunch is far larger than the caches, which
-            // are left to the bin phase's tables
-            stnt((g_f64x2 *)(zp + 2 * p), z0, z1);
-            stnt((g_f64x2 *)(ep + 2 * p), e0, e1);
+            if (tid < lim) {
+                if (wake) {
+                    bin_and_sum<LH, CIC>(c, ghist, n_bad, z0, v);
+                    bin_and_sum<LH, CIC>(c, ghist, n_bad, z1, v);
+                }
+                if (CIC) {
+                    cic_deposit(c, cb, z0);
+                    cic_deposit(c, cb, z1);
+                }
+                v[2] += d0;
+                v[2] += d1;
+                // streaming stores: the bunch is far larger than the caches,
+                // which are left to the bin phase's tables
+                stnt(at(zp, base, tid * 16u), z0, z1);
+                stnt(at(ep, base, tid * 16u), e0, e1);
+            }
         }
         if (odd_tile && t == cnt - 1) break;   // v kept for the single particle
         if (!wake) { v[0] = 0.0; v[1] = 0.0; }
         flush(v, lt);
+        lt = ltn;
     }
     // the single particle of an odd bunch (last pair), out of the tile loop so
     // that its inlined turn does not add to the loop's register pressure
@@ -818,12 +851,12 @@ __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *
             double z0 = zp[i], e0 = ep[i], r0 = 0.0, r1 = 0.0;
             if (qe) {
                 if (inj) r0 = nrm[i];
-                else qe_pair_normals(seed, (uint64_t)full, tabs, r0, r1);
+                else qe_pair_normals32(seed, full, tabs, r0, r1);
             }
             e0 = apply_pending(c, z0, e0);
             double d0;
             advance(c, fl, z0, e0, r0, d0);
-            if (wake) bin_and_sum<LH>(c, ghist, z0, v);
+            if (wake) bin_and_sum<LH, CIC>(c, ghist, n_bad, z0, v);
             if (CIC) cic_deposit(c, cb, z0);
             v[2] += d0;
             zp[i] = z0;
@@ -846,25 +879,25 @@ __device__ inline void flush_hist(const BunchDev &B) {
     }
     if (B.flags & F_CIC) {   // and the deposit into this turn's counters
         const int nb = B.nbins;
-        const unsigned long long *sH =
-            reinterpret_cast<const unsigned long long *>(pass_lds() + B.cic_off);
-        const uint32_t *sN = reinterpret_cast<const uint32_t *>(sH + 2 * nb);
+        const ulonglong2 *sC = reinterpret_cast<const ulonglong2 *>(pass_lds() + B.cic_off);
         g_u64 *gH = (g_u64 *)B.cic;
         g_u32 *gN = (g_u32 *)(B.cic + 2 * nb);
-        for (int b = threadIdx.x; b <= nb; b += blockDim.x) {
-            const uint32_t cnt = sN[b];
-            if (!cnt) continue;
-            __hip_atomic_fetch_add(gN + b, cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (b < nb) {
-                __hip_atomic_fetch_add(gH + b, sH[b], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                __hip_atomic_fetch_add(gH + nb + b, sH[nb + b], __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT);
-            }
+        for (int b = threadIdx.x; b < nb; b += blockDim.x) {
+            const ulonglong2 c = sC[b];
+            if (!c.x) continue;
+            __hip_atomic_fetch_add(gN + b, (uint32_t)(c.x >> kCicCountBit), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_fetch_add(gH + b, (c.x & ((1ull << kCicCountBit) - 1)) + (c.y >> 32),
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_fetch_add(gH + nb + b, c.y & 0xffffffffull, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
         }
     }
 }
 
-// Clears the LDS histogram of bunch B and loads its potential window.
+// Clears the LDS histogram of bunch B and loads its potential window (zero
+// before the first turn's bin phase; the all-flags pass reads it from the start).
+template <uint32_t FX>
 __device__ inline void stage_bunch(const BunchDev &B) {
     __syncthreads();   // the previous bunch's LDS is no longer read
     const int hb = pass_hist_bytes(B);
@@ -875,7 +908,7 @@ __device__ inline void stage_bunch(const BunchDev &B) {
         for (int b = threadIdx.x; b < cic_bytes(B.nbins) / 4; b += blockDim.x) sC[b] = 0u;
     }
     const TurnScalars &sc = *B.sc;
-    if (sc.pending_kick && B.win > 0) {
+    if ((FX || sc.pending_kick) && B.win > 0) {
         double *sP = reinterpret_cast<double *>(pass_lds() + hb);
         const g_f64 *P = (const g_f64 *)(B.P + window_lo(sc.centre_bin, B.win, B.nbins));
         for (int k = threadIdx.x; k < B.win; k += blockDim.x) sP[k] = P[k];
@@ -883,47 +916,37 @@ __device__ inline void stage_bunch(const BunchDev &B) {
     __syncthreads();
 }
 
-// The fused pass over a tile table.  Each workgroup takes a contiguous range
-// of entries of the pass's tile order, with about the same number of pairs as
-// every other workgroup's (one workgroup per CU), stages a bunch's LDS once
-// for its run of the bunch's tiles in the range, streams the run and flushes
-// the histogram when it moves on.  The per-tile sums depend on the tile and
-// the block size only, not on which workgroup takes the tile.
+// The fused pass over a tile order.  Each workgroup takes its runs
+// (runs[rr[g]..rr[g+1]): consecutive entries of the pass's tile order of one
+// bunch, with about the same number of pairs as every other workgroup's, one
+// workgroup per CU), and for each stages the bunch's LDS, streams the run and
+// flushes the histogram.  The per-tile sums depend on the tile and the block
+// size only, not on which workgroup takes the tile.  The runs are found on the
+// host: found in the kernel, from the tile table, they cost two dependent
+// scalar loads per tile before the first byte was streamed.
 template <uint32_t FX>
 __device__ __forceinline__ void turn_pass_blocks(const BunchDev *__restrict__ bds,
-                                                 const int32_t *__restrict__ tile_bunch,
                                                  const int32_t *__restrict__ order,
-                                                 const int32_t *__restrict__ ranges) {
+                                                 const RunDev *__restrict__ runs,
+                                                 const int32_t *__restrict__ rr) {
     // kStdFlags has the wake on and F_GHIST off: its histogram is in LDS
     constexpr bool kLdsOnly = (FX & F_WAKE) && !(FX & F_GHIST);
-    const int e0 = ranges[blockIdx.x];
-    const int e1 = ranges[blockIdx.x + 1];
-    int staged = -1;
-    for (int e = e0; e < e1;) {
-        const int bi = tile_bunch[order[e]];
-        const BunchDev &B = bds[bi];
-        // the run: this workgroup's consecutive entries of the bunch
-        int ee = e + 1;
-        while (ee < e1 && tile_bunch[order[ee]] == bi) ++ee;
-        if (bi != staged) {
-            if (staged >= 0) flush_hist(bds[staged]);
-            stage_bunch(B);
-            staged = bi;
-        }
+    const int r1 = rr[blockIdx.x + 1];
+    for (int r = rr[blockIdx.x]; r < r1; ++r) {
+        const RunDev rd = runs[r];
+        const BunchDev &B = bds[rd.bunch];
+        stage_bunch<FX>(B);
         const int hb = pass_hist_bytes(B);
-        const int32_t *run = order + e;
-        const int cnt = ee - e;
+        const int32_t *run = order + rd.begin;
+        const int cnt = rd.count;
         // a partial window of P: gather first in the pass with compile-time
         // flags (only it has the registers), prefetch first in the generic one
         constexpr int kPartial = FX != 0 ? kGatherFirst : kPrefetchFirst;
         const bool full = B.win >= B.nbins;
         const int cb = B.cic_off;
         if (kLdsOnly || hb) {
-            if (B.flags & F_CIC) {   // the deposit needs the LDS histogram's room
-                if (full)
-                    turn_pass_run<FX, true, kFullWindow, true>(B, run, cnt, hb, cb);
-                else
-                    turn_pass_run<FX, true, kPartial, true>(B, run, cnt, hb, cb);
+            if (B.flags & F_CIC) {   // the deposit comes with the whole table
+                turn_pass_run<FX, true, kFullWindow, true>(B, run, cnt, hb, cb);
             } else {
                 if (full)
                     turn_pass_run<FX, true, kFullWindow, false>(B, run, cnt, hb, cb);
@@ -936,23 +959,23 @@ __device__ __forceinline__ void turn_pass_blocks(const BunchDev *__restrict__ bd
             else
                 turn_pass_run<FX, false, kPrefetchFirst, false>(B, run, cnt, hb, cb);
         }
-        e = ee;
+        flush_hist(B);
     }
-    if (staged >= 0) flush_hist(bds[staged]);
 }
 
 __global__ __launch_bounds__(kPassThreads) void k_turn_pass(const BunchDev *__restrict__ bds,
-                                                            const int32_t *__restrict__ tile_bunch,
                                                             const int32_t *__restrict__ order,
-                                                            const int32_t *__restrict__ ranges) {
-    turn_pass_blocks<0>(bds, tile_bunch, order, ranges);
+                                                            const RunDev *__restrict__ runs,
+                                                            const int32_t *__restrict__ rr) {
+    turn_pass_blocks<0>(bds, order, runs, rr);
 }
 
-// the same for tables whose bunches all have exactly kStdFlags
-__global__ __launch_bounds__(kPassThreads) void k_turn_pass_std(
-    const BunchDev *__restrict__ bds, const int32_t *__restrict__ tile_bunch,
-    const int32_t *__restrict__ order, const int32_t *__restrict__ ranges) {
-    turn_pass_blocks<kStdFlags>(bds, tile_bunch, order, ranges);
+// the same for tables whose bunches all have exactly kStdFlags and two bins or more
+__global__ __launch_bounds__(kPassThreads) void k_turn_pass_std(const BunchDev *__restrict__ bds,
+                                                                const int32_t *__restrict__ order,
+                                                                const RunDev *__restrict__ runs,
+                                                                const int32_t *__restrict__ rr) {
+    turn_pass_blocks<kStdFlags>(bds, order, runs, rr);
 }
 
 // ---------------------------------------------------------------------------
@@ -1055,7 +1078,7 @@ __device__ inline bool slices_done(const BunchDev &B, int r, const double (&v)[N
 }
 
 // The turn scalars from the reduced pass sums t = {sum z, sum z^2,
-// sum (dE'-dE_init), binned count}.
+// sum (dE'-dE_init), particles not binned}.
 // bin_scalars_on updates the turn scalars sc in place (the bin phase in one
 // workgroup keeps them in registers).
 __device__ inline void bin_scalars_on(const BunchDev &B, const double (&t)[4], TurnScalars &sc) {
@@ -1068,7 +1091,7 @@ __device__ inline void bin_scalars_on(const BunchDev &B, const double (&t)[4], T
                      ? B.charge
                      : (((B.pf / sc.E0) / (kTwoPi * B.radius)) * sz) /
                            (sc.eta0 * (B.sigma_E0 * B.sigma_E0));
-    sc.n_h = t[3];
+    sc.n_h = (double)B.n - t[3];
     const double kc = floor((mz - B.c_first) * B.inv_s);
     const double top = (double)(B.nbins - 1);
     sc.centre_bin = (kc == kc) ? (int)(kc < 0.0 ? 0.0 : (kc > top ? top : kc)) : 0;
@@ -1076,7 +1099,7 @@ __device__ inline void bin_scalars_on(const BunchDev &B, const double (&t)[4], T
         double *m = B.mon + 4 * sc.turn;
         m[0] = mz;
         m[1] = sz;
-        m[3] = t[3];
+        m[3] = sc.n_h;
     }
 }
 
@@ -1167,7 +1190,7 @@ __global__ __launch_bounds__(kRedThreads) void k_bin_reduce(const BunchDev *__re
     const BunchDev &B = bds[items[2 * blockIdx.x]];
     const int r = items[2 * blockIdx.x + 1];
     if (!(B.flags & (F_WAKE | F_E0))) return;
-    double v[4] = {0.0, 0.0, 0.0, 0.0};   // sum z, sum z^2, sum (dE'-dE_init), binned count
+    double v[4] = {0.0, 0.0, 0.0, 0.0};   // sum z, sum z^2, sum (dE'-dE_init), not binned
     slice_sum<4>(B.part, B.ntiles * kTileWaves, r, v, s_red);
     double t[4];
     if (!slices_done<4>(B, r, v, t) || threadIdx.x != 0) return;
@@ -1682,41 +1705,36 @@ __device__ __forceinline__ void interp_sum_run(const BunchDev &B, const int32_t 
 }
 
 // The interpolation sums of the wake + update_E0 bunches over a tile table:
-// each workgroup walks its contiguous range of entries of the sums' tile
-// order, one run per bunch (a bunch shared by several workgroups has its
-// tiles dealt to them in turn, as in the pass).
+// each workgroup walks its runs of the sums' tile order (a bunch shared by
+// several workgroups has its tiles dealt to them in turn, as in the pass).
 template <int G>
 __device__ __forceinline__ void interp_sum_blocks(const BunchDev *__restrict__ bds,
-                                         const int32_t *__restrict__ tile_bunch,
-                                         const int32_t *__restrict__ order,
-                                         const int32_t *__restrict__ ranges) {
-    const int e0 = ranges[blockIdx.x];
-    const int e1 = ranges[blockIdx.x + 1];
-    for (int e = e0; e < e1;) {
-        const int bi = tile_bunch[order[e]];
-        const BunchDev &B = bds[bi];
-        int ee = e + 1;
-        while (ee < e1 && tile_bunch[order[ee]] == bi) ++ee;
+                                                  const int32_t *__restrict__ order,
+                                                  const RunDev *__restrict__ runs,
+                                                  const int32_t *__restrict__ rr) {
+    const int r1 = rr[blockIdx.x + 1];
+    for (int r = rr[blockIdx.x]; r < r1; ++r) {
+        const RunDev rd = runs[r];
+        const BunchDev &B = bds[rd.bunch];
         if ((B.flags & F_WAKE) && (B.flags & F_E0) && !(B.flags & F_CIC))
-            interp_sum_run<G>(B, order + e, ee - e);
-        e = ee;
+            interp_sum_run<G>(B, order + rd.begin, rd.count);
     }
 }
 
 // At most 64 VGPRs, so that two workgroups fit a CU when both windows fit its
 // LDS; rings of four loads.
 __global__ __launch_bounds__(kInterpThreads) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_interp_sum(
-    const BunchDev *__restrict__ bds, const int32_t *__restrict__ tile_bunch,
-    const int32_t *__restrict__ order, const int32_t *__restrict__ ranges) {
-    interp_sum_blocks<4>(bds, tile_bunch, order, ranges);
+    const BunchDev *__restrict__ bds, const int32_t *__restrict__ order,
+    const RunDev *__restrict__ runs, const int32_t *__restrict__ rr) {
+    interp_sum_blocks<4>(bds, order, runs, rr);
 }
 
 // One workgroup per CU (a window of P larger than half the LDS): the
 // registers of four waves per SIMD allow rings of eight loads.
 __global__ __launch_bounds__(kInterpThreads) void k_interp_sum_deep(
-    const BunchDev *__restrict__ bds, const int32_t *__restrict__ tile_bunch,
-    const int32_t *__restrict__ order, const int32_t *__restrict__ ranges) {
-    interp_sum_blocks<8>(bds, tile_bunch, order, ranges);
+    const BunchDev *__restrict__ bds, const int32_t *__restrict__ order,
+    const RunDev *__restrict__ runs, const int32_t *__restrict__ rr) {
+    interp_sum_blocks<8>(bds, order, runs, rr);
 }
 
 // Per-tile sums of z, z^2, dE, dE^2 (the initial and final spreads,
@@ -1892,7 +1910,7 @@ __device__ inline void finish_turn(const BunchDev &B, double psum) {
 
 // The sum over the bunch of the interpolated potential from the cloud-in-cell
 // deposit (F_CIC): sum_k (N_k - S_k) P[k] + S_k P[k+1] with
-// S_k = (hi_k 2^20 + lo_k) / 2^51, over the cells with particles (a cell
+// S_k = (hi_k 2^32 + lo_k) / 2^51, over the cells with particles (a cell
 // without particles adds nothing, even where P is not finite); NaN when some
 // particle's weight was not finite (as its interpolated value is).  Threads
 // [0, kRedThreads) take cells k = t + kRedThreads*j in ascending j and clear
@@ -1926,8 +1944,7 @@ __device__ inline double cic_psum(const BunchDev &B, double *s_red) {
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 if (cnt[u]) {
-                    const double sk = ((double)hi[u] * (double)(1 << kCicLoBits) + (double)lo[u]) *
-                                      (1.0 / kCicScale);
+                    const double sk = ((double)hi[u] * 0x1p32 + (double)lo[u]) * (1.0 / kCicScale);
                     v += ((double)cnt[u] - sk) * p0[u] + sk * p1[u];
                 }
             }
@@ -2009,8 +2026,7 @@ __device__ inline double cic_psum_lds(const BunchDev &B, const uint32_t *sN,
         for (int k = (int)threadIdx.x; k < nb - 1; k += kRedThreads) {
             const uint32_t cnt = sN[k];
             if (cnt) {
-                const double sk = ((double)sH[k] * (double)(1 << kCicLoBits) + (double)sH[nb + k]) *
-                                  (1.0 / kCicScale);
+                const double sk = ((double)sH[k] * 0x1p32 + (double)sH[nb + k]) * (1.0 / kCicScale);
                 v += ((double)cnt - sk) * sP[k] + sk * sP[k + 1];
                 N[k] = 0u;
                 H[k] = 0ull;
@@ -2485,15 +2501,15 @@ hipError_t launch_init(const BunchDev *bds, const int32_t *list, int nb, hipStre
     return hipGetLastError();
 }
 
-hipError_t launch_turn_pass(const BunchDev *bds, const int32_t *tb, const int32_t *order,
-                            const int32_t *ranges, int grid, size_t lds, int std_only, hipStream_t s) {
+hipError_t launch_turn_pass(const BunchDev *bds, const int32_t *order, const RunDev *runs,
+                            const int32_t *rr, int grid, size_t lds, int std_only, hipStream_t s) {
     if (grid <= 0) return hipSuccess;
     if (std_only)
         hipLaunchKernelGGL(k_turn_pass_std, dim3((unsigned)grid), dim3(kPassThreads), lds, s, bds,
-                           tb, order, ranges);
+                           order, runs, rr);
     else
-        hipLaunchKernelGGL(k_turn_pass, dim3((unsigned)grid), dim3(kPassThreads), lds, s, bds, tb,
-                           order, ranges);
+        hipLaunchKernelGGL(k_turn_pass, dim3((unsigned)grid), dim3(kPassThreads), lds, s, bds,
+                           order, runs, rr);
     return hipGetLastError();
 }
 
@@ -2515,16 +2531,16 @@ hipError_t launch_conv(int kind, const BunchDev *bds, const int32_t *items, int 
     return hipGetLastError();
 }
 
-hipError_t launch_interp_sum(const BunchDev *bds, const int32_t *tb, const int32_t *order,
-                             const int32_t *ranges, int grid, size_t lds_bytes, bool deep,
+hipError_t launch_interp_sum(const BunchDev *bds, const int32_t *order, const RunDev *runs,
+                             const int32_t *rr, int grid, size_t lds_bytes, bool deep,
                              hipStream_t s) {
     if (grid <= 0) return hipSuccess;
     if (deep)
         hipLaunchKernelGGL(k_interp_sum_deep, dim3((unsigned)grid), dim3(kInterpThreads), lds_bytes,
-                           s, bds, tb, order, ranges);
+                           s, bds, order, runs, rr);
     else
         hipLaunchKernelGGL(k_interp_sum, dim3((unsigned)grid), dim3(kInterpThreads), lds_bytes, s,
-                           bds, tb, order, ranges);
+                           bds, order, runs, rr);
     return hipGetLastError();
 }
 

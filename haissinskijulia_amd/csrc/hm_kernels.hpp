@@ -68,21 +68,22 @@ hipError_t launch_moments(const BunchDev *bds, const int32_t *tile_bunch, int nt
 hipError_t launch_moments_final(const BunchDev *bds, const int32_t *bunch_list, int nb, int mode,
                                 hipStream_t s);
 hipError_t launch_init(const BunchDev *bds, const int32_t *bunch_list, int nb, hipStream_t s);
-// `grid` workgroups over the tile table, workgroup g taking tiles
-// [ranges[g], ranges[g+1]); lds_bytes = the largest per-bunch histogram +
-// potential window; std_only: every tile's bunch has (flags & kPhysMask) == kStdFlags
-hipError_t launch_turn_pass(const BunchDev *bds, const int32_t *tile_bunch, const int32_t *order,
-                            const int32_t *ranges, int grid, size_t lds, int std_only, hipStream_t s);
+// `grid` workgroups over the tile order, workgroup g taking the runs
+// [rr[g], rr[g+1]); lds_bytes = the largest per-bunch histogram + potential
+// window; std_only: every bunch has (flags & kPhysMask) == kStdFlags and two
+// bins or more
+hipError_t launch_turn_pass(const BunchDev *bds, const int32_t *order, const RunDev *runs,
+                            const int32_t *rr, int grid, size_t lds, int std_only, hipStream_t s);
 // items are (bunch, block) pairs, for CONV_SPEC (bunch, frequency chunk)
 // pairs; Fmax is the largest FFT length among them, for CONV_SPEC the largest
 // conv_spec_lds of their bunches in bytes
 hipError_t launch_conv(int kind, const BunchDev *bds, const int32_t *items, int nitems, int Fmax,
                        hipStream_t s);
 // interpolation sums of the wake + update_E0 bunches: `grid` workgroups over
-// the tile table (ranges as for the pass); lds_bytes = 8 x the largest iwin;
+// their tile order (runs as for the pass); lds_bytes = 8 x the largest iwin;
 // deep: one workgroup per CU, eight streaming loads in flight per thread
-hipError_t launch_interp_sum(const BunchDev *bds, const int32_t *tile_bunch, const int32_t *order,
-                             const int32_t *ranges, int grid, size_t lds_bytes, bool deep,
+hipError_t launch_interp_sum(const BunchDev *bds, const int32_t *order, const RunDev *runs,
+                             const int32_t *rr, int grid, size_t lds_bytes, bool deep,
                              hipStream_t s);
 // per-bunch reduction of the pass's tile sums into the turn scalars (sum of
 // dE'-dE_init; sigma_z, current, binned count, centroid cell of a wake bunch),

@@ -12,7 +12,7 @@
 //   Y[nA][F]      (complex)     their products with the wake spectra, summed
 //                               per output block (before its inverse FFT)
 //   part[ntiles][16][4]         per-wave sums of each tile (sum z, sum z^2,
-//                               sum dE'-dE_init, in-range count)
+//                               sum dE'-dE_init, particles not binned)
 //   ipart[ntiles][16]           per-wave sums of each tile of the interpolated
 //                               potential (E0 update)
 //   moments[ntiles][4]          per-tile sums of z, z^2, dE, dE^2 (initial / final spreads)
@@ -49,14 +49,18 @@ enum BunchFlags : uint32_t {
 // those z.  The interpolation is linear in P: with (k_i, w_i) the cell and
 // weight of z_i, the sum is sum_k (N_k - S_k) P_t[k] + S_k P_t[k+1], where
 // N_k counts the particles of cell k and S_k adds their weights.  The pass
-// counts N_k and adds W_i = round(w_i 2^51) into two 64-bit counters per cell
-// (W >> 20 and the low 20 bits): integer sums, so they do not depend on the
-// order of the additions, and 2^-52 of a weight is as fine as the weight's
-// own FP64 rounding.  Layout, in LDS and in global memory: hi[nbins],
-// lo[nbins] (64-bit), then n[nbins + 1] (32-bit; n[nbins] counts particles
-// whose weight is not finite).
+// adds W_i = round(w_i 2^51): integer sums, so they do not depend on the order
+// of the additions, and 2^-52 of a weight is as fine as the weight's own FP64
+// rounding.  In LDS a cell is a pair of 64-bit counters: N_k (from bit
+// kCicCountBit) with the sum of W >> 32, and the sum of W's low words, so a
+// particle costs two atomics at one address; the count's field bounds a run
+// to kCicRunPairs pairs between two flushes.  In global memory: hi[nbins],
+// lo[nbins] (64-bit; the flush carries lo's high word into hi, so lo stays
+// exact in a double), then n[nbins + 1] (32-bit; n[nbins] counts NaN
+// positions).
 constexpr double kCicScale = 2251799813685248.0;   // 2^51
-constexpr int kCicLoBits = 20;
+constexpr int kCicCountBit = 42;
+constexpr int64_t kCicRunPairs = (int64_t)1 << 20;
 
 // the all-physics-on configuration the turn pass is specialised for, and the
 // flags that select the pass's code path
@@ -123,9 +127,16 @@ struct BunchDev {
     uint32_t *cnt;
     int32_t nred;
     int32_t cic_off;      // F_CIC: byte offset of the pass's LDS deposit
+    int32_t cic_tiles;    // F_CIC: tiles of a run between two flushes of the deposit
     TurnScalars *sc;
     double *mon;          // device [n_turns][4] turn monitor or null
     unsigned long long *cic;   // F_CIC: this turn's deposit (hi, lo, n; zero between turns)
+};
+
+// A run of a workgroup: `count` consecutive entries, from `begin`, of a tile
+// order, all of one bunch.
+struct RunDev {
+    int32_t bunch, begin, count;
 };
 
 // LDS of a turn-pass workgroup for one bunch: its histogram (nbins counts,
@@ -136,7 +147,7 @@ __host__ __device__ inline int pass_hist_bytes(const BunchDev &B) {
     return ((B.flags & F_WAKE) && !(B.flags & F_GHIST)) ? ((B.nbins * 4 + 15) & ~15) : 0;
 }
 
-__host__ __device__ inline int cic_bytes(int nbins) { return (16 * nbins + 4 * (nbins + 1) + 15) & ~15; }
+__host__ __device__ inline int cic_bytes(int nbins) { return 16 * nbins; }
 __host__ __device__ inline int pass_cic_bytes(const BunchDev &B) {
     return (B.flags & F_CIC) ? cic_bytes(B.nbins) : 0;
 }
