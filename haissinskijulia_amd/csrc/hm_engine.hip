@@ -417,7 +417,7 @@ hm_status Batch::stage_descriptors() {
 
 // launch tables of the active bunches
 hm_status Batch::build_tables() {
-    std::vector<int32_t> tiles, conv[kConvKinds], red, list, bw;
+    std::vector<int32_t> tiles, conv[kConvKinds], red, list, bw, b64;
     pass_lds_ = 0;
     bw_lds_ = 0;
     spec_lds_ = 0;
@@ -454,7 +454,8 @@ hm_status Batch::build_tables() {
                 bin_whole_layout(wake ? q.d.nbins : 0, q.d.nA, q.d.nJ, q.d.F, dep).bytes;
             if (q.o.bin_whole == 0 && q.d.ntiles <= kBinWholeMaxTiles && lds <= kBinWholeMaxLds &&
                 (!wake || !(f & F_E0) || (f & F_CIC))) {
-                bw.push_back((int32_t)i);
+                (fits_bin_64(wake, q.d.nbins, q.d.win, q.d.nA, q.d.nJ, q.d.F, q.d.nred) ? b64 : bw)
+                    .push_back((int32_t)i);
                 bw_lds_ = std::max(bw_lds_, lds);
                 continue;
             }
@@ -502,6 +503,8 @@ hm_status Batch::build_tables() {
     nred_ = (int)red.size() / 2;
     nlist_ = (int)list.size();
     nbw_ = (int)bw.size();
+    nb64_ = (int)b64.size();
+    bw.insert(bw.begin(), b64.begin(), b64.end());
     // Workgroup ranges: contiguous runs of the tile table with equal numbers
     // of pairs (tiles of different bunches differ in size), for the pass and
     // for the interpolation sums (which only count wake + update_E0 bunches).
@@ -973,7 +976,8 @@ hm_status Batch::one_turn() {
     HIP_TRY(launch_turn_pass(d_bd_.p, d_order_.p, d_runs_.p, d_ranges_.p, pass_grid_, pass_lds_,
                              std_only_ ? 1 : 0, s));
     if (timing_) HIP_TRY(hipEventRecord(e1, s));
-    HIP_TRY(launch_bin_whole(d_bd_.p, d_bw_.p, nbw_, bw_lds_, s));
+    HIP_TRY(launch_bin_64(d_bd_.p, d_bw_.p, nb64_, bw_lds_, s));
+    HIP_TRY(launch_bin_whole(d_bd_.p, d_bw_.p + nb64_, nbw_, bw_lds_, s));
     const bool whole = nlist_ >= kWholeMinBunches;
     if (any_reduce_)
         HIP_TRY(whole ? launch_bin_reduce_whole(d_bd_.p, d_list_.p, nlist_, s)
@@ -1004,7 +1008,7 @@ hm_status Batch::flush_timing() {
         HIP_TRY(hipEventElapsedTime(&b, ev_pool_[k + 1], ev_pool_[k + 2]));
         pass_ms_ += a;
         ++pass_count_;
-        if (any_wake_ || nbw_ > 0) {
+        if (any_wake_ || nbw_ + nb64_ > 0) {
             conv_ms_ += b;
             ++conv_count_;
         }

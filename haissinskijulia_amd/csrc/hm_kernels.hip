@@ -243,15 +243,59 @@ __device__ __forceinline__ int hist_bin(double z, double e0, double e1, double i
     return min(b, nb - 1);
 }
 
+// One DPP lane move of a double (two 32-bit moves with the same control);
+// lanes whose row is not in ROWS receive 0.0.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_move(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, ROWS, 0xF, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xF, false);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+// v[lane ^ OFF] + v[lane] for OFF = 32, 16, 8, 4, 2, 1 by lane swaps and DPP
+// moves: the same sum as with __shfl_xor (an addition's operands commute)
+// without its trip through LDS, whose latency is most of a butterfly's.
+template <int OFF>
+__device__ __forceinline__ double add_xor(double v) {
+    const long long b = __double_as_longlong(v);
+    const unsigned lo = (unsigned)b, hi = (unsigned)(b >> 32);
+    if constexpr (OFF == 32) {
+        const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+        const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+        return __longlong_as_double(((long long)h[0] << 32) | l[0]) +
+               __longlong_as_double(((long long)h[1] << 32) | l[1]);
+    } else if constexpr (OFF == 16) {
+        const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+        const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+        return __longlong_as_double(((long long)h[0] << 32) | l[0]) +
+               __longlong_as_double(((long long)h[1] << 32) | l[1]);
+    } else if constexpr (OFF == 8) {
+        return v + dpp_move<0x128, 0xF>(v);                       // row_ror:8
+    } else if constexpr (OFF == 4) {
+        return v + dpp_move<0x1B, 0xF>(dpp_move<0x141, 0xF>(v));  // half-row mirror, quad mirror
+    } else if constexpr (OFF == 2) {
+        return v + dpp_move<0x4E, 0xF>(v);                        // quad_perm [2,3,0,1]
+    } else {
+        return v + dpp_move<0xB1, 0xF>(v);                        // quad_perm [1,0,3,2]
+    }
+}
+// the butterfly sum over the wave, offsets 32 down to 1; every lane gets it
+__device__ __forceinline__ double butterfly(double v) {
+    v = add_xor<32>(v);
+    v = add_xor<16>(v);
+    v = add_xor<8>(v);
+    v = add_xor<4>(v);
+    v = add_xor<2>(v);
+    return add_xor<1>(v);
+}
+
 // Deterministic block sum of NV values: wave butterflies, then the waves in
 // order.  The result is valid in thread 0.  s_red holds NV * 16 doubles.
 template <int NV>
 __device__ inline void block_sum(double (&v)[NV], double *s_red) {
 #pragma unroll
-    for (int k = 0; k < NV; ++k) {
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) v[k] += __shfl_xor(v[k], off, 64);
-    }
+    for (int k = 0; k < NV; ++k) v[k] = butterfly(v[k]);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
     if (lane == 0) {
 #pragma unroll
@@ -276,16 +320,6 @@ __device__ __forceinline__ void wave_sum(double (&v)[NV]) {
 #pragma unroll
         for (int off = 32; off > 0; off >>= 1) v[k] += __shfl_xor(v[k], off, 64);
     }
-}
-
-// One DPP lane move of a double (two 32-bit moves with the same control);
-// lanes whose row is not in ROWS receive 0.0.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ double dpp_move(double v) {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, ROWS, 0xF, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xF, false);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
 // Sum of NV values over one wave in lane 63, by DPP lane moves (no LDS):
@@ -1155,9 +1189,7 @@ __device__ inline void whole_sum(const BunchDev &B, const double *a, double (&t)
         }
         // block_sum's order within the group: wave butterflies, then its four waves
 #pragma unroll
-        for (int j = 0; j < NV; ++j)
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1) v[j] += __shfl_xor(v[j], off, 64);
+        for (int j = 0; j < NV; ++j) v[j] = butterfly(v[j]);
         if (lane == 0)
 #pragma unroll
             for (int j = 0; j < NV; ++j) s_red[g][j * 16 + wave] = v[j];
@@ -1958,8 +1990,7 @@ __device__ inline double cic_psum(const BunchDev &B, double *s_red) {
                 }
             }
         }
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+        v = butterfly(v);
         if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = v;
     }
     __syncthreads();
@@ -2033,8 +2064,7 @@ __device__ inline double cic_psum_lds(const BunchDev &B, const uint32_t *sN,
                 H[nb + k] = 0ull;
             }
         }
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+        v = butterfly(v);
         if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = v;
     }
     __syncthreads();
@@ -2177,6 +2207,361 @@ __device__ inline void bin_phase_whole(const BunchDev &B) {
         t = B.nred == 1 ? d : 0.0 + d;
     }
     if (threadIdx.x == 0) {
+        finish_on(B, t, sc);
+        *B.sc = sc;
+    }
+}
+
+// LDS ordering within one wave: its LDS operations execute in order, so only
+// the compiler has to keep them so.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// A workgroup barrier for data exchanged through LDS alone: __syncthreads also
+// waits for the wave's outstanding global loads and stores.
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// The radix-2^2 butterflies of fft_dit_forward and fft_dif_inverse on four
+// points in registers.
+__device__ __forceinline__ void dit_pair(double2 (&x)[4], double2 w1, double2 wa, double2 wb) {
+    double2 t = cmul(x[1], w1);
+    const double2 a0 = cadd(x[0], t), a1 = csub(x[0], t);
+    t = cmul(x[3], w1);
+    const double2 a2 = cadd(x[2], t), a3 = csub(x[2], t);
+    t = cmul(a2, wa);
+    x[0] = cadd(a0, t);
+    x[2] = csub(a0, t);
+    t = cmul(a3, wb);
+    x[1] = cadd(a1, t);
+    x[3] = csub(a1, t);
+}
+// x holds points 0, h2, h, h + h2 of the inverse butterfly
+__device__ __forceinline__ void dif_pair(double2 (&x)[4], double2 wa, double2 wb, double2 wc) {
+    const double2 a0 = cadd(x[0], x[2]), a2 = cmul(csub(x[0], x[2]), wa);
+    const double2 a1 = cadd(x[1], x[3]), a3 = cmul(csub(x[1], x[3]), wb);
+    x[0] = cadd(a0, a1);
+    x[1] = cmul(csub(a0, a1), wc);
+    x[2] = cadd(a2, a3);
+    x[3] = cmul(csub(a2, a3), wc);
+}
+__device__ __forceinline__ double2 dpp_swap1(double2 v) {   // the neighbouring lane's (lane ^ 1)
+    return make_double2(dpp_move<0xB1, 0xF>(v.x), dpp_move<0xB1, 0xF>(v.y));
+}
+
+// k_bin_whole for the grids whose blocks are 64 bins (fits_bin_64: F = 128, at
+// most 16 blocks, more than one wake block): the same products, sums and
+// twiddles in the same order, so the same bits, arranged for latency.
+// - A block's 32 butterflies stay in one half-wave from the packing to the last
+//   stage, four points and all nine twiddles of a thread in registers: the
+//   stages exchange through LDS without workgroup barriers, and the first
+//   (its other inputs are the zero padding) and the last (half of its outputs
+//   are needed, each from a neighbouring lane) cost no LDS pass.
+// - The spectral sums take two consecutive output blocks per thread, so a wake
+//   and a line-density value are read once per two products; every SIMD's
+//   waves have the same number of products.
+// - The phase's barriers order LDS only, so a load is waited for where its
+//   value is used and not at the next barrier.
+// - The binned count comes from the counts themselves, so the transforms do
+//   not wait for the pass sums, which the waves that have no butterflies
+//   reduce meanwhile; one of their lanes (kScalarThread) does the scalars.
+// It is bound by LDS bandwidth: 264 KB for the forward transforms and 320 KB for
+// the spectral sums of 1024 bins, at 128 B a cycle.  Measured in a turn: 1024
+// bins 17.7 us (k_bin_whole) -> 9.5 us, 512 bins 12.7 -> 7.4 us.
+constexpr int kScalarThread = 512;
+// A point's place in its block in LDS: the stages' strides (2, 8 and 32 points of
+// 16 bytes) and the contiguous reads then spread over all banks.
+__device__ __forceinline__ int swz64(int e) { return e ^ ((e >> 3) & 7) ^ ((e >> 2) & 8); }
+__global__ __launch_bounds__(1024) void k_bin_64(const BunchDev *__restrict__ bds,
+                                                 const int32_t *__restrict__ list) {
+    const BunchDev &B = bds[list[blockIdx.x]];
+    extern __shared__ __align__(16) uint8_t s_bw[];
+    __shared__ double s_sum[4][4 * 16], s_cur, s_red[16];
+    __shared__ uint32_t s_cnt[16];
+    __shared__ double2 s_tw[126];   // w1, wa, wb of stages (1,2): 2 each, (3,4): 8 each, (5,6): 32 each
+    constexpr int F = 128, Bk = 64, logF = 7;
+    const uint32_t fl = B.flags;
+    const int nb = B.nbins, nA = B.nA, nJ = B.nJ, nred = B.nred;
+    const bool cic = (fl & F_E0) && (fl & F_CIC);
+    double2 *sX = reinterpret_cast<double2 *>(s_bw);
+    double2 *sW = sX + nA * F, *sY = sW + nJ * F;
+    double *sG = reinterpret_cast<double *>(sY + nA * F);   // the line density, nA * 64
+    double *sP = sG + nA * Bk;
+    const int tid = (int)threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t turn = ((const TurnScalars *)B.sc)->turn;
+    // the binned count, from both halves' counts (this turn's is known a load later)
+    const g_u32 *hist = (const g_u32 *)B.hist;
+    const int bin = min(tid, nb - 1);
+    const uint32_t h0 = hist[bin], h1 = hist[nb + bin];
+    const double lam = ((const g_f64 *)B.lam)[bin];
+    {
+        int r = 0, c = tid;   // s_tw[tid] = w1, wa or wb (c) of stage pair r at butterfly index k
+        if (c >= 30) { r = 2; c -= 30; } else if (c >= 6) { r = 1; c -= 6; }
+        const int hh = 2 << (2 * r), k = c & (hh - 1), sh = 5 - 2 * r;
+        c >>= 2 * r + 1;
+        if (tid < 126)
+            s_tw[tid] = ld2((const g_f64x2 *)B.tw + (c == 0 ? k << sh : (c == 1 ? k : k + hh) << (sh - 1)));
+    }
+    const uint32_t hc = tid < nb ? ((turn & 1) ? h1 : h0) : 0u;
+    {
+        uint32_t c = hc;
+        c += __builtin_amdgcn_update_dpp(0, c, 0xB1, 0xF, 0xF, false);
+        c += __builtin_amdgcn_update_dpp(0, c, 0x4E, 0xF, 0xF, false);
+        c += __builtin_amdgcn_update_dpp(0, c, 0x141, 0xF, 0xF, false);
+        c += __builtin_amdgcn_update_dpp(0, c, 0x140, 0xF, 0xF, false);
+        c += __builtin_amdgcn_update_dpp(0, c, 0x142, 0xA, 0xF, false);
+        c += __builtin_amdgcn_update_dpp(0, c, 0x143, 0x8, 0xF, false);
+        if (lane == 63) s_cnt[wave] = c;   // row sums, then the rows into lane 63
+    }
+    lds_barrier();
+    uint32_t total = 0;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) total += s_cnt[w];
+    const double nh = (double)total;
+    if (tid < nb) ((g_u32 *)B.hist)[((turn + 1) & 1) * nb + tid] = 0u;   // the next turn's half
+    const double inv_nh = 1.0 / nh;
+    if (tid < nA * Bk)   // line_density, in the convolution's order
+        sG[(fl & F_LAG) && tid < nb ? nb - 1 - tid : tid] = tid < nb ? lam * ((double)hc * inv_nh) : 0.0;
+    lds_barrier();
+    // The other loads, by the waves without butterflies and while those run:
+    // waves 8-15 the wake spectra and the pass sums, waves 12-15 this turn's
+    // deposit as well.  (Issued before the density was packed, they held up
+    // its barrier: a CU takes about 16 cycles for each 16-byte-per-lane load.)
+    const int q = tid & 31, blk = tid >> 5;   // this thread's butterfly and its block
+    const bool fft = wave < 8 && blk < nA;
+    double2 R[12];   // waves 8-15: the pass sums' loads, then the spectra's; waves 0-7: the
+                     // twiddles, 3 r + {0, 1, 2} = w1, wa, wb of stages 2r+1, 2r+2
+    uint32_t cnt[4] = {0u, 0u, 0u, 0u};
+    unsigned long long hi[4] = {0ull, 0ull, 0ull, 0ull}, lo[4] = {0ull, 0ull, 0ull, 0ull};
+    uint32_t bad = 0;
+    g_u64 *H = (g_u64 *)B.cic;
+    g_u32 *N = (g_u32 *)(B.cic + 2 * nb);
+    const int ct = tid - 768;   // cic_psum's thread
+    const int npart = B.ntiles * kTileWaves, tl = tid & 255;
+    // group g of the pass sums (whole_sum's slices): waves 8-11 the even ones, 12-15 the odd ones
+    auto load_part = [&](int g) {
+#pragma unroll
+        for (int k = 0; k < kRedPer; ++k) {
+            const int e = g * kRedEntries + tl + k * kRedThreads;
+            double2 a = make_double2(0.0, 0.0), b = make_double2(0.0, 0.0);
+            if (e < npart) {
+                const g_f64x2 *p = (const g_f64x2 *)B.part + 2 * (int64_t)e;
+                a = ld2(p);
+                b = ld2(p + 1);
+            }
+            R[2 * k] = a;
+            R[2 * k + 1] = b;
+        }
+    };
+    const int g0 = wave >= 12 ? 1 : 0;
+    const int nW = nJ * F;
+    if (wave >= 8) {
+        const g_f64x2 *Wg = (const g_f64x2 *)B.What;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) R[8 + u] = ld2(Wg + min(tid - 512 + 512 * u, nW - 1));
+        if (g0 < nred) load_part(g0);
+        if (cic && wave >= 12) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int k = ct + u * kRedThreads;
+                if (k < nb - 1) {
+                    cnt[u] = N[k];
+                    hi[u] = H[k];
+                    lo[u] = H[nb + k];
+                }
+            }
+        }
+    }
+    if (wave >= 8) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (tid - 512 + 512 * u < nW) sW[tid - 512 + 512 * u] = R[8 + u];
+        // the pass sums' slices, block_sum's order within the group
+        for (int g = g0; g < nred; g += 2) {
+            if (g > 1) load_part(g);
+            double v[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int k = 0; k < kRedPer; ++k) {
+                v[0] += R[2 * k].x;
+                v[1] += R[2 * k].y;
+                v[2] += R[2 * k + 1].x;
+                v[3] += R[2 * k + 1].y;
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                v[j] = butterfly(v[j]);
+                if (lane == 0) s_sum[g][j * 16 + (tl >> 6)] = v[j];
+            }
+        }
+    }
+    const bool conv = nh != 0.0;   // else the potential is zero (wakefield.jl:305-311)
+    if (fft) {
+#pragma unroll
+        for (int r = 0; r < 3; ++r) {
+            const int hh = 2 << (2 * r), k = q & (hh - 1), t0 = r == 0 ? 0 : (r == 1 ? 6 : 30);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) R[3 * r + c] = s_tw[t0 + c * hh + k];
+        }
+    }
+    // the thread's places in its block at the stage pairs' strides
+    const int e1 = ((q >> 1) << 3) | (q & 1), e3 = ((q >> 3) << 5) | (q & 7);
+    if (conv && fft) {
+        // stages 1 and 2 on packed points 8 (q >> 1) + (q & 1) + {0, 2, 4, 6},
+        // which stage 0 leaves equal in pairs: input bitrev(8 (q >> 1) + 2 j)
+        double2 y[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int i = blk * Bk + bitrev(8 * (q >> 1) + 2 * j, logF);
+            y[j] = make_double2(sG[i], blk >= 1 ? sG[i - Bk] : 0.0);
+        }
+        dit_pair(y, R[0], R[1], R[2]);
+        double2 *X = sX + blk * F;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) X[swz64(e1 + 2 * j)] = y[j];
+        wave_lds_fence();
+#pragma unroll
+        for (int j = 0; j < 4; ++j) y[j] = X[swz64(e3 + 8 * j)];
+        dit_pair(y, R[3], R[4], R[5]);
+        wave_lds_fence();
+#pragma unroll
+        for (int j = 0; j < 4; ++j) X[swz64(e3 + 8 * j)] = y[j];
+        wave_lds_fence();
+#pragma unroll
+        for (int j = 0; j < 4; ++j) y[j] = X[swz64(q + 32 * j)];
+        dit_pair(y, R[6], R[7], R[8]);
+        wave_lds_fence();
+#pragma unroll
+        for (int j = 0; j < 4; ++j) X[swz64(q + 32 * j)] = y[j];
+    }
+    lds_barrier();
+    if (conv) {
+        // output blocks o0 = 2 og and o0 + 1 at frequency k.  og by wave pair, so
+        // that every SIMD's four waves (w, w + 4, ...) have 68 products
+        constexpr unsigned kGroups = 0x31462057u;   // 7, 5, 0, 2, 6, 4, 1, 3
+        const int o0 = 2 * (int)((kGroups >> (4 * (wave >> 1))) & 7u);
+        const int k = (wave & 1) * 64 + lane, kx = swz64(k);
+        if (o0 < nA) {
+            double2 a0 = make_double2(0.0, 0.0), a1 = a0;
+            double2 x0 = sX[o0 * F + kx], x1 = o0 + 1 < nA ? sX[(o0 + 1) * F + kx] : a0;
+            double2 w = sW[k];
+            // step j: X_{o0-j}, X_{o0+1-j} times FFT(W_j); the next step's two
+            // values are read before this step's products
+            const int jm = min(o0, nJ - 1);
+            for (int j = 0; j <= jm; ++j) {
+                const double2 wn = sW[min(j + 1, nJ - 1) * F + k];
+                const double2 xn = sX[max(o0 - j - 1, 0) * F + kx];
+                a0 = cadd(a0, cmul(x0, w));
+                a1 = cadd(a1, cmul(x1, w));
+                x1 = x0;
+                x0 = xn;
+                w = wn;
+            }
+            if (jm + 1 < nJ) a1 = cadd(a1, cmul(x1, w));   // j = o0 + 1: block o0 + 1 alone
+            sY[o0 * F + kx] = a0;
+            if (o0 + 1 < nA) sY[(o0 + 1) * F + kx] = a1;
+        }
+    }
+    lds_barrier();
+    TurnScalars sc;
+    if (tid == kScalarThread) {   // whole_sum's and slices_done's order
+        sc = *B.sc;
+        if (cic) bad = N[nb];
+        double t[4] = {0.0, 0.0, 0.0, 0.0};
+        for (int r = 0; r < nred; ++r)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                double s = 0.0;
+                for (int w = 0; w < 4; ++w) s += s_sum[r][j * 16 + w];
+                t[j] = nred == 1 ? s : t[j] + s;
+            }
+        bin_scalars_on(B, t, sc);
+        s_cur = sc.current;
+    }
+    g_f64 *P = (g_f64 *)B.P;
+    double2 y[4];
+    if (conv && fft) {
+        double2 *Y = sY + blk * F;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) y[j] = Y[swz64(q + 32 * j)];
+        dif_pair(y, conj2(R[7]), conj2(R[8]), conj2(R[6]));
+        wave_lds_fence();
+#pragma unroll
+        for (int j = 0; j < 4; ++j) Y[swz64(q + 32 * j)] = y[j];
+        wave_lds_fence();
+#pragma unroll
+        for (int j = 0; j < 4; ++j) y[j] = Y[swz64(e3 + 8 * j)];
+        dif_pair(y, conj2(R[4]), conj2(R[5]), conj2(R[3]));
+        wave_lds_fence();
+#pragma unroll
+        for (int j = 0; j < 4; ++j) Y[swz64(e3 + 8 * j)] = y[j];
+        wave_lds_fence();
+#pragma unroll
+        for (int j = 0; j < 4; ++j) y[j] = Y[swz64(e1 + 2 * j)];
+        dif_pair(y, conj2(R[1]), conj2(R[2]), conj2(R[0]));
+    }
+    lds_barrier();   // the current (kScalarThread)
+    if (conv && fft) {
+        // stage 0 on points 8 (q >> 1) + 2 j (this lane or its neighbour, even q)
+        // and the one after it (odd q): output m = bitrev(8 (q >> 1) + 2 j) is
+        // Re of their sum plus Im of their difference times tw[0]; even lanes
+        // take j = 0, 1, odd lanes j = 2, 3
+        const bool odd = q & 1;
+        const double2 s0 = dpp_swap1(odd ? y[0] : y[2]), s1 = dpp_swap1(odd ? y[1] : y[3]);
+        const double2 w0 = conj2(ld2((const g_f64x2 *)B.tw));
+        const double scale = s_cur / (double)F;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const double2 s = u ? s1 : s0;
+            const double2 a = odd ? s : y[u], c = odd ? y[2 + u] : s;
+            const int i = blk * Bk + bitrev(8 * (q >> 1) + 2 * (u + (odd ? 2 : 0)), logF);
+            const double2 d = csub(a, c);
+            const double p = (cadd(a, c).x + (d.x * w0.y + d.y * w0.x)) * scale;
+            if (i < nb) {
+                const int k = (fl & F_LAG) ? nb - 1 - i : i;
+                P[k] = p;
+                sP[k] = p;
+            }
+        }
+    } else if (!conv && tid < nb) {
+        P[tid] = 0.0;
+        sP[tid] = 0.0;
+    }
+    lds_barrier();
+    double t = 0.0;
+    if (cic) {   // cic_psum's cells per thread and order
+        if (wave >= 12) {
+            double a = 0.0;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int k = ct + u * kRedThreads;
+                if (cnt[u]) {
+                    const double sk = ((double)hi[u] * 0x1p32 + (double)lo[u]) * (1.0 / kCicScale);
+                    a += ((double)cnt[u] - sk) * sP[k] + sk * sP[k + 1];
+                    N[k] = 0u;
+                    H[k] = 0ull;
+                    H[nb + k] = 0ull;
+                }
+            }
+            a = butterfly(a);
+            if (lane == 0) s_red[wave - 12] = a;
+        }
+        lds_barrier();
+        if (tid == kScalarThread) {
+            for (int w = 0; w < kRedThreads / 64; ++w) t += s_red[w];
+            if (bad) {
+                N[nb] = 0u;
+                t = __builtin_nan("");
+            }
+            if (nred != 1) t = 0.0 + t;
+        }
+    }
+    if (tid == kScalarThread) {
         finish_on(B, t, sc);
         *B.sc = sc;
     }
@@ -2463,7 +2848,7 @@ hipError_t configure_kernels(int lds) {
                          (const void *)k_conv_spec, (const void *)k_conv_out,
                          (const void *)k_fft_wake, (const void *)k_stage_hist,
                          (const void *)k_interp_sum, (const void *)k_interp_sum_deep,
-                         (const void *)k_bin_whole};
+                         (const void *)k_bin_whole, (const void *)k_bin_64};
     hipError_t last = hipSuccess;
     for (const void *f : fns) {
         hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
@@ -2566,6 +2951,13 @@ hipError_t launch_bin_whole(const BunchDev *bds, const int32_t *list, int nb, si
                             hipStream_t s) {
     if (nb <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_bin_whole, dim3(nb), dim3(1024), lds, s, bds, list);
+    return hipGetLastError();
+}
+
+hipError_t launch_bin_64(const BunchDev *bds, const int32_t *list, int nb, size_t lds,
+                         hipStream_t s) {
+    if (nb <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_bin_64, dim3(nb), dim3(1024), lds, s, bds, list);
     return hipGetLastError();
 }
 

@@ -126,6 +126,18 @@ __host__ __device__ inline BinWholeLayout bin_whole_layout(int nb, int nA, int n
 }
 hipError_t launch_bin_whole(const BunchDev *bds, const int32_t *bunch_list, int nb, size_t lds,
                             hipStream_t s);
+// The same for the bunches that fit k_bin_64's arrangement: blocks of 64 bins
+// (what the tuned table gives 256 to 1024 bins), at most 16 of them, a wake of
+// more than one block (one block has nothing to sum), at most four reduction
+// slices, and the whole potential in the pass's window `win` (k_bin_64 leaves
+// the neighbour-pair table out).  Same bits; in a turn 9.5 us against 17.7 us
+// at 1024 bins, 7.4 against 12.7 us at 512.  Its LDS fits in
+// bin_whole_layout(...).bytes.
+inline bool fits_bin_64(bool wake, int nbins, int win, int nA, int nJ, int F, int nred) {
+    return wake && F == 128 && nbins >= 2 && nA <= 16 && nJ > 1 && nJ <= 16 && nred <= 4 && win >= nbins;
+}
+hipError_t launch_bin_64(const BunchDev *bds, const int32_t *bunch_list, int nb, size_t lds,
+                         hipStream_t s);
 // Broadband resonators of a lag-indexed wake table, (R_s [Ohm], f_r [Hz], Q)
 // each, passed by value.
 constexpr int kMaxResonators = 8;
