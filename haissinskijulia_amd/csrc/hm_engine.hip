@@ -388,7 +388,7 @@ static void balanced_ranges(const std::vector<int64_t> &w, const std::vector<int
 Batch::~Batch() {
     drop_graph();
     for (auto e : ev_pool_) (void)hipEventDestroy(e);
-    d_bd_.release(); d_runs_.release(); d_order_.release();
+    d_bd_.release(); d_runs_.release(); d_order_.release(); d_free_.release();
     for (auto &c : d_conv_) c.release();
     d_red_.release(); d_list_.release(); d_bw_.release();
     d_tmp_tiles_.release(); d_tmp_list_.release(); d_ranges_.release();
@@ -415,8 +415,57 @@ hm_status Batch::stage_descriptors() {
     return stage_copy(ctx_, d_bd_.p, h.data(), h.size() * sizeof(BunchDev));
 }
 
-// launch tables of the active bunches
+// Launch tables of the active bunches.  Where none of them has a wake or the
+// E0 update, k_free_turns advances them by many turns at a time: its items are
+// all that is built.
+hm_status Batch::build_free_tables() {
+    std::vector<RunDev> items;
+    std::vector<int32_t> list;
+    free_pairs_ = 0;
+    for (size_t i = 0; i < rb_.size(); ++i)
+        if (used_[i] && rb_[i].active) free_pairs_ += rb_[i].d.npairs;
+    // one pair per thread until that fills the SIMDs several times over, then
+    // four in turn (3e6 particles: 6 rounds of waves either way), and at most
+    // about 65536 items
+    int64_t per_thread = free_pairs_ > (int64_t)kFreeThreads * 32 * ctx_->cus ? 4 : 1;
+    per_thread = std::max(per_thread, free_pairs_ / ((int64_t)kFreeThreads << 16) + 1);
+    const int64_t chunk = kFreeThreads * per_thread;
+    for (size_t i = 0; i < rb_.size(); ++i) {
+        if (!used_[i] || !rb_[i].active) continue;
+        list.push_back((int32_t)i);
+        const int64_t np = rb_[i].d.npairs;
+        for (int64_t p = 0; p < np; p += chunk)
+            items.push_back({(int32_t)i, (int32_t)p, (int32_t)std::min(chunk, np - p)});
+    }
+    nfree_ = (int)items.size();
+    nlist_ = (int)list.size();
+    HM_TRY(d_free_.ensure(std::max<size_t>(items.size(), 1)));
+    HM_TRY(d_list_.ensure(std::max<size_t>(list.size(), 1)));
+    HM_TRY(stage_begin(ctx_, stage_size(items.size() * sizeof(RunDev)) + stage_size(list.size() * 4) +
+                                 stage_size(rb_.size() * sizeof(BunchDev))));
+    HM_TRY(stage_copy(ctx_, d_free_.p, items.data(), items.size() * sizeof(RunDev)));
+    HM_TRY(stage_copy(ctx_, d_list_.p, list.data(), list.size() * 4));
+    HM_TRY(stage_descriptors());
+    HM_TRY(stage_end(ctx_));
+    dirty_ = false;
+    return HM_OK;
+}
+
+// turns of the free bunches, at most about 4e9 pair-turns (40 ms) per launch
+hm_status Batch::free_turns(int64_t turns) {
+    const int64_t most = std::min<int64_t>(
+        1 << 20, std::max<int64_t>(1, (int64_t)4e9 / std::max<int64_t>(1, free_pairs_)));
+    for (int64_t t = 0; t < turns; t += most)
+        HIP_TRY(launch_free_turns(d_bd_.p, d_free_.p, nfree_, d_list_.p, nlist_,
+                                  (int)std::min(most, turns - t), ctx_->stream));
+    return HM_OK;
+}
+
 hm_status Batch::build_tables() {
+    free_only_ = !timing_;   // timing asks for one launch of the pass per turn
+    for (size_t i = 0; i < rb_.size(); ++i)
+        if (used_[i] && rb_[i].active && (rb_[i].d.flags & (F_WAKE | F_E0))) free_only_ = false;
+    if (free_only_) return build_free_tables();
     std::vector<int32_t> tiles, conv[kConvKinds], red, list, bw, b64;
     pass_lds_ = 0;
     bw_lds_ = 0;
@@ -1075,7 +1124,10 @@ hm_status Batch::advance(int64_t turns) {
         for (size_t i = 0; i < rb_.size(); ++i)
             if (used_[i] && rb_[i].active) active_particles += rb_[i].d.n;
         int64_t did = 1;
-        if (graphs_ && !timing_ && left >= kGraphTurns && active_particles < kGraphMaxParticles) {
+        if (free_only_) {
+            HM_TRY(free_turns(left));
+            did = left;
+        } else if (graphs_ && !timing_ && left >= kGraphTurns && active_particles < kGraphMaxParticles) {
             if (!graph_exec_) HM_TRY(capture_graph());
             HIP_TRY(hipGraphLaunch(graph_exec_, ctx_->stream));
             did = kGraphTurns;

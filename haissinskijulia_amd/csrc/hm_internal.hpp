@@ -213,11 +213,13 @@ class Batch {
   private:
     hm_status add_slots(const std::vector<RunBunch> &specs, std::vector<int32_t> &fresh);
     hm_status build_tables();
+    hm_status build_free_tables();
     hm_status upload_descriptors();
     hm_status stage_descriptors();
     hm_status run_subset_moments(const std::vector<int32_t> &which, int mode);
     hm_status epilogue(const std::vector<int32_t> &which);
     hm_status one_turn();
+    hm_status free_turns(int64_t turns);
     hm_status flush_timing();
     hm_status capture_graph();
     void drop_graph();
@@ -240,6 +242,12 @@ class Batch {
     DevBuf<int32_t> d_ranges_;
     int pass_grid_ = 0, interp_grid_ = 0;
     bool interp_deep_ = false;   // one interpolation workgroup per CU: deeper rings
+    // no active bunch needs a sum over its particles between turns: the items
+    // of k_free_turns, and the pairs they cover
+    bool free_only_ = false;
+    int nfree_ = 0;
+    int64_t free_pairs_ = 0;
+    DevBuf<RunDev> d_free_;
     DevBuf<int32_t> d_conv_[kConvKinds];   // convolution items of each ConvKind
     DevBuf<int32_t> d_red_;       // (bunch, slice) items of the reductions
     DevBuf<int32_t> d_list_;      // the active bunches of the launch-per-phase bin phase

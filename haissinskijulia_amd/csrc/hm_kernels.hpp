@@ -74,6 +74,11 @@ hipError_t launch_init(const BunchDev *bds, const int32_t *bunch_list, int nb, h
 // bins or more
 hipError_t launch_turn_pass(const BunchDev *bds, const int32_t *order, const RunDev *runs,
                             const int32_t *rr, int grid, size_t lds, int std_only, hipStream_t s);
+// `turns` turns of bunches without a wake and without the E0 update: items
+// cover the listed bunches' pairs
+constexpr int kFreeThreads = 256;
+hipError_t launch_free_turns(const BunchDev *bds, const RunDev *items, int nitems,
+                             const int32_t *bunch_list, int nlist, int turns, hipStream_t s);
 // items are (bunch, block) pairs, for CONV_SPEC (bunch, frequency chunk)
 // pairs; Fmax is the largest FFT length among them, for CONV_SPEC the largest
 // conv_spec_lds of their bunches in bytes
