@@ -390,7 +390,7 @@ Batch::~Batch() {
     for (auto e : ev_pool_) (void)hipEventDestroy(e);
     d_bd_.release(); d_runs_.release(); d_order_.release(); d_free_.release();
     for (auto &c : d_conv_) c.release();
-    d_red_.release(); d_list_.release(); d_bw_.release();
+    d_red_.release(); d_slab_.release(); d_list_.release(); d_bw_.release();
     d_tmp_tiles_.release(); d_tmp_list_.release(); d_ranges_.release();
 }
 
@@ -435,7 +435,7 @@ hm_status Batch::build_free_tables() {
         list.push_back((int32_t)i);
         const int64_t np = rb_[i].d.npairs;
         for (int64_t p = 0; p < np; p += chunk)
-            items.push_back({(int32_t)i, (int32_t)p, (int32_t)std::min(chunk, np - p)});
+            items.push_back({(int32_t)i, (int32_t)p, (int32_t)std::min(chunk, np - p), -1});
     }
     nfree_ = (int)items.size();
     nlist_ = (int)list.size();
@@ -466,7 +466,7 @@ hm_status Batch::build_tables() {
     for (size_t i = 0; i < rb_.size(); ++i)
         if (used_[i] && rb_[i].active && (rb_[i].d.flags & (F_WAKE | F_E0))) free_only_ = false;
     if (free_only_) return build_free_tables();
-    std::vector<int32_t> tiles, conv[kConvKinds], red, list, bw, b64;
+    std::vector<int32_t> tiles, conv[kConvKinds], red, list, bw, b64, slab;
     pass_lds_ = 0;
     bw_lds_ = 0;
     spec_lds_ = 0;
@@ -491,7 +491,15 @@ hm_status Batch::build_tables() {
         if (!used_[i] || !q.active) continue;
         q.d.tile_begin = (int32_t)tiles.size();
         for (int t = 0; t < q.d.ntiles; ++t) tiles.push_back((int32_t)i);
-        if ((q.d.flags & kPhysMask) != kStdFlags || q.d.nbins < 2) std_only_ = false;
+        if ((q.d.flags & kPhysMask) != kStdFlags || q.d.nbins < 2 ||
+            ((q.d.flags & F_GHIST) && q.d.hwin == 0))
+            std_only_ = false;
+        q.d.nslabs = 0;
+        if ((q.d.flags & F_WAKE) && (q.d.flags & F_GHIST) && q.d.hwin > 0)
+            for (int g = 0; g * 512 < q.d.hwin; ++g) {
+                slab.push_back((int32_t)i);
+                slab.push_back(g);
+            }
         if (q.d.flags & F_WAKE) pass_lds_ = std::max(pass_lds_, (size_t)pass_lds_bytes(q.d));
         // the whole bin phase in one workgroup (k_bin_whole) for a small bunch
         // without interpolation sums; the other bunches take a launch per phase
@@ -584,37 +592,50 @@ hm_status Batch::build_tables() {
     deal_tiles(tiles, ranges.data(), pass_grid_, order);
     deal_tiles(tiles, ranges.data() + pass_grid_ + 1, interp_grid_, order);
     // each workgroup's entries as runs of one bunch, a bunch with the deposit
-    // at most cic_tiles at a time; then `ranges` counts runs instead of tiles
+    // at most cic_tiles at a time, one with 16-bit counts kHistRunPairs pairs;
+    // then `ranges` counts runs instead of tiles
     std::vector<RunDev> runs;
-    auto find_runs = [&](size_t r0, int grid, size_t base) {
+    auto find_runs = [&](size_t r0, int grid, size_t base, bool pass) {
         for (int g = 0; g <= grid; ++g) {
             const int32_t e0 = g < grid ? ranges[r0 + (size_t)g] : 0;
             const int32_t e1 = g < grid ? ranges[r0 + (size_t)g + 1] : 0;
             ranges[r0 + (size_t)g] = (int32_t)runs.size();
             for (int32_t e = e0; e < e1;) {
                 const int32_t b = tiles[(size_t)order[base + (size_t)e]];
-                const BunchDev &d = rb_[(size_t)b].d;
-                const int32_t em = (d.flags & F_CIC) ? e + std::min(e1 - e, d.cic_tiles) : e1;
+                BunchDev &d = rb_[(size_t)b].d;
+                const bool window = pass && (d.flags & F_GHIST) && d.hwin > 0;
+                int32_t em = e1;
+                if (d.flags & F_CIC) em = e + std::min(e1 - e, d.cic_tiles);
+                if (window)
+                    em = e + (int32_t)std::min<int64_t>(e1 - e, kHistRunPairs / d.pairs_per_tile);
                 int32_t ee = e + 1;
                 while (ee < em && tiles[(size_t)order[base + (size_t)ee]] == b) ++ee;
-                runs.push_back({b, (int32_t)base + e, ee - e});
+                runs.push_back({b, (int32_t)base + e, ee - e, window ? d.nslabs++ : -1});
                 e = ee;
             }
         }
     };
-    if (pass_grid_ > 0) find_runs(0, pass_grid_, 0);
-    if (interp_grid_ > 0) find_runs((size_t)pass_grid_ + 1, interp_grid_, (size_t)ntiles_);
+    if (pass_grid_ > 0) find_runs(0, pass_grid_, 0, true);
+    if (interp_grid_ > 0) find_runs((size_t)pass_grid_ + 1, interp_grid_, (size_t)ntiles_, false);
+    nslab_ = (int)slab.size() / 2;
+    for (size_t i = 0; i < rb_.size(); ++i)
+        if (used_[i] && rb_[i].active && rb_[i].d.nslabs > 0) {
+            BunchDev &d = rb_[i].d;
+            HM_TRY(rb_[i].b->w.slabs.ensure((size_t)d.nslabs * (size_t)(d.hwin / 2)));
+            d.slabs = rb_[i].b->w.slabs.p;
+        }
     // one staging round for every table and the descriptors
     size_t bytes = stage_size(ranges.size() * 4) + stage_size(list.size() * 4) +
                    stage_size(bw.size() * 4) +
-                   stage_size(red.size() * 4) + stage_size(runs.size() * sizeof(RunDev)) +
-                   stage_size(order.size() * 4) +
+                   stage_size(red.size() * 4) + stage_size(slab.size() * 4) +
+                   stage_size(runs.size() * sizeof(RunDev)) + stage_size(order.size() * 4) +
                    stage_size(rb_.size() * sizeof(BunchDev));
     for (int k = 0; k < kConvKinds; ++k) bytes += stage_size(conv[k].size() * 4);
     HM_TRY(d_ranges_.ensure(std::max<size_t>(ranges.size(), 1)));
     HM_TRY(d_runs_.ensure(std::max<size_t>(runs.size(), 1)));
     HM_TRY(d_order_.ensure(std::max<size_t>(order.size(), 1)));
     HM_TRY(d_red_.ensure(std::max<size_t>(red.size(), 2)));
+    HM_TRY(d_slab_.ensure(std::max<size_t>(slab.size(), 2)));
     HM_TRY(d_list_.ensure(std::max<size_t>(list.size(), 1)));
     HM_TRY(d_bw_.ensure(std::max<size_t>(bw.size(), 1)));
     for (int k = 0; k < kConvKinds; ++k) {
@@ -626,6 +647,7 @@ hm_status Batch::build_tables() {
     HM_TRY(stage_copy(ctx_, d_list_.p, list.data(), list.size() * 4));
     HM_TRY(stage_copy(ctx_, d_bw_.p, bw.data(), bw.size() * 4));
     HM_TRY(stage_copy(ctx_, d_red_.p, red.data(), red.size() * 4));
+    HM_TRY(stage_copy(ctx_, d_slab_.p, slab.data(), slab.size() * 4));
     for (int k = 0; k < kConvKinds; ++k)
         HM_TRY(stage_copy(ctx_, d_conv_[k].p, conv[k].data(), conv[k].size() * 4));
     HM_TRY(stage_copy(ctx_, d_runs_.p, runs.data(), runs.size() * sizeof(RunDev)));
@@ -915,9 +937,15 @@ hm_status Batch::add_slots(const std::vector<RunBunch> &specs, std::vector<int32
         d.logF = ilog2(d.F);
         d.nA = (int32_t)((nb + Bk - 1) / Bk);
         d.nJ = (int32_t)((nw + Bk - 1) / Bk);
-        // the histogram in LDS only with room for a window of at least two
-        // entries of P beside it (the all-flags pass relies on that)
-        if ((size_t)nb * 4 + 16 > (size_t)ctx_->lds_max - 1024) d.flags |= F_GHIST;
+        // The whole histogram in LDS only with room for a window of at least
+        // two entries of P beside it (the all-flags pass relies on that), or,
+        // where a window of 16-bit counts can take its place (a tile's counts
+        // fit them), of kHistMinWin.
+        const bool hwin = d.pairs_per_tile <= kHistRunPairs && d.npairs <= kHistMaxPairs;
+        if ((size_t)nb * 4 + 8 * (size_t)(hwin ? kHistMinWin : 2) > (size_t)ctx_->lds_max - 1024) {
+            d.flags |= F_GHIST;
+            d.hwin = hwin ? (int32_t)std::min<int64_t>(nb, kHistWin) & ~1 : 0;
+        }
         // With update_E0 the pass deposits the interpolation weights of its
         // post-drift z (cloud in cell) where its LDS holds the counters beside
         // the histogram and the whole table of P, instead of the interpolation
@@ -1025,6 +1053,7 @@ hm_status Batch::one_turn() {
     HIP_TRY(launch_turn_pass(d_bd_.p, d_order_.p, d_runs_.p, d_ranges_.p, pass_grid_, pass_lds_,
                              std_only_ ? 1 : 0, s));
     if (timing_) HIP_TRY(hipEventRecord(e1, s));
+    HIP_TRY(launch_hist_slabs(d_bd_.p, d_slab_.p, nslab_, s));
     HIP_TRY(launch_bin_64(d_bd_.p, d_bw_.p, nb64_, bw_lds_, s));
     HIP_TRY(launch_bin_whole(d_bd_.p, d_bw_.p + nb64_, nbw_, bw_lds_, s));
     const bool whole = nlist_ >= kWholeMinBunches;

@@ -87,20 +87,20 @@ struct DevBuf {
 
 // per-bunch work buffers of an evolve call (kept between calls)
 struct Work {
-    DevBuf<uint32_t> hist;
+    DevBuf<uint32_t> hist, slabs;
     DevBuf<double> P, P2, lam, What, X, Wtmp, part, ipart, moments, normals, out, stats, mon;
     DevBuf<TurnScalars> sc;
     DevBuf<double> red, Y;
     DevBuf<uint32_t> cnt;
     DevBuf<unsigned long long> cic;
     void release() {
-        hist.release(); P.release(); P2.release(); lam.release(); What.release(); X.release();
+        hist.release(); slabs.release(); P.release(); P2.release(); lam.release(); What.release(); X.release();
         Wtmp.release(); part.release(); ipart.release(); moments.release(); normals.release();
         out.release(); stats.release(); mon.release(); sc.release(); red.release(); cnt.release();
         Y.release(); cic.release();
     }
     size_t bytes() const {
-        return hist.bytes() + P.bytes() + P2.bytes() + lam.bytes() + What.bytes() + X.bytes() +
+        return hist.bytes() + slabs.bytes() + P.bytes() + P2.bytes() + lam.bytes() + What.bytes() + X.bytes() +
                Wtmp.bytes() + part.bytes() + ipart.bytes() + moments.bytes() + normals.bytes() +
                out.bytes() + stats.bytes() + mon.bytes() + sc.bytes() + red.bytes() + cnt.bytes() +
                Y.bytes() + cic.bytes();
@@ -250,6 +250,8 @@ class Batch {
     DevBuf<RunDev> d_free_;
     DevBuf<int32_t> d_conv_[kConvKinds];   // convolution items of each ConvKind
     DevBuf<int32_t> d_red_;       // (bunch, slice) items of the reductions
+    DevBuf<int32_t> d_slab_;      // (bunch, group of bins) items of the windowed histograms
+    int nslab_ = 0;
     DevBuf<int32_t> d_list_;      // the active bunches of the launch-per-phase bin phase
     DevBuf<int32_t> d_bw_;        // the active bunches of k_bin_64, then of k_bin_whole
     int ntiles_ = 0, nred_ = 0, nlist_ = 0, nbw_ = 0, nb64_ = 0;

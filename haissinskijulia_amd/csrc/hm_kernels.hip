@@ -617,20 +617,25 @@ __device__ __forceinline__ uint8_t *pass_lds() {
     return s_lds;
 }
 
-// LH: the histogram is in LDS (else straight to global memory).  v[3] counts
+// HM: the histogram is in LDS, straight in global memory, or its window from bin
+// hlo in 16-bit LDS counts and the rest in global memory.  v[3] counts
 // the particles that are not binned (a branch most waves skip), n_bad (CIC
 // only) the NaN positions among them, one atomic each.
-template <bool LH, bool CIC>
-__device__ __forceinline__ void bin_and_sum(const PassCtx &c, g_u32 *ghist, g_u32 *n_bad, double z,
-                                            double (&v)[4]) {
+enum HistMode { kHistGlobal = 0, kHistLds = 1, kHistWindow = 2 };
+template <int HM, bool CIC>
+__device__ __forceinline__ void bin_and_sum(const PassCtx &c, g_u32 *ghist, int hlo, int hwin,
+                                            g_u32 *n_bad, double z, double (&v)[4]) {
     v[0] += z;
     v[1] = __builtin_fma(z, z, v[1]);
     // hist_bin with its range test as the branch: in range, u = (z - e0) * inv
     // is >= 0, and its conversion to int (truncation) is floor(u)
     if ((z >= c.e0) & (z <= c.e1)) {
         const int b = min((int)((z - c.e0) * c.inv_step), c.nb - 1);
-        if (LH)
+        const unsigned w = (unsigned)(b - hlo);
+        if (HM == kHistLds)
             atomicAdd(reinterpret_cast<uint32_t *>(pass_lds()) + b, 1u);
+        else if (HM == kHistWindow && w < (unsigned)hwin)
+            atomicAdd(reinterpret_cast<uint32_t *>(pass_lds()) + (w >> 1), 1u << (16 * (w & 1)));
         else
             __hip_atomic_fetch_add(ghist + b, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     } else {
@@ -665,7 +670,8 @@ __device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlan
 // The fused pass over a run of tiles.  FX = kStdFlags is the common configuration
 // with the flags folded at compile time; FX = 0 handles any other.  Both
 // evaluate the same expressions, so a bunch gets the same bits from either.
-// LH: histogram in LDS at offset 0; the window of P follows at byte hb.
+// HM: where the histogram is (bin_and_sum), in LDS at offset 0; the window of P
+// follows at byte hb.
 //
 // One call covers the run's tiles run[0..cnt) of bunch B (indices into the
 // tile table, in ascending order but not necessarily adjacent: a bunch shared
@@ -690,7 +696,7 @@ __device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlan
 // With FX = kStdFlags the kick is applied from the first turn on: P is zero
 // before it, and subtracting 0 changes nothing.
 enum KickMode { kFullWindow = 0, kGatherFirst = 1, kPrefetchFirst = 2 };
-template <uint32_t FX, bool LH, int KM, bool CIC>
+template <uint32_t FX, int HM, int KM, bool CIC>
 __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *__restrict__ run,
                                               int cnt, int hb, int cb) {
     PassCtx c;
@@ -718,6 +724,8 @@ __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *
     g_f64 *zp = (g_f64 *)B.z;
     g_f64 *ep = (g_f64 *)B.dE;
     g_u32 *ghist = (g_u32 *)hist_of(B, sc.turn);
+    const int hwin = B.hwin;
+    const int hlo = HM == kHistWindow ? uni(window_lo(sc.centre_bin, hwin, c.nb)) : 0;
     g_u32 *n_bad = CIC ? (g_u32 *)(B.cic + 2 * (int64_t)c.nb) + c.nb : nullptr;
     const unsigned tid = threadIdx.x;
     const int wave = uni((int)(tid >> 6));
@@ -799,8 +807,8 @@ __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *
                     q1 = make_double2(sP[k1], sP[k1 + 1]);
                 } else {
                     const unsigned j0 = (unsigned)(k0 - wlo), j1 = (unsigned)(k1 - wlo);
-                    // any window of the all-flags pass (its histogram is in LDS,
-                    // so its window has at least two entries) has wpairs >= 1
+                    // any window of the all-flags pass (its histogram's share of
+                    // the LDS leaves at least two entries) has wpairs >= 1
                     if (FX != 0 || wpairs) {
                         const unsigned i0 = min(j0, wpairs - 1), i1 = min(j1, wpairs - 1);
                         q0 = make_double2(sP[i0], sP[i0 + 1]);
@@ -857,8 +865,8 @@ __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *
             __builtin_amdgcn_s_waitcnt(0x0F70);
             if (tid < lim) {
                 if (wake) {
-                    bin_and_sum<LH, CIC>(c, ghist, n_bad, z0, v);
-                    bin_and_sum<LH, CIC>(c, ghist, n_bad, z1, v);
+                    bin_and_sum<HM, CIC>(c, ghist, hlo, hwin, n_bad, z0, v);
+                    bin_and_sum<HM, CIC>(c, ghist, hlo, hwin, n_bad, z1, v);
                 }
                 if (CIC) {
                     cic_deposit(c, cb, z0);
@@ -890,7 +898,7 @@ __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *
             e0 = apply_pending(c, z0, e0);
             double d0;
             advance(c, fl, z0, e0, r0, d0);
-            if (wake) bin_and_sum<LH, CIC>(c, ghist, n_bad, z0, v);
+            if (wake) bin_and_sum<HM, CIC>(c, ghist, hlo, hwin, n_bad, z0, v);
             if (CIC) cic_deposit(c, cb, z0);
             v[2] += d0;
             zp[i] = z0;
@@ -901,11 +909,18 @@ __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *
     }
 }
 
-// Adds the LDS histogram of bunch B into this turn's global counts.
-__device__ inline void flush_hist(const BunchDev &B) {
+// Adds the LDS histogram of bunch B into this turn's global counts; a windowed
+// one goes to the run's slab as it is.
+__device__ inline void flush_hist(const BunchDev &B, int slab) {
     if (!pass_hist_bytes(B)) return;
     __syncthreads();
     const uint32_t *s_hist = reinterpret_cast<const uint32_t *>(pass_lds());
+    if (B.flags & F_GHIST) {
+        const int words = B.hwin / 2;
+        g_u32 *o = (g_u32 *)B.slabs + (int64_t)slab * words;
+        for (int w = threadIdx.x; w < words; w += blockDim.x) o[w] = s_hist[w];
+        return;
+    }
     g_u32 *g = (g_u32 *)hist_of(B, B.sc->turn);
     for (int b = threadIdx.x; b < B.nbins; b += blockDim.x) {
         const uint32_t h = s_hist[b];
@@ -963,8 +978,6 @@ __device__ __forceinline__ void turn_pass_blocks(const BunchDev *__restrict__ bd
                                                  const int32_t *__restrict__ order,
                                                  const RunDev *__restrict__ runs,
                                                  const int32_t *__restrict__ rr) {
-    // kStdFlags has the wake on and F_GHIST off: its histogram is in LDS
-    constexpr bool kLdsOnly = (FX & F_WAKE) && !(FX & F_GHIST);
     const int r1 = rr[blockIdx.x + 1];
     for (int r = rr[blockIdx.x]; r < r1; ++r) {
         const RunDev rd = runs[r];
@@ -978,22 +991,19 @@ __device__ __forceinline__ void turn_pass_blocks(const BunchDev *__restrict__ bd
         constexpr int kPartial = FX != 0 ? kGatherFirst : kPrefetchFirst;
         const bool full = B.win >= B.nbins;
         const int cb = B.cic_off;
-        if (kLdsOnly || hb) {
-            if (B.flags & F_CIC) {   // the deposit comes with the whole table
-                turn_pass_run<FX, true, kFullWindow, true>(B, run, cnt, hb, cb);
-            } else {
-                if (full)
-                    turn_pass_run<FX, true, kFullWindow, false>(B, run, cnt, hb, cb);
-                else
-                    turn_pass_run<FX, true, kPartial, false>(B, run, cnt, hb, cb);
-            }
-        } else {
+        if (B.flags & F_CIC) {   // the deposit comes with the whole table
+            turn_pass_run<FX, kHistLds, kFullWindow, true>(B, run, cnt, hb, cb);
+        } else if (!(B.flags & F_GHIST)) {   // a bunch without a wake among them
             if (full)
-                turn_pass_run<FX, false, kFullWindow, false>(B, run, cnt, hb, cb);
+                turn_pass_run<FX, kHistLds, kFullWindow, false>(B, run, cnt, hb, cb);
             else
-                turn_pass_run<FX, false, kPrefetchFirst, false>(B, run, cnt, hb, cb);
+                turn_pass_run<FX, kHistLds, kPartial, false>(B, run, cnt, hb, cb);
+        } else if (FX != 0 || B.hwin > 0) {
+            turn_pass_run<FX, kHistWindow, kPartial, false>(B, run, cnt, hb, cb);
+        } else {
+            turn_pass_run<FX, kHistGlobal, kPrefetchFirst, false>(B, run, cnt, hb, cb);
         }
-        flush_hist(B);
+        flush_hist(B, rd.slab);
     }
 }
 
@@ -1004,7 +1014,8 @@ __global__ __launch_bounds__(kPassThreads) void k_turn_pass(const BunchDev *__re
     turn_pass_blocks<0>(bds, order, runs, rr);
 }
 
-// the same for tables whose bunches all have exactly kStdFlags and two bins or more
+// the same for tables whose bunches all have exactly kStdFlags, two bins or more
+// and some of their histogram in LDS
 __global__ __launch_bounds__(kPassThreads) void k_turn_pass_std(const BunchDev *__restrict__ bds,
                                                                 const int32_t *__restrict__ order,
                                                                 const RunDev *__restrict__ runs,
@@ -1289,6 +1300,43 @@ __device__ inline void whole_sum(const BunchDev &B, const double *a, double (&t)
 #pragma unroll
                 for (int j = 0; j < NV; ++j) t[j] = nred == 1 ? s_slice[q][j] : t[j] + s_slice[q][j];
         __syncthreads();
+    }
+}
+
+// The counts of the LDS windows, slab by slab, added to this turn's histogram:
+// a workgroup takes 256 words (512 bins) of one bunch's window, each of its
+// four groups of waves a quarter of the slabs with 16 loads in flight.  Before
+// k_bin_reduce, which moves the centroid that places the window.  Bound by the
+// 25 MB of 256 slabs: 8 us with its launch, where flushing 49152 bins of every
+// workgroup by atomics would take about 28 (14 us per 6.3e6 of them).
+__global__ __launch_bounds__(1024) void k_hist_slabs(const BunchDev *__restrict__ bds,
+                                                     const int32_t *__restrict__ items) {
+    __shared__ uint32_t s_part[4][512];
+    const BunchDev &B = bds[items[2 * blockIdx.x]];
+    const int words = B.hwin / 2, col = (int)threadIdx.x & 255, grp = (int)threadIdx.x >> 8;
+    const int w = items[2 * blockIdx.x + 1] * 256 + col;
+    const g_u32 *slab = (const g_u32 *)B.slabs + min(w, words - 1);
+    const int n = B.nslabs, q = (n + 3) / 4, s1 = min(n, (grp + 1) * q);
+    uint32_t lo = 0, hi = 0;
+    for (int s = grp * q; s < s1; s += 16) {
+        uint32_t x[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) x[u] = s + u < s1 ? slab[(int64_t)(s + u) * words] : 0u;
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            lo += x[u] & 0xffffu;
+            hi += x[u] >> 16;
+        }
+    }
+    s_part[grp][2 * col] = lo;
+    s_part[grp][2 * col + 1] = hi;
+    __syncthreads();
+    const int b = (int)threadIdx.x;   // 512 bins on the first 512 threads
+    const int i = items[2 * blockIdx.x + 1] * 512 + b;
+    if (b < 512 && i < B.hwin) {
+        const TurnScalars &sc = *B.sc;
+        uint32_t *h = hist_of(B, sc.turn) + window_lo(sc.centre_bin, B.hwin, B.nbins) + i;
+        *h += s_part[0][b] + s_part[1][b] + s_part[2][b] + s_part[3][b];
     }
 }
 
@@ -1988,7 +2036,7 @@ __global__ __launch_bounds__(kFinalThreads) void k_init(const BunchDev *__restri
         s.pending_m = 0;
         s.drift_skipped_count = 0;
         s.turn = 0;
-        s.centre_bin = 0;
+        s.centre_bin = B.nbins / 2;   // the windows start at the middle of the grid
         *B.sc = s;
     }
 }
@@ -3024,6 +3072,12 @@ hipError_t launch_interp_sum(const BunchDev *bds, const int32_t *order, const Ru
 hipError_t launch_finalize(const BunchDev *bds, const int32_t *items, int nitems, hipStream_t s) {
     if (nitems <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_finalize, dim3(nitems), dim3(kRedThreads), 0, s, bds, items);
+    return hipGetLastError();
+}
+
+hipError_t launch_hist_slabs(const BunchDev *bds, const int32_t *items, int nitems, hipStream_t s) {
+    if (nitems <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_hist_slabs, dim3(nitems), dim3(1024), 0, s, bds, items);
     return hipGetLastError();
 }
 

@@ -70,8 +70,8 @@ hipError_t launch_moments_final(const BunchDev *bds, const int32_t *bunch_list, 
 hipError_t launch_init(const BunchDev *bds, const int32_t *bunch_list, int nb, hipStream_t s);
 // `grid` workgroups over the tile order, workgroup g taking the runs
 // [rr[g], rr[g+1]); lds_bytes = the largest per-bunch histogram + potential
-// window; std_only: every bunch has (flags & kPhysMask) == kStdFlags and two
-// bins or more
+// window; std_only: every bunch has (flags & kPhysMask) == kStdFlags, two bins
+// or more and (F_GHIST) hwin > 0
 hipError_t launch_turn_pass(const BunchDev *bds, const int32_t *order, const RunDev *runs,
                             const int32_t *rr, int grid, size_t lds, int std_only, hipStream_t s);
 // `turns` turns of bunches without a wake and without the E0 update: items
@@ -90,6 +90,9 @@ hipError_t launch_conv(int kind, const BunchDev *bds, const int32_t *items, int 
 hipError_t launch_interp_sum(const BunchDev *bds, const int32_t *order, const RunDev *runs,
                              const int32_t *rr, int grid, size_t lds_bytes, bool deep,
                              hipStream_t s);
+// the slabs of the windowed histograms added up: items are (bunch, group of 512
+// bins of its window) pairs
+hipError_t launch_hist_slabs(const BunchDev *bds, const int32_t *items, int nitems, hipStream_t s);
 // per-bunch reduction of the pass's tile sums into the turn scalars (sum of
 // dE'-dE_init; sigma_z, current, binned count, centroid cell of a wake bunch),
 // and of the interpolation sums into the E0 update.  items holds nitems

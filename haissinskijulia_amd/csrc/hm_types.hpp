@@ -39,7 +39,7 @@ enum BunchFlags : uint32_t {
     F_QE = 16u,        // use_excitation
     F_INJ = 32u,       // injected normals instead of Philox
     F_CHARGE = 64u,    // fixed wake current (charge extension / stage entry)
-    F_GHIST = 128u,    // histogram straight to global memory (too many bins for LDS)
+    F_GHIST = 128u,    // too many bins for a histogram in LDS: hwin of them there, or none
     F_LAG = 256u,      // wake table by lag behind the source: bin k feels bins k+j (causal)
     F_CIC = 512u,      // the pass deposits the interpolation weights of the new z (cic)
 };
@@ -65,7 +65,29 @@ constexpr int64_t kCicRunPairs = (int64_t)1 << 20;
 // the all-physics-on configuration the turn pass is specialised for, and the
 // flags that select the pass's code path
 constexpr uint32_t kStdFlags = F_WAKE | F_ETA | F_E0 | F_SR | F_QE;
-constexpr uint32_t kPhysMask = F_WAKE | F_ETA | F_E0 | F_SR | F_QE | F_INJ | F_GHIST;
+constexpr uint32_t kPhysMask = F_WAKE | F_ETA | F_E0 | F_SR | F_QE | F_INJ;
+
+// Histograms of more bins than the LDS holds 32-bit counts for (F_GHIST).  An
+// addition to global memory per particle was bound by the crowded lines: 1e7
+// particles, 131072 bins: a pass of 0.40 ms; 45056 bins 0.54 ms.  So the pass
+// counts a window of kHistWin bins around the centroid in LDS, in 16 bits (a run
+// has at most kHistRunPairs pairs, so they cannot overflow), stores each run's
+// window to a slab of its own without atomics, and k_hist_slabs adds the slabs
+// up; only particles outside the window add to global memory: 0.108 ms and
+// 0.083 ms.  49152 bins are +-2.8 sigma of a bunch on 131072 bins over +-7.5
+// sigma (one particle in 200 outside) and leave 8000 entries for the window of
+// P, which the kick reads; 32768, 40960 and 57344 bins: 0.084, 0.085 and 0.098
+// ms against 0.089 at 65536 bins, 0.105, 0.105 and 0.111 at 131072, but 0.173,
+// 0.153 and 0.138 against 0.145 at 262144.  Slabs cost a launch of 8 us a turn
+// (25 MB written and read), so 32-bit counts of all bins stay as long as they
+// leave kHistMinWin entries of P: 1e7 particles, 34000 bins 95 + 35 us of pass
+// and bin phase, 36000 bins by the window 80 + 43, 40000 bins 118 + 35 before and
+// 81 + 43 after.  Tiles of more than kHistRunPairs pairs cannot use 16 bits;
+// kHistMaxPairs bounds the slabs of one bunch to a few hundred MB.
+constexpr int kHistWin = 49152;
+constexpr int kHistRunPairs = 32767;
+constexpr int64_t kHistMaxPairs = 1 << 26;
+constexpr int kHistMinWin = 3072;
 
 // Scalars of one turn of one bunch (evolution.jl:300-304 plus the pending
 // state of the fused pass).  Written by k_init / k_finalize, read by the
@@ -126,6 +148,9 @@ struct BunchDev {
     double *red;          // [nred][4]
     uint32_t *cnt;
     int32_t nred;
+    int32_t hwin;         // F_GHIST: bins counted in LDS (even; 0: all in global memory)
+    int32_t nslabs;       // F_GHIST with hwin: the bunch's runs, one slab of counts each
+    uint32_t *slabs;      // [nslabs][hwin / 2], two 16-bit counts per word
     int32_t cic_off;      // F_CIC: byte offset of the pass's LDS deposit
     int32_t cic_tiles;    // F_CIC: tiles of a run between two flushes of the deposit
     TurnScalars *sc;
@@ -134,17 +159,18 @@ struct BunchDev {
 };
 
 // A run of a workgroup: `count` consecutive entries, from `begin`, of a tile
-// order, all of one bunch.
+// order, all of one bunch; its slab of the bunch's windowed histogram.
 struct RunDev {
-    int32_t bunch, begin, count;
+    int32_t bunch, begin, count, slab;
 };
 
-// LDS of a turn-pass workgroup for one bunch: its histogram (nbins counts,
-// unless F_GHIST), then a window of `win` entries of the previous turn's
+// LDS of a turn-pass workgroup for one bunch: its histogram (nbins counts, with
+// F_GHIST hwin 16-bit ones), then a window of `win` entries of the previous turn's
 // potential, P[lo .. lo+win), for the wake-kick gathers, then with F_CIC the
 // deposit's counters at cic_off.
 __host__ __device__ inline int pass_hist_bytes(const BunchDev &B) {
-    return ((B.flags & F_WAKE) && !(B.flags & F_GHIST)) ? ((B.nbins * 4 + 15) & ~15) : 0;
+    if (!(B.flags & F_WAKE)) return 0;
+    return (((B.flags & F_GHIST) ? B.hwin * 2 : B.nbins * 4) + 15) & ~15;
 }
 
 __host__ __device__ inline int cic_bytes(int nbins) { return 16 * nbins; }
