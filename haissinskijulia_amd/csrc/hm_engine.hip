@@ -162,13 +162,6 @@ static double ref_wake(double z, double wf, double ws, double inv_ctau) {
     return z > 0 ? 0.0 : (wf * std::exp(z * inv_ctau)) * std::cos(ws * z);
 }
 
-// utils.jl:58-66
-static double ref_delta(double x, double sigma) {
-    const double s_inv = 1.0 / (std::sqrt(kTwoPi) * sigma);
-    const double ef = -0.5 / (sigma * sigma);
-    return s_inv * std::exp((x * x) * ef);
-}
-
 // evolution.jl:377-383
 double particle_factor(int64_t N) {
     static const double p10[11] = {1e0, 1e1, 1e2, 1e3, 1e4, 1e5, 1e6, 1e7, 1e8, 1e9, 1e10};
@@ -856,7 +849,7 @@ hm_status Batch::add_slots(const std::vector<RunBunch> &specs, std::vector<int32
         HIP_TRY(hipMemcpyAsync(q.d.out + 1, q.d.out + 11, sizeof(double), hipMemcpyDeviceToDevice,
                                s));
     }
-    // host tables, uploaded in one staging round after the loop
+    // the callers' tables, uploaded in one staging round after the loop
     std::vector<std::pair<double *, std::vector<double>>> keep;
     for (int32_t i : fresh) {
         RunBunch &q = rb_[(size_t)i];
@@ -875,37 +868,26 @@ hm_status Batch::add_slots(const std::vector<RunBunch> &specs, std::vector<int32
         // with a charge the line density is counts/n_h: the delta kernel
         // belongs to the reference's dimensionless current heuristic
         const double dsig = q.o.charge > 0 ? -1.0 : (q.o.delta_sigma == 0.0 ? 0.15 : q.o.delta_sigma);
-        // every centre only where a table is a function of the centres (the
-        // reference's wake W(c_j), the delta kernel); else the two ends
-        const bool lag_table = !q.wake_copy.empty() || !q.res_copy.empty();
-        const bool need_centres = !lag_table || dsig > 0;
-        std::vector<double> centers(need_centres ? (size_t)nb : 0);
         double step;
-        if (need_centres) {
-            bin_grid(zw, nb, nullptr, centers.data(), &step);
-            d.c_first = centers[0];
-            d.c_last = centers[(size_t)nb - 1];
-        } else {
-            bin_grid(zw, nb, nullptr, nullptr, &step);
-            d.c_first = rn_ratio(zw, 1 - nb, nb);
-            d.c_last = rn_ratio(zw, nb - 1, nb);
-        }
+        bin_grid(zw, nb, nullptr, nullptr, &step);
+        d.c_first = rn_ratio(zw, 1 - nb, nb);
+        d.c_last = rn_ratio(zw, nb - 1, nb);
         d.e_first = -zw;
         d.e_last = zw;
         d.inv_step = 1.0 / step;                                              // utils.jl:378
         d.inv_s = nb > 1 ? 1.0 / ((d.c_last - d.c_first) / (double)(nb - 1)) : 0.0;  // wakefield.jl:39-42
         d.u_last = (d.c_last - d.c_first) * d.inv_s;
-        std::vector<double> W, lam;
         const double wf = ((120.0 * kPi) * kSpeedLight) / (kPi * q.p.pipe_radius);   // evolution.jl:279
         const double ws = std::sqrt(jl_max_h(0.0, (2.0 * 30.0) / q.p.pipe_radius));  // evolution.jl:280
         const double inv_ctau = 1.0 / 4e-3;                                          // wakefield.jl:158
-        if (dsig > 0) {   // else lam = 1, filled on the device
-            lam.resize((size_t)nb);
-            for (int64_t k = 0; k < nb; ++k) lam[(size_t)k] = ref_delta(centers[(size_t)k], dsig);
-        }
-        // the wake table: the caller's, the reference's W(c_j) on the host, or
-        // the resonators' W(j step) computed on the device (k_resonator_table;
-        // a resonator's wake has no zero tail on any grid here: support nb)
+        const double d_inv = dsig > 0 ? 1.0 / (std::sqrt(kTwoPi) * dsig) : 0.0;       // utils.jl:61-62
+        const double d_ef = dsig > 0 ? -0.5 / (dsig * dsig) : 0.0;
+        // the wake table: the caller's, the reference's W(c_j)
+        // (k_reference_tables) or the resonators' W(j step)
+        // (k_resonator_table; a resonator's wake has no zero tail on any grid
+        // here: support nb)
+        const bool ref_table = q.wake_copy.empty() && q.res_copy.empty();
+        std::vector<double> W = std::move(q.wake_copy);
         int64_t nw = nb;
         ResonatorSet rset{};
         if (!q.res_copy.empty()) {
@@ -917,14 +899,11 @@ hm_status Batch::add_slots(const std::vector<RunBunch> &specs, std::vector<int32
                 rset.fr[r] = q.res_copy[(size_t)(3 * r + 1)];
                 rset.Q[r] = q.res_copy[(size_t)(3 * r + 2)];
             }
+        } else if (ref_table) {   // zero ahead of the source: the last c <= 0, unless it underflows there
+            nw = (nb + 1) / 2;
+            while (nw > 0 && ref_wake(rn_ratio(zw, 2 * nw - 1 - nb, nb), wf, ws, inv_ctau) == 0.0) --nw;
         } else {
-            W.assign((size_t)nb, 0.0);
-            for (int64_t k = 0; k < nb; ++k)
-                W[(size_t)k] = q.wake_copy.empty() ? ref_wake(centers[(size_t)k], wf, ws, inv_ctau)
-                                                   : q.wake_copy[(size_t)k];
-            nw = 0;
-            for (int64_t k = nb - 1; k >= 0; --k)
-                if (W[(size_t)k] != 0.0) { nw = k + 1; break; }
+            while (nw > 0 && W[(size_t)(nw - 1)] == 0.0) --nw;
         }
         q.wake_copy.clear();
         q.res_copy.clear();
@@ -981,13 +960,14 @@ hm_status Batch::add_slots(const std::vector<RunBunch> &specs, std::vector<int32
                 d.Y = w.Y.p;
             }
         }
-        if (lam.empty())
-            HIP_TRY(launch_fill(w.lam.p, (size_t)nb, 1.0, s));
-        else
-            keep.emplace_back(w.lam.p, std::move(lam));
+        // (centres beyond 1e300 or NaN: the tables are those of 1e300, finite as ever)
+        HIP_TRY(launch_reference_tables(ref_table ? w.Wtmp.p : nullptr, dsig > 0 ? w.lam.p : nullptr,
+                                        (int)nb, zw <= 1e300 ? zw : 1e300, wf, ws, inv_ctau, d_inv, d_ef,
+                                        s));
+        if (!(dsig > 0)) HIP_TRY(launch_fill(w.lam.p, (size_t)nb, 1.0, s));
         if (rset.n > 0)
             HIP_TRY(launch_resonator_table(w.Wtmp.p, (int)nb, step, rset, s));
-        else
+        else if (!ref_table)
             keep.emplace_back(w.Wtmp.p, std::move(W));
         HIP_TRY(launch_zero(w.P.p, (size_t)nb * 8, s));
         HIP_TRY(launch_zero(w.P2.p, (size_t)nb * 16, s));
@@ -1007,7 +987,7 @@ hm_status Batch::add_slots(const std::vector<RunBunch> &specs, std::vector<int32
         HM_TRY(twiddles(ctx_, d.F, &tw));
         d.tw = tw;
     }
-    {   // the host tables, the descriptors and the new bunches' list: one round
+    {   // the callers' tables, the descriptors and the new bunches' list: one round
         HM_TRY(d_tmp_list_.ensure(fresh.size()));
         size_t bytes = stage_size(rb_.size() * sizeof(BunchDev)) + stage_size(fresh.size() * 4);
         for (auto &kv : keep) bytes += stage_size(kv.second.size() * 8);

@@ -156,6 +156,10 @@ struct ResonatorSet {
 // W[j] = sum of the resonators' wakes at s = j * step, j < nb
 hipError_t launch_resonator_table(double *W, int nb, double step, const ResonatorSet &rs,
                                   hipStream_t s);
+// the reference's W(c) and delta kernel of the bin centres (either may be NULL;
+// nb < 2^28, 1e-200 < zw <= 1e300)
+hipError_t launch_reference_tables(double *W, double *lam, int nb, double zw, double wf, double ws,
+                                   double inv_ctau, double s_inv, double ef, hipStream_t s);
 // FFT of the wake blocks: What[j] = FFT_F(W[jB .. jB+B) zero-padded)
 hipError_t launch_fft_wake(const BunchDev *bd_dev, const double *W, int nJ, int F,
                            hipStream_t s);
