@@ -575,6 +575,13 @@ hm_status Batch::build_tables() {
     }
     const int per_cu = interp_lds_ + 1024 <= (size_t)ctx_->lds_max / 2 ? 2 : 1;
     pass_grid_ = std::min(ntiles_, ctx_->cus);
+    // Few tiles: two workgroups of half the waves each per tile.  A tile's sums
+    // are per wave, so nothing depends on it, and a CU's SIMDs serve two waves
+    // instead of four (1e6 particles, 512 bins, 123 tiles: 28.0 -> 25.8 us a
+    // turn; 20000 particles, 10 tiles: 17.2 -> 15.2; 1e5 particles, 49 tiles: 20.2 ->
+    // 19.5).  Four of a quarter each lose the gain to four times the flushes
+    // of the histogram and the deposit (25.8, 15.3 and 22.8 us).
+    pass_slices_ = 2 * pass_grid_ <= ctx_->cus ? 2 : 1;
     interp_grid_ = any_wake_e0_ ? std::min(ntiles_, per_cu * ctx_->cus) : 0;
     interp_deep_ = per_cu == 1;
     // ranges: [pass_grid_ + 1] then [interp_grid_ + 1] boundaries; order: the
@@ -603,7 +610,8 @@ hm_status Batch::build_tables() {
                     em = e + (int32_t)std::min<int64_t>(e1 - e, kHistRunPairs / d.pairs_per_tile);
                 int32_t ee = e + 1;
                 while (ee < em && tiles[(size_t)order[base + (size_t)ee]] == b) ++ee;
-                runs.push_back({b, (int32_t)base + e, ee - e, window ? d.nslabs++ : -1});
+                runs.push_back({b, (int32_t)base + e, ee - e, d.nslabs});
+                if (window) d.nslabs += pass_slices_;
                 e = ee;
             }
         }
@@ -1030,7 +1038,7 @@ hm_status Batch::one_turn() {
         ev_used_ += 3;
         HIP_TRY(hipEventRecord(e0, s));
     }
-    HIP_TRY(launch_turn_pass(d_bd_.p, d_order_.p, d_runs_.p, d_ranges_.p, pass_grid_, pass_lds_,
+    HIP_TRY(launch_turn_pass(d_bd_.p, d_order_.p, d_runs_.p, d_ranges_.p, pass_grid_, pass_slices_, pass_lds_,
                              std_only_ ? 1 : 0, s));
     if (timing_) HIP_TRY(hipEventRecord(e1, s));
     HIP_TRY(launch_hist_slabs(d_bd_.p, d_slab_.p, nslab_, s));

@@ -240,7 +240,7 @@ class Batch {
     // [interp_grid_ + 1] entries
     DevBuf<RunDev> d_runs_;
     DevBuf<int32_t> d_ranges_;
-    int pass_grid_ = 0, interp_grid_ = 0;
+    int pass_grid_ = 0, pass_slices_ = 1, interp_grid_ = 0;
     bool interp_deep_ = false;   // one interpolation workgroup per CU: deeper rings
     // no active bunch needs a sum over its particles between turns: the items
     // of k_free_turns, and the pairs they cover

@@ -698,7 +698,7 @@ __device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlan
 enum KickMode { kFullWindow = 0, kGatherFirst = 1, kPrefetchFirst = 2 };
 template <uint32_t FX, int HM, int KM, bool CIC>
 __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *__restrict__ run,
-                                              int cnt, int hb, int cb) {
+                                              int cnt, unsigned t0, int hb, int cb) {
     PassCtx c;
     load_ctx(B, c);
     const Flags<FX> fl{c.flags};
@@ -727,7 +727,7 @@ __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *
     const int hwin = B.hwin;
     const int hlo = HM == kHistWindow ? uni(window_lo(sc.centre_bin, hwin, c.nb)) : 0;
     g_u32 *n_bad = CIC ? (g_u32 *)(B.cic + 2 * (int64_t)c.nb) + c.nb : nullptr;
-    const unsigned tid = threadIdx.x;
+    const unsigned tid = t0 + threadIdx.x;
     const int wave = uni((int)(tid >> 6));
     constexpr unsigned step = kPassThreads;
 
@@ -888,7 +888,7 @@ __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *
     // the single particle of an odd bunch (last pair), out of the tile loop so
     // that its inlined turn does not add to the loop's register pressure
     if (odd_tile) {
-        if (threadIdx.x == 0) {
+        if (tid == 0) {
             const int64_t i = n - 1;
             double z0 = zp[i], e0 = ep[i], r0 = 0.0, r1 = 0.0;
             if (qe) {
@@ -972,14 +972,19 @@ __device__ inline void stage_bunch(const BunchDev &B) {
 // flushes the histogram.  The per-tile sums depend on the tile and the block
 // size only, not on which workgroup takes the tile.  The runs are found on the
 // host: found in the kernel, from the tile table, they cost two dependent
-// scalar loads per tile before the first byte was streamed.
+// scalar loads per tile before the first byte was streamed.  Launched with half
+// the threads, two consecutive workgroups share a range, each with the tiles'
+// lower or upper eight waves and LDS tables of its own.
 template <uint32_t FX>
 __device__ __forceinline__ void turn_pass_blocks(const BunchDev *__restrict__ bds,
                                                  const int32_t *__restrict__ order,
                                                  const RunDev *__restrict__ runs,
                                                  const int32_t *__restrict__ rr) {
-    const int r1 = rr[blockIdx.x + 1];
-    for (int r = rr[blockIdx.x]; r < r1; ++r) {
+    const unsigned slices = kPassThreads / blockDim.x;
+    const unsigned g = blockIdx.x / slices, slice = blockIdx.x % slices;
+    const unsigned t0 = slice * blockDim.x;
+    const int r1 = rr[g + 1];
+    for (int r = rr[g]; r < r1; ++r) {
         const RunDev rd = runs[r];
         const BunchDev &B = bds[rd.bunch];
         stage_bunch<FX>(B);
@@ -992,18 +997,18 @@ __device__ __forceinline__ void turn_pass_blocks(const BunchDev *__restrict__ bd
         const bool full = B.win >= B.nbins;
         const int cb = B.cic_off;
         if (B.flags & F_CIC) {   // the deposit comes with the whole table
-            turn_pass_run<FX, kHistLds, kFullWindow, true>(B, run, cnt, hb, cb);
+            turn_pass_run<FX, kHistLds, kFullWindow, true>(B, run, cnt, t0, hb, cb);
         } else if (!(B.flags & F_GHIST)) {   // a bunch without a wake among them
             if (full)
-                turn_pass_run<FX, kHistLds, kFullWindow, false>(B, run, cnt, hb, cb);
+                turn_pass_run<FX, kHistLds, kFullWindow, false>(B, run, cnt, t0, hb, cb);
             else
-                turn_pass_run<FX, kHistLds, kPartial, false>(B, run, cnt, hb, cb);
+                turn_pass_run<FX, kHistLds, kPartial, false>(B, run, cnt, t0, hb, cb);
         } else if (FX != 0 || B.hwin > 0) {
-            turn_pass_run<FX, kHistWindow, kPartial, false>(B, run, cnt, hb, cb);
+            turn_pass_run<FX, kHistWindow, kPartial, false>(B, run, cnt, t0, hb, cb);
         } else {
-            turn_pass_run<FX, kHistGlobal, kPrefetchFirst, false>(B, run, cnt, hb, cb);
+            turn_pass_run<FX, kHistGlobal, kPrefetchFirst, false>(B, run, cnt, t0, hb, cb);
         }
-        flush_hist(B, rd.slab);
+        flush_hist(B, rd.slab + (int)slice);
     }
 }
 
@@ -3041,14 +3046,14 @@ hipError_t launch_init(const BunchDev *bds, const int32_t *list, int nb, hipStre
 }
 
 hipError_t launch_turn_pass(const BunchDev *bds, const int32_t *order, const RunDev *runs,
-                            const int32_t *rr, int grid, size_t lds, int std_only, hipStream_t s) {
+                            const int32_t *rr, int grid, int slices, size_t lds, int std_only,
+                            hipStream_t s) {
     if (grid <= 0) return hipSuccess;
+    const dim3 blocks((unsigned)(grid * slices)), threads((unsigned)(kPassThreads / slices));
     if (std_only)
-        hipLaunchKernelGGL(k_turn_pass_std, dim3((unsigned)grid), dim3(kPassThreads), lds, s, bds,
-                           order, runs, rr);
+        hipLaunchKernelGGL(k_turn_pass_std, blocks, threads, lds, s, bds, order, runs, rr);
     else
-        hipLaunchKernelGGL(k_turn_pass, dim3((unsigned)grid), dim3(kPassThreads), lds, s, bds,
-                           order, runs, rr);
+        hipLaunchKernelGGL(k_turn_pass, blocks, threads, lds, s, bds, order, runs, rr);
     return hipGetLastError();
 }
 

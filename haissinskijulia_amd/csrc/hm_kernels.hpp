@@ -73,7 +73,8 @@ hipError_t launch_init(const BunchDev *bds, const int32_t *bunch_list, int nb, h
 // window; std_only: every bunch has (flags & kPhysMask) == kStdFlags, two bins
 // or more and (F_GHIST) hwin > 0
 hipError_t launch_turn_pass(const BunchDev *bds, const int32_t *order, const RunDev *runs,
-                            const int32_t *rr, int grid, size_t lds, int std_only, hipStream_t s);
+                            const int32_t *rr, int grid, int slices, size_t lds, int std_only,
+                            hipStream_t s);
 // `turns` turns of bunches without a wake and without the E0 update: items
 // cover the listed bunches' pairs
 constexpr int kFreeThreads = 256;
