@@ -182,10 +182,11 @@ __host__ __device__ inline int pass_lds_bytes(const BunchDev &B) {
     return (B.flags & F_CIC) ? B.cic_off + pass_cic_bytes(B) : pass_hist_bytes(B) + 8 * B.win;
 }
 
-// first entry of a window of w entries of P centred on `centre`
+// first entry of a window of w entries of P centred on `centre`; even, so that
+// the window is read by 16-byte loads
 __host__ __device__ inline int window_lo(int centre, int w, int nbins) {
     const int lo = centre - w / 2;
-    return lo < 0 ? 0 : (lo > nbins - w ? nbins - w : lo);
+    return (lo < 0 ? 0 : (lo > nbins - w ? nbins - w : lo)) & ~1;
 }
 
 }  // namespace hm
