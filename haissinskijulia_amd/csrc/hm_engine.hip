@@ -805,6 +805,7 @@ hm_status Batch::add_slots(const std::vector<RunBunch> &specs, std::vector<int32
         HM_TRY(w.sc.ensure(1));
         HM_TRY(w.out.ensure(16));
         HIP_TRY(launch_zero(w.out.p, 16 * sizeof(double), s));
+        d.spread = d.ntiles >= kSpreadTiles ? ~31 : 0;
         d.nred = red_slices(d.ntiles);
         HM_TRY(w.red.ensure((size_t)d.nred * 4));
         HM_TRY(w.cnt.ensure(1));
@@ -953,7 +954,7 @@ hm_status Batch::add_slots(const std::vector<RunBunch> &specs, std::vector<int32
             d.iwin = (int32_t)std::min<int64_t>(nb, ((int64_t)ctx_->lds_max - 1024) / 8);
         }
         Work &w = q.b->w;
-        HM_TRY(w.hist.ensure((size_t)nb * 2));
+        HM_TRY(w.hist.ensure((size_t)hist_half((int)nb) * 2));
         HM_TRY(w.P.ensure((size_t)nb));
         HM_TRY(w.P2.ensure((size_t)nb * 2));
         HM_TRY(w.lam.ensure((size_t)nb));
@@ -981,7 +982,7 @@ hm_status Batch::add_slots(const std::vector<RunBunch> &specs, std::vector<int32
         HIP_TRY(launch_zero(w.P2.p, (size_t)nb * 16, s));
         d.cic = nullptr;
         if (d.flags & F_CIC) {   // cleared again by each turn's finalize
-            const size_t words = 2 * (size_t)nb + ((size_t)nb + 2) / 2;   // hi, lo, n
+            const size_t words = cic_words((int)nb);
             HM_TRY(w.cic.ensure(words));
             HIP_TRY(launch_zero(w.cic.p, words * 8, s));
             d.cic = w.cic.p;

@@ -231,7 +231,7 @@ __device__ __forceinline__ double interp_pot(const double *__restrict__ P, doubl
 
 // this turn's half of the two-turn histogram buffer
 __device__ __forceinline__ uint32_t *hist_of(const BunchDev &B, int64_t turn) {
-    return B.hist + (turn & 1) * (int64_t)B.nbins;
+    return B.hist + (int)(turn & 1) * hist_half(B.nbins);
 }
 
 // histogram bin of calculate_local_histogram! (utils.jl:387-397); -1 = not counted
@@ -584,6 +584,11 @@ typedef __attribute__((address_space(1))) uint32_t g_u32;
 typedef __attribute__((address_space(1))) uint8_t g_u8;
 typedef __attribute__((address_space(1))) unsigned long long g_u64;
 
+// a deposit's counts n, and behind them the count of NaN positions
+__device__ __forceinline__ g_u32 *cic_n(const BunchDev &B) {
+    return (g_u32 *)(B.cic + 2 * cic_half(B.nbins));
+}
+
 __device__ __forceinline__ double2 ld2(const g_f64x2 *a) {
     const f64x2 v = *a;
     return make_double2(v.x, v.y);
@@ -654,8 +659,8 @@ __device__ __forceinline__ void clear_lds(uint8_t *s, int bytes) {
 // only) the NaN positions among them, one atomic each.
 enum HistMode { kHistGlobal = 0, kHistLds = 1, kHistWindow = 2 };
 template <int HM, bool CIC>
-__device__ __forceinline__ void bin_and_sum(const PassCtx &c, g_u32 *ghist, int hlo, int hwin,
-                                            g_u32 *n_bad, double z, double (&v)[4]) {
+__device__ __forceinline__ void bin_and_sum(const PassCtx &c, g_u32 *ghist, int spread, int hlo,
+                                            int hwin, g_u32 *n_bad, double z, double (&v)[4]) {
     v[0] += z;
     v[1] = __builtin_fma(z, z, v[1]);
     // hist_bin with its range test as the branch: in range, u = (z - e0) * inv
@@ -668,7 +673,8 @@ __device__ __forceinline__ void bin_and_sum(const PassCtx &c, g_u32 *ghist, int 
         else if (HM == kHistWindow && w < (unsigned)hwin)
             atomicAdd(reinterpret_cast<uint32_t *>(pass_lds()) + (w >> 1), 1u << (16 * (w & 1)));
         else
-            __hip_atomic_fetch_add(ghist + b, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_fetch_add(ghist + spread32(spread, b), 1u, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
     } else {
         v[3] += 1.0;
         if (CIC && z != z)
@@ -755,9 +761,9 @@ __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *
     g_f64 *zp = (g_f64 *)B.z;
     g_f64 *ep = (g_f64 *)B.dE;
     g_u32 *ghist = (g_u32 *)hist_of(B, sc.turn);
-    const int hwin = B.hwin;
+    const int spread = HM == kHistLds ? 0 : B.spread, hwin = B.hwin;
     const int hlo = HM == kHistWindow ? uni(window_lo(sc.centre_bin, hwin, c.nb)) : 0;
-    g_u32 *n_bad = CIC ? (g_u32 *)(B.cic + 2 * (int64_t)c.nb) + c.nb : nullptr;
+    g_u32 *n_bad = CIC ? cic_n(B) + hist_half(c.nb) : nullptr;
     const unsigned tid = t0 + threadIdx.x;
     const int wave = uni((int)(tid >> 6));
     constexpr unsigned step = kPassThreads;
@@ -896,8 +902,8 @@ __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *
             __builtin_amdgcn_s_waitcnt(0x0F70);
             if (tid < lim) {
                 if (wake) {
-                    bin_and_sum<HM, CIC>(c, ghist, hlo, hwin, n_bad, z0, v);
-                    bin_and_sum<HM, CIC>(c, ghist, hlo, hwin, n_bad, z1, v);
+                    bin_and_sum<HM, CIC>(c, ghist, spread, hlo, hwin, n_bad, z0, v);
+                    bin_and_sum<HM, CIC>(c, ghist, spread, hlo, hwin, n_bad, z1, v);
                 }
                 if (CIC) {
                     cic_deposit(c, cb, z0);
@@ -929,7 +935,7 @@ __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *
             e0 = apply_pending(c, z0, e0);
             double d0;
             advance(c, fl, z0, e0, r0, d0);
-            if (wake) bin_and_sum<HM, CIC>(c, ghist, hlo, hwin, n_bad, z0, v);
+            if (wake) bin_and_sum<HM, CIC>(c, ghist, spread, hlo, hwin, n_bad, z0, v);
             if (CIC) cic_deposit(c, cb, z0);
             v[2] += d0;
             zp[i] = z0;
@@ -955,23 +961,25 @@ __device__ inline void flush_hist(const BunchDev &B, int slab) {
         return;
     }
     g_u32 *g = (g_u32 *)hist_of(B, B.sc->turn);
+    const int sp = B.spread;
     for (int b = t; b < B.nbins; b += blockDim.x) {
         const uint32_t h = s_hist[b];
-        if (h) __hip_atomic_fetch_add(g + b, h, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (h)
+            __hip_atomic_fetch_add(g + spread32(sp, b), h, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     if (B.flags & F_CIC) {   // and the deposit into this turn's counters
         const int nb = B.nbins;
         const ulonglong2 *sC = reinterpret_cast<const ulonglong2 *>(pass_lds() + B.cic_off);
-        g_u64 *gH = (g_u64 *)B.cic;
-        g_u32 *gN = (g_u32 *)(B.cic + 2 * nb);
+        g_u64 *gH = (g_u64 *)B.cic, *gL = gH + cic_half(nb);
+        g_u32 *gN = cic_n(B);
         for (int b = t; b < nb; b += blockDim.x) {
             const ulonglong2 c = sC[b];
             if (!c.x) continue;
-            __hip_atomic_fetch_add(gN + b, (uint32_t)(c.x >> kCicCountBit), __ATOMIC_RELAXED,
+            __hip_atomic_fetch_add(gN + spread32(sp, b), (uint32_t)(c.x >> kCicCountBit), __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_fetch_add(gH + b, (c.x & ((1ull << kCicCountBit) - 1)) + (c.y >> 32),
+            __hip_atomic_fetch_add(gH + spread64(sp, b), (c.x & ((1ull << kCicCountBit) - 1)) + (c.y >> 32),
                                    __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_fetch_add(gH + nb + b, c.y & 0xffffffffull, __ATOMIC_RELAXED,
+            __hip_atomic_fetch_add(gL + spread64(sp, b), c.y & 0xffffffffull, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
         }
     }
@@ -1367,7 +1375,8 @@ __global__ __launch_bounds__(1024) void k_hist_slabs(const BunchDev *__restrict_
     const int i = items[2 * blockIdx.x + 1] * 512 + b;
     if (b < 512 && i < B.hwin) {
         const TurnScalars &sc = *B.sc;
-        uint32_t *h = hist_of(B, sc.turn) + window_lo(sc.centre_bin, B.hwin, B.nbins) + i;
+        uint32_t *h = hist_of(B, sc.turn) +
+                      spread32(B.spread, window_lo(sc.centre_bin, B.hwin, B.nbins) + i);
         *h += s_part[0][b] + s_part[1][b] + s_part[2][b] + s_part[3][b];
     }
 }
@@ -1407,7 +1416,7 @@ __global__ __launch_bounds__(1024) void k_bin_reduce_whole(const BunchDev *__res
 __device__ __forceinline__ double line_density(const BunchDev &B, const uint32_t *h, int i,
                                                double inv_nh) {
     if (B.flags & F_LAG) i = B.nbins - 1 - i;
-    return B.lam[i] * ((double)h[i] * inv_nh);
+    return B.lam[i] * ((double)h[spread32(B.spread, i)] * inv_nh);
 }
 
 // sX <- bit-reversed g_a + i g_{a-1}, zero-padded to F
@@ -1431,7 +1440,7 @@ __device__ inline void clear_next_hist(const BunchDev &B, int a) {
     const int nb = B.nbins, Bk = B.B;
     uint32_t *h = hist_of(B, B.sc->turn + 1);
     for (int m = threadIdx.x; m < Bk; m += blockDim.x)
-        if (a * Bk + m < nb) h[a * Bk + m] = 0u;
+        if (a * Bk + m < nb) h[spread32(B.spread, a * Bk + m)] = 0u;
 }
 
 // writes P[i] and its two places in the neighbour-pair table,
@@ -2083,7 +2092,7 @@ __global__ __launch_bounds__(kFinalThreads) void k_init(const BunchDev *__restri
                                                         const int32_t *__restrict__ list) {
     const BunchDev &B = bds[list[blockIdx.x]];
     if (B.flags & F_WAKE)
-        for (int b = threadIdx.x; b < 2 * B.nbins; b += blockDim.x) B.hist[b] = 0u;
+        for (int b = threadIdx.x; b < 2 * hist_half(B.nbins); b += blockDim.x) B.hist[b] = 0u;
     if (threadIdx.x == 0) {
         TurnScalars s = {};
         turn_scalars(B, B.E0_init, s);
@@ -2137,8 +2146,9 @@ __device__ inline void finish_turn(const BunchDev &B, double psum) {
 // whole-bunch finalize get the same bits from it.
 __device__ inline double cic_psum(const BunchDev &B, double *s_red) {
     const int nb = B.nbins;
-    g_u64 *H = (g_u64 *)B.cic;
-    g_u32 *N = (g_u32 *)(B.cic + 2 * nb);
+    const int sp = B.spread;
+    g_u64 *H = (g_u64 *)B.cic, *Lo = H + cic_half(nb);
+    g_u32 *N = cic_n(B);
     const g_f64 *P = (const g_f64 *)B.P;
     if ((int)threadIdx.x < kRedThreads) {
         // U cells per thread at a time, every load of the group issued before
@@ -2153,9 +2163,9 @@ __device__ inline double cic_psum(const BunchDev &B, double *s_red) {
             for (int u = 0; u < U; ++u) {
                 const int k = k0 + u * kRedThreads;
                 const bool in = k < nb - 1;
-                cnt[u] = in ? N[k] : 0u;
-                hi[u] = in ? H[k] : 0ull;
-                lo[u] = in ? H[nb + k] : 0ull;
+                cnt[u] = in ? N[spread32(sp, k)] : 0u;
+                hi[u] = in ? H[spread64(sp, k)] : 0ull;
+                lo[u] = in ? Lo[spread64(sp, k)] : 0ull;
                 p0[u] = in ? P[k] : 0.0;
                 p1[u] = in ? P[k + 1] : 0.0;
             }
@@ -2170,9 +2180,9 @@ __device__ inline double cic_psum(const BunchDev &B, double *s_red) {
             for (int u = 0; u < U; ++u) {
                 const int k = k0 + u * kRedThreads;
                 if (cnt[u]) {
-                    N[k] = 0u;
-                    H[k] = 0ull;
-                    H[nb + k] = 0ull;
+                    N[spread32(sp, k)] = 0u;
+                    H[spread64(sp, k)] = 0ull;
+                    Lo[spread64(sp, k)] = 0ull;
                 }
             }
         }
@@ -2183,8 +2193,8 @@ __device__ inline double cic_psum(const BunchDev &B, double *s_red) {
     double t = 0.0;
     if (threadIdx.x == 0) {
         for (int w = 0; w < kRedThreads / 64; ++w) t += s_red[w];
-        const uint32_t bad = N[nb];
-        N[nb] = 0u;
+        const uint32_t bad = N[hist_half(nb)];
+        N[hist_half(nb)] = 0u;
         if (bad) t = __builtin_nan("");
     }
     return t;
@@ -2236,8 +2246,9 @@ __device__ inline double cic_psum_lds(const BunchDev &B, const uint32_t *sN,
                                       const unsigned long long *sH, const double *sP,
                                       double *s_red) {
     const int nb = B.nbins;
-    g_u64 *H = (g_u64 *)B.cic;
-    g_u32 *N = (g_u32 *)(B.cic + 2 * nb);
+    const int sp = B.spread;
+    g_u64 *H = (g_u64 *)B.cic, *Lo = H + cic_half(nb);
+    g_u32 *N = cic_n(B);
     if ((int)threadIdx.x < kRedThreads) {
         double v = 0.0;
         for (int k = (int)threadIdx.x; k < nb - 1; k += kRedThreads) {
@@ -2245,9 +2256,9 @@ __device__ inline double cic_psum_lds(const BunchDev &B, const uint32_t *sN,
             if (cnt) {
                 const double sk = ((double)sH[k] * 0x1p32 + (double)sH[nb + k]) * (1.0 / kCicScale);
                 v += ((double)cnt - sk) * sP[k] + sk * sP[k + 1];
-                N[k] = 0u;
-                H[k] = 0ull;
-                H[nb + k] = 0ull;
+                N[spread32(sp, k)] = 0u;
+                H[spread64(sp, k)] = 0ull;
+                Lo[spread64(sp, k)] = 0ull;
             }
         }
         v = butterfly(v);
@@ -2258,7 +2269,7 @@ __device__ inline double cic_psum_lds(const BunchDev &B, const uint32_t *sN,
     if (threadIdx.x == 0) {
         for (int w = 0; w < kRedThreads / 64; ++w) t += s_red[w];
         const uint32_t bad = sN[nb];
-        N[nb] = 0u;
+        N[hist_half(nb)] = 0u;
         if (bad) t = __builtin_nan("");
     }
     return t;
@@ -2294,13 +2305,14 @@ __device__ inline void bin_phase_whole(const BunchDev &B) {
     double2 *sTw = reinterpret_cast<double2 *>(s_bw + L.tw);
     unsigned long long *sH = reinterpret_cast<unsigned long long *>(s_bw + L.cic);
     uint32_t *sN = reinterpret_cast<uint32_t *>(sH + 2 * nb);
+    const int sp = B.spread;
     TurnScalars sc;
     if (threadIdx.x == 0) sc = *B.sc;
     const int64_t turn = B.sc->turn;
     if (wake) {
         const uint32_t *h = hist_of(B, turn);
         for (int i = threadIdx.x; i < nb; i += blockDim.x) {
-            sHist[i] = h[i];
+            sHist[i] = h[spread32(sp, i)];
             sLam[i] = B.lam[i];
         }
         if (nJ > 1) {
@@ -2310,10 +2322,14 @@ __device__ inline void bin_phase_whole(const BunchDev &B) {
         const double2 *twg = reinterpret_cast<const double2 *>(B.tw);
         for (int u = threadIdx.x; u < F / 2; u += blockDim.x) sTw[u] = twg[u];
         if (cic) {
-            const unsigned long long *C = B.cic;
-            const uint32_t *N = reinterpret_cast<const uint32_t *>(B.cic + 2 * nb);
-            for (int i = threadIdx.x; i < 2 * nb; i += blockDim.x) sH[i] = C[i];
-            for (int i = threadIdx.x; i <= nb; i += blockDim.x) sN[i] = N[i];
+            const g_u64 *C = (const g_u64 *)B.cic;
+            const g_u32 *N = cic_n(B);
+            for (int i = threadIdx.x; i < nb; i += blockDim.x) {
+                sH[i] = C[spread64(sp, i)];
+                sH[nb + i] = C[cic_half(nb) + spread64(sp, i)];
+                sN[i] = N[spread32(sp, i)];
+            }
+            if (threadIdx.x == 0) sN[nb] = N[hist_half(nb)];
         }
     }
     if (fl & (F_WAKE | F_E0)) {
@@ -2330,7 +2346,7 @@ __device__ inline void bin_phase_whole(const BunchDev &B) {
         const double nh = s_nh, cur = s_cur;
         const double2 *tw = sTw;   // the twiddles from LDS: no global load per FFT stage
         uint32_t *hn = hist_of(B, turn + 1);   // the next turn's half, cleared
-        for (int i = threadIdx.x; i < nb; i += blockDim.x) hn[i] = 0u;
+        for (int i = threadIdx.x; i < nb; i += blockDim.x) hn[spread32(sp, i)] = 0u;
         if (nh == 0.0 || nJ == 0) {   // wakefield.jl:305-311
             for (int i = threadIdx.x; i < nb; i += blockDim.x) {
                 put_potential(B, i, 0.0);
@@ -2479,12 +2495,13 @@ __global__ __launch_bounds__(1024) void k_bin_64(const BunchDev *__restrict__ bd
     double *sG = reinterpret_cast<double *>(sY + nA * F);   // the line density, nA * 64
     double *sP = sG + nA * Bk;
     const int tid = (int)threadIdx.x, lane = tid & 63;
+    const int sp = B.spread;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int64_t turn = ((const TurnScalars *)B.sc)->turn;
     // the binned count, from both halves' counts (this turn's is known a load later)
     const g_u32 *hist = (const g_u32 *)B.hist;
     const int bin = min(tid, nb - 1);
-    const uint32_t h0 = hist[bin], h1 = hist[nb + bin];
+    const uint32_t h0 = hist[spread32(sp, bin)], h1 = hist[hist_half(nb) + spread32(sp, bin)];
     const double lam = ((const g_f64 *)B.lam)[bin];
     {
         int r = 0, c = tid;   // s_tw[tid] = w1, wa or wb (c) of stage pair r at butterfly index k
@@ -2510,7 +2527,7 @@ __global__ __launch_bounds__(1024) void k_bin_64(const BunchDev *__restrict__ bd
 #pragma unroll
     for (int w = 0; w < 16; ++w) total += s_cnt[w];
     const double nh = (double)total;
-    if (tid < nb) ((g_u32 *)B.hist)[((turn + 1) & 1) * nb + tid] = 0u;   // the next turn's half
+    if (tid < nb) ((g_u32 *)hist_of(B, turn + 1))[spread32(sp, tid)] = 0u;   // the next turn's half
     const double inv_nh = 1.0 / nh;
     if (tid < nA * Bk)   // line_density, in the convolution's order
         sG[(fl & F_LAG) && tid < nb ? nb - 1 - tid : tid] = tid < nb ? lam * ((double)hc * inv_nh) : 0.0;
@@ -2526,8 +2543,8 @@ __global__ __launch_bounds__(1024) void k_bin_64(const BunchDev *__restrict__ bd
     uint32_t cnt[4] = {0u, 0u, 0u, 0u};
     unsigned long long hi[4] = {0ull, 0ull, 0ull, 0ull}, lo[4] = {0ull, 0ull, 0ull, 0ull};
     uint32_t bad = 0;
-    g_u64 *H = (g_u64 *)B.cic;
-    g_u32 *N = (g_u32 *)(B.cic + 2 * nb);
+    g_u64 *H = (g_u64 *)B.cic, *Lo = H + cic_half(nb);
+    g_u32 *N = cic_n(B);
     const int ct = tid - 768;   // cic_psum's thread
     const int npart = B.ntiles * kTileWaves, tl = tid & 255;
     // group g of the pass sums (whole_sum's slices): waves 8-11 the even ones, 12-15 the odd ones
@@ -2557,9 +2574,9 @@ __global__ __launch_bounds__(1024) void k_bin_64(const BunchDev *__restrict__ bd
             for (int u = 0; u < 4; ++u) {
                 const int k = ct + u * kRedThreads;
                 if (k < nb - 1) {
-                    cnt[u] = N[k];
-                    hi[u] = H[k];
-                    lo[u] = H[nb + k];
+                    cnt[u] = N[spread32(sp, k)];
+                    hi[u] = H[spread64(sp, k)];
+                    lo[u] = Lo[spread64(sp, k)];
                 }
             }
         }
@@ -2657,7 +2674,7 @@ __global__ __launch_bounds__(1024) void k_bin_64(const BunchDev *__restrict__ bd
     TurnScalars sc;
     if (tid == kScalarThread) {   // whole_sum's and slices_done's order
         sc = *B.sc;
-        if (cic) bad = N[nb];
+        if (cic) bad = N[hist_half(nb)];
         double t[4] = {0.0, 0.0, 0.0, 0.0};
         for (int r = 0; r < nred; ++r)
 #pragma unroll
@@ -2729,9 +2746,9 @@ __global__ __launch_bounds__(1024) void k_bin_64(const BunchDev *__restrict__ bd
                 if (cnt[u]) {
                     const double sk = ((double)hi[u] * 0x1p32 + (double)lo[u]) * (1.0 / kCicScale);
                     a += ((double)cnt[u] - sk) * sP[k] + sk * sP[k + 1];
-                    N[k] = 0u;
-                    H[k] = 0ull;
-                    H[nb + k] = 0ull;
+                    N[spread32(sp, k)] = 0u;
+                    H[spread64(sp, k)] = 0ull;
+                    Lo[spread64(sp, k)] = 0ull;
                 }
             }
             a = butterfly(a);
@@ -2741,7 +2758,7 @@ __global__ __launch_bounds__(1024) void k_bin_64(const BunchDev *__restrict__ bd
         if (tid == kScalarThread) {
             for (int w = 0; w < kRedThreads / 64; ++w) t += s_red[w];
             if (bad) {
-                N[nb] = 0u;
+                N[hist_half(nb)] = 0u;
                 t = __builtin_nan("");
             }
             if (nred != 1) t = 0.0 + t;

@@ -26,7 +26,7 @@
 namespace {
 
 // 8 MiB: the work set of a bunch of up to 32768 bins (about 32 B per bin for
-// each of the three spectra tables, 40 B per bin for the histogram halves and
+// each of the three spectra tables, 48 B per bin for the histogram halves and
 // the potential tables, ~0.7 MB of per-tile sums for the at most 1025 tiles of
 // any bunch size)
 constexpr size_t kScratchBytes = size_t(8) << 20;

@@ -137,7 +137,7 @@ hm_status hm_wake_potential(hm_ctx *ctx, const int64_t *counts, int64_t nbins,
     HM_TRY(set_device(ctx));
     hipStream_t s = ctx->stream;
     int64_t nh = 0;
-    std::vector<uint32_t> h((size_t)nbins);
+    std::vector<uint32_t> h((size_t)hist_half((int)nbins));
     for (int64_t i = 0; i < nbins; ++i) {
         if (counts[i] < 0 || counts[i] > 0xffffffffLL) return fail(HM_ERR_ARG, "count out of range");
         h[(size_t)i] = (uint32_t)counts[i];
@@ -163,7 +163,7 @@ hm_status hm_wake_potential(hm_ctx *ctx, const int64_t *counts, int64_t nbins,
     d.nJ = (int32_t)((nw + Bk - 1) / Bk);
     const size_t what = (size_t)std::max(d.nJ, 1) * (size_t)d.F * 2;
     const size_t xs = (size_t)d.nA * (size_t)d.F * 2;
-    HM_TRY(ctx->shist.ensure((size_t)nbins * 2));
+    HM_TRY(ctx->shist.ensure(h.size() * 2));
     HM_TRY(ctx->sbuf[0].ensure((size_t)nbins));   // W
     HM_TRY(ctx->sbuf[1].ensure((size_t)nbins));   // lam
     HM_TRY(ctx->sbuf[2].ensure((size_t)nbins));   // P
@@ -193,7 +193,7 @@ hm_status hm_wake_potential(hm_ctx *ctx, const int64_t *counts, int64_t nbins,
     }
     DevBuf<int32_t> di;
     HM_TRY(di.ensure(items.size()));
-    HIP_TRY(hipMemcpyAsync(ctx->shist.p, h.data(), (size_t)nbins * 4, hipMemcpyHostToDevice, s));
+    HIP_TRY(hipMemcpyAsync(ctx->shist.p, h.data(), h.size() * 4, hipMemcpyHostToDevice, s));
     HIP_TRY(hipMemcpyAsync(ctx->sbuf[0].p, wake_tab, (size_t)nbins * 8, hipMemcpyHostToDevice, s));
     HIP_TRY(hipMemcpyAsync(ctx->sbuf[1].p, lam_tab, (size_t)nbins * 8, hipMemcpyHostToDevice, s));
     HIP_TRY(hipMemcpyAsync(ctx->ssc.p, &sc, sizeof(sc), hipMemcpyHostToDevice, s));
