@@ -5,7 +5,7 @@
 //   set-up   k_moments + k_moments_final   sigma_E0, sigma_z0 (evolution.jl:245-253)
 //            host: bin grid, wake and line-density tables (evolution.jl:261-281,
 //            wakefield.jl:194-221), FFT block plan; k_fft_wake; k_init
-//   turns    k_turn_pass, k_bin_reduce, k_conv, [k_interp_sum], k_finalize   per turn
+//   turns    k_turn_pass, k_reduce_fwd, k_conv, [k_interp_sum], k_finalize   per turn
 //   epilogue k_moments(mode 1) + k_moments_final            (evolution.jl:461-470)
 // A batch of bunches shares every launch: tiles, convolution items and
 // finalize blocks are looked up through per-launch tables.
@@ -507,10 +507,12 @@ hm_status Batch::build_tables() {
                 (fits_bin_64(wake, q.d.nbins, q.d.win, q.d.nA, q.d.nJ, q.d.F, q.d.nred) ? b64 : bw)
                     .push_back((int32_t)i);
                 bw_lds_ = std::max(bw_lds_, lds);
+                q.d.unb = nullptr;
                 continue;
             }
         }
         list.push_back((int32_t)i);
+        q.d.unb = (q.d.flags & F_WAKE) && q.d.nJ > 1 ? q.d.hist + 2 * hist_half(q.d.nbins) : nullptr;
         for (int r = 0; r < q.d.nred; ++r) {
             red.push_back((int32_t)i);
             red.push_back(r);
@@ -954,7 +956,7 @@ hm_status Batch::add_slots(const std::vector<RunBunch> &specs, std::vector<int32
             d.iwin = (int32_t)std::min<int64_t>(nb, ((int64_t)ctx_->lds_max - 1024) / 8);
         }
         Work &w = q.b->w;
-        HM_TRY(w.hist.ensure((size_t)hist_half((int)nb) * 2));
+        HM_TRY(w.hist.ensure((size_t)hist_half((int)nb) * 2 + 2 * kUnbSlots * 16));
         HM_TRY(w.P.ensure((size_t)nb));
         HM_TRY(w.P2.ensure((size_t)nb * 2));
         HM_TRY(w.lam.ensure((size_t)nb));
@@ -1040,18 +1042,16 @@ hm_status Batch::one_turn() {
         HIP_TRY(hipEventRecord(e0, s));
     }
     HIP_TRY(launch_turn_pass(d_bd_.p, d_order_.p, d_runs_.p, d_ranges_.p, pass_grid_, pass_slices_, pass_lds_,
-                             std_only_ ? 1 : 0, s));
+                             std_only_ ? 1 : 0, nconv_[CONV_FWD] > 0 ? 1 : 0, s));
     if (timing_) HIP_TRY(hipEventRecord(e1, s));
     HIP_TRY(launch_hist_slabs(d_bd_.p, d_slab_.p, nslab_, s));
     HIP_TRY(launch_bin_64(d_bd_.p, d_bw_.p, nb64_, bw_lds_, s));
     HIP_TRY(launch_bin_whole(d_bd_.p, d_bw_.p + nb64_, nbw_, bw_lds_, s));
     const bool whole = nlist_ >= kWholeMinBunches;
-    if (any_reduce_)
-        HIP_TRY(whole ? launch_bin_reduce_whole(d_bd_.p, d_list_.p, nlist_, s)
-                      : launch_bin_reduce(d_bd_.p, d_red_.p, nred_, s));
+    HIP_TRY(launch_reduce_fwd(d_bd_.p, d_red_.p, any_reduce_ ? nred_ : 0, d_conv_[CONV_FWD].p,
+                              nconv_[CONV_FWD], Fmax_, s));
     if (any_wake_) {
         HIP_TRY(launch_conv(CONV_FUSED, d_bd_.p, d_conv_[CONV_FUSED].p, nconv_[CONV_FUSED], Fmax_, s));
-        HIP_TRY(launch_conv(CONV_FWD, d_bd_.p, d_conv_[CONV_FWD].p, nconv_[CONV_FWD], Fmax_, s));
         HIP_TRY(launch_conv(CONV_SPEC, d_bd_.p, d_conv_[CONV_SPEC].p, nconv_[CONV_SPEC],
                             (int)spec_lds_, s));
         HIP_TRY(launch_conv(CONV_OUT, d_bd_.p, d_conv_[CONV_OUT].p, nconv_[CONV_OUT], Fmax_, s));

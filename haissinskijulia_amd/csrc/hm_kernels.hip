@@ -8,11 +8,12 @@
 //                 drift (evolution.jl:330-347); it bins the new z into an
 //                 LDS-privatised histogram (utils.jl:351-401) and writes
 //                 deterministic per-wave partial sums of each tile.
-//   k_bin_reduce  one workgroup per slice of 1024 of those sums; the last
+//   k_reduce_fwd  one workgroup per slice of 1024 of those sums; the last
 //                 slice of a bunch to finish adds the slice sums in order:
 //                 sigma_z, the wake current (evolution.jl:373-386), the
-//                 binned count and the sum of the energy changes.
-//   k_conv_*      the line-density convolution with the wake
+//                 binned count and the sum of the energy changes; beside
+//                 them the line density's blocks transformed.
+//   k_conv_*      the rest of the line-density convolution with the wake
 //                 (wakefield.jl:186-319) by blocked LDS FFTs.
 //   k_interp_sum  (update_E0 with the wake) sum of the interpolated potential
 //                 over the post-drift z, which the E0 update of
@@ -230,6 +231,10 @@ __device__ __forceinline__ double interp_pot(const double *__restrict__ P, doubl
 }
 
 // this turn's half of the two-turn histogram buffer
+// the slots of `turn`'s count of particles that are not binned
+__device__ __forceinline__ uint32_t *unb_of(const BunchDev &B, int64_t turn) {
+    return B.unb + (int)(turn & 1) * (kUnbSlots * 16);
+}
 __device__ __forceinline__ uint32_t *hist_of(const BunchDev &B, int64_t turn) {
     return B.hist + (int)(turn & 1) * hist_half(B.nbins);
 }
@@ -622,6 +627,12 @@ __device__ __forceinline__ uint8_t *pass_lds() {
     return s_lds;
 }
 
+// the workgroup's count of particles that are not binned
+__device__ __forceinline__ uint32_t &pass_unbinned() {
+    __shared__ uint32_t s_unb;
+    return s_unb;
+}
+
 // Copies the w entries from P to LDS, both 16-byte aligned, by 16-byte loads,
 // kStageLoads in flight per thread (eight spend registers and gain nothing).  In
 // 8-byte loads a window of 97 KB took 3 us of a pass and 128 KB 3 us of an
@@ -735,7 +746,7 @@ __device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlan
 enum KickMode { kFullWindow = 0, kGatherFirst = 1, kPrefetchFirst = 2 };
 template <uint32_t FX, int HM, int KM, bool CIC>
 __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *__restrict__ run,
-                                              int cnt, unsigned t0, int hb, int cb) {
+                                              int cnt, unsigned t0, int hb, int cb, int unb) {
     PassCtx c;
     load_ctx(B, c);
     const Flags<FX> fl{c.flags};
@@ -779,6 +790,7 @@ __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *
         const int lane = (int)tid & 63;
         g_f64 *o = (g_f64 *)B.part + 4 * ((int64_t)lt * kTileWaves + wave);
         if (lane >= 60) o[lane - 60] = tot;
+        if (unb && lane == 63 && tot != 0.0) atomicAdd(&pass_unbinned(), (uint32_t)tot);
     };
     // the single particle of an odd bunch sits in the bunch's last tile, the
     // last of this run if the run has it: that tile is flushed after the loop
@@ -946,11 +958,18 @@ __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *
     }
 }
 
-// Adds the LDS histogram of bunch B into this turn's global counts; a windowed
-// one goes to the run's slab as it is.
-__device__ inline void flush_hist(const BunchDev &B, int slab) {
-    if (!pass_hist_bytes(B)) return;
+// Adds the LDS histogram of bunch B, and the count of particles not binned, into
+// this turn's global counts; a windowed one goes to the run's slab as it is.
+__device__ inline void flush_hist(const BunchDev &B, int slab, int unb) {
+    if (!(B.flags & F_WAKE)) return;
     __syncthreads();
+    if (unb && threadIdx.x == 0) {
+        const uint32_t u = pass_unbinned();
+        if (u && B.unb)
+            __hip_atomic_fetch_add((g_u32 *)unb_of(B, B.sc->turn) + 16 * (blockIdx.x % kUnbSlots), u,
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (!pass_hist_bytes(B)) return;
     int t = (int)threadIdx.x;
     asm volatile("" : "+v"(t));   // as in stage_window
     const uint32_t *s_hist = reinterpret_cast<const uint32_t *>(pass_lds());
@@ -988,8 +1007,9 @@ __device__ inline void flush_hist(const BunchDev &B, int slab) {
 // Clears the LDS histogram of bunch B and loads its potential window (zero
 // before the first turn's bin phase; the all-flags pass reads it from the start).
 template <uint32_t FX>
-__device__ inline void stage_bunch(const BunchDev &B) {
+__device__ inline void stage_bunch(const BunchDev &B, int unb) {
     __syncthreads();   // the previous bunch's LDS is no longer read
+    if (unb && threadIdx.x == 0) pass_unbinned() = 0u;
     const int hb = pass_hist_bytes(B);
     clear_lds(pass_lds(), hb);
     if (B.flags & F_CIC) clear_lds(pass_lds() + B.cic_off, cic_bytes(B.nbins));
@@ -1014,7 +1034,7 @@ template <uint32_t FX>
 __device__ __forceinline__ void turn_pass_blocks(const BunchDev *__restrict__ bds,
                                                  const int32_t *__restrict__ order,
                                                  const RunDev *__restrict__ runs,
-                                                 const int32_t *__restrict__ rr) {
+                                                 const int32_t *__restrict__ rr, int unb) {
     const unsigned slices = kPassThreads / blockDim.x;
     const unsigned g = blockIdx.x / slices, slice = blockIdx.x % slices;
     const unsigned t0 = slice * blockDim.x;
@@ -1022,7 +1042,7 @@ __device__ __forceinline__ void turn_pass_blocks(const BunchDev *__restrict__ bd
     for (int r = rr[g]; r < r1; ++r) {
         const RunDev rd = runs[r];
         const BunchDev &B = bds[rd.bunch];
-        stage_bunch<FX>(B);
+        stage_bunch<FX>(B, unb);
         const int hb = pass_hist_bytes(B);
         const int32_t *run = order + rd.begin;
         const int cnt = rd.count;
@@ -1032,26 +1052,26 @@ __device__ __forceinline__ void turn_pass_blocks(const BunchDev *__restrict__ bd
         const bool full = B.win >= B.nbins;
         const int cb = B.cic_off;
         if (B.flags & F_CIC) {   // the deposit comes with the whole table
-            turn_pass_run<FX, kHistLds, kFullWindow, true>(B, run, cnt, t0, hb, cb);
+            turn_pass_run<FX, kHistLds, kFullWindow, true>(B, run, cnt, t0, hb, cb, unb);
         } else if (!(B.flags & F_GHIST)) {   // a bunch without a wake among them
             if (full)
-                turn_pass_run<FX, kHistLds, kFullWindow, false>(B, run, cnt, t0, hb, cb);
+                turn_pass_run<FX, kHistLds, kFullWindow, false>(B, run, cnt, t0, hb, cb, unb);
             else
-                turn_pass_run<FX, kHistLds, kPartial, false>(B, run, cnt, t0, hb, cb);
+                turn_pass_run<FX, kHistLds, kPartial, false>(B, run, cnt, t0, hb, cb, unb);
         } else if (FX != 0 || B.hwin > 0) {
-            turn_pass_run<FX, kHistWindow, kPartial, false>(B, run, cnt, t0, hb, cb);
+            turn_pass_run<FX, kHistWindow, kPartial, false>(B, run, cnt, t0, hb, cb, unb);
         } else {
-            turn_pass_run<FX, kHistGlobal, kPrefetchFirst, false>(B, run, cnt, t0, hb, cb);
+            turn_pass_run<FX, kHistGlobal, kPrefetchFirst, false>(B, run, cnt, t0, hb, cb, unb);
         }
-        flush_hist(B, rd.slab + (int)slice);
+        flush_hist(B, rd.slab + (int)slice, unb);
     }
 }
 
 __global__ __launch_bounds__(kPassThreads) void k_turn_pass(const BunchDev *__restrict__ bds,
                                                             const int32_t *__restrict__ order,
                                                             const RunDev *__restrict__ runs,
-                                                            const int32_t *__restrict__ rr) {
-    turn_pass_blocks<0>(bds, order, runs, rr);
+                                                            const int32_t *__restrict__ rr, int unb) {
+    turn_pass_blocks<0>(bds, order, runs, rr, unb);
 }
 
 // the same for tables whose bunches all have exactly kStdFlags, two bins or more
@@ -1059,8 +1079,8 @@ __global__ __launch_bounds__(kPassThreads) void k_turn_pass(const BunchDev *__re
 __global__ __launch_bounds__(kPassThreads) void k_turn_pass_std(const BunchDev *__restrict__ bds,
                                                                 const int32_t *__restrict__ order,
                                                                 const RunDev *__restrict__ runs,
-                                                                const int32_t *__restrict__ rr) {
-    turn_pass_blocks<kStdFlags>(bds, order, runs, rr);
+                                                                const int32_t *__restrict__ rr, int unb) {
+    turn_pass_blocks<kStdFlags>(bds, order, runs, rr, unb);
 }
 
 // ---------------------------------------------------------------------------
@@ -1346,7 +1366,7 @@ __device__ inline void whole_sum(const BunchDev &B, const double *a, double (&t)
 // The counts of the LDS windows, slab by slab, added to this turn's histogram:
 // a workgroup takes 256 words (512 bins) of one bunch's window, each of its
 // four groups of waves a quarter of the slabs with 16 loads in flight.  Before
-// k_bin_reduce, which moves the centroid that places the window.  Bound by the
+// k_reduce_fwd, which moves the centroid that places the window.  Bound by the
 // 25 MB of 256 slabs: 8 us with its launch, where flushing 49152 bins of every
 // workgroup by atomics would take about 28 (14 us per 6.3e6 of them).
 __global__ __launch_bounds__(1024) void k_hist_slabs(const BunchDev *__restrict__ bds,
@@ -1387,27 +1407,14 @@ __global__ __launch_bounds__(1024) void k_hist_slabs(const BunchDev *__restrict_
 // the binned count, and the interpolation cell of the centroid (where the LDS
 // windows of P are placed; the placement changes no result); the turn
 // monitor's centroid, sigma_z and binned count.  One workgroup per slice.
-__global__ __launch_bounds__(kRedThreads) void k_bin_reduce(const BunchDev *__restrict__ bds,
-                                                            const int32_t *__restrict__ items) {
+__device__ __forceinline__ void bin_reduce(const BunchDev &B, int r) {
     __shared__ double s_red[4 * 16];
-    const BunchDev &B = bds[items[2 * blockIdx.x]];
-    const int r = items[2 * blockIdx.x + 1];
     if (!(B.flags & (F_WAKE | F_E0))) return;
     double v[4] = {0.0, 0.0, 0.0, 0.0};   // sum z, sum z^2, sum (dE'-dE_init), not binned
     slice_sum<4>(B.part, B.ntiles * kTileWaves, r, v, s_red);
     double t[4];
     if (!slices_done<4>(B, r, v, t) || threadIdx.x != 0) return;
     bin_scalars(B, t);
-}
-
-// k_bin_reduce with one 1024-thread workgroup per bunch (whole_sum)
-__global__ __launch_bounds__(1024) void k_bin_reduce_whole(const BunchDev *__restrict__ bds,
-                                                           const int32_t *__restrict__ list) {
-    const BunchDev &B = bds[list[blockIdx.x]];
-    if (!(B.flags & (F_WAKE | F_E0))) return;
-    double t[4];
-    whole_sum<4>(B, B.part, t);
-    if (threadIdx.x == 0) bin_scalars(B, t);
 }
 
 // g_i = lam_i * (cnt_i / n_h) (wakefield.jl:210,238).  A wake table by lag
@@ -1496,18 +1503,44 @@ __global__ __launch_bounds__(kConvThreads) void k_conv_fused(const BunchDev *__r
 }
 
 // phase A of the blocked convolution: X_a = FFT(g_a + i g_{a-1})
-__global__ __launch_bounds__(kConvThreads) void k_conv_fwd(const BunchDev *__restrict__ bds,
-                                                           const int32_t *__restrict__ items) {
+__device__ __forceinline__ void conv_fwd(const BunchDev &B, int a, double nh) {
     extern __shared__ double2 sX[];
-    const BunchDev &B = bds[items[2 * blockIdx.x]];
-    const int a = items[2 * blockIdx.x + 1];
-    const double nh = B.sc->n_h;
     clear_next_hist(B, a);
     if (nh == 0.0) return;
     load_packed(sX, B, a, 1.0 / nh);
     fft_dit_forward(sX, B.F, B.logF, reinterpret_cast<const double2 *>(B.tw));
     double2 *X = reinterpret_cast<double2 *>(B.X) + (int64_t)a * B.F;
     for (int k = threadIdx.x; k < B.F; k += blockDim.x) X[k] = sX[k];
+}
+
+__global__ __launch_bounds__(kConvThreads) void k_conv_fwd(const BunchDev *__restrict__ bds,
+                                                           const int32_t *__restrict__ items) {
+    const BunchDev &B = bds[items[2 * blockIdx.x]];
+    conv_fwd(B, items[2 * blockIdx.x + 1], B.sc->n_h);
+}
+
+// The reductions of the pass's sums (the first nred workgroups, bin_reduce) and
+// phase A of the convolutions in one launch.  Phase A needs of the reductions
+// only the binned count, which it takes from the pass's counts of particles
+// not binned (the same whole number).  In launches of their own the two took
+// 5 to 7 us each, one after the other: 1e6 particles, 16384 bins: 56.5 -> 52.4 us a
+// turn; 1e7, 8192 bins: 120 -> 117; 28 bunches of 4096 bins, which had one
+// workgroup per bunch for the reductions: 212 -> 210.
+__global__ __launch_bounds__(kConvThreads) void k_reduce_fwd(const BunchDev *__restrict__ bds,
+                                                             const int32_t *__restrict__ red, int nred,
+                                                             const int32_t *__restrict__ items) {
+    if ((int)blockIdx.x < nred) {
+        bin_reduce(bds[red[2 * blockIdx.x]], red[2 * blockIdx.x + 1]);
+        return;
+    }
+    const int32_t *it = items + 2 * ((int)blockIdx.x - nred);
+    const BunchDev &B = bds[it[0]];
+    const int64_t turn = B.sc->turn;
+    const int lane = (int)threadIdx.x & 63;
+    int c = (int)((g_u32 *)unb_of(B, turn))[16 * lane];   // every wave: kUnbSlots lanes
+    for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off, 64);
+    if (it[1] == 0 && (int)threadIdx.x < kUnbSlots) ((g_u32 *)unb_of(B, turn + 1))[16 * lane] = 0u;
+    conv_fwd(B, it[1], (double)(B.n - (int64_t)(uint32_t)c));
 }
 
 // phase B1: Y_o[k] = sum_{j <= min(o, nJ-1)} X_{o-j}[k] FFT(W_j)[k] for every
@@ -2092,7 +2125,8 @@ __global__ __launch_bounds__(kFinalThreads) void k_init(const BunchDev *__restri
                                                         const int32_t *__restrict__ list) {
     const BunchDev &B = bds[list[blockIdx.x]];
     if (B.flags & F_WAKE)
-        for (int b = threadIdx.x; b < 2 * hist_half(B.nbins); b += blockDim.x) B.hist[b] = 0u;
+        for (int b = threadIdx.x; b < 2 * hist_half(B.nbins) + 2 * kUnbSlots * 16; b += blockDim.x)
+            B.hist[b] = 0u;   // and the counts of particles not binned behind it
     if (threadIdx.x == 0) {
         TurnScalars s = {};
         turn_scalars(B, B.E0_init, s);
@@ -2276,7 +2310,7 @@ __device__ inline double cic_psum_lds(const BunchDev &B, const uint32_t *sN,
 }
 
 // The bin phase of a small bunch in one 1024-thread workgroup, in place of
-// k_bin_reduce, the convolution kernels and k_finalize.  Everything it reads
+// k_reduce_fwd, the convolution kernels and k_finalize.  Everything it reads
 // is staged first, side by side (the turn scalars in thread 0's registers,
 // this turn's counts, the line-density kernel, the wake spectra, the FFT
 // twiddles, the deposit), so the phase waits on memory about twice instead
@@ -3091,13 +3125,13 @@ hipError_t launch_init(const BunchDev *bds, const int32_t *list, int nb, hipStre
 
 hipError_t launch_turn_pass(const BunchDev *bds, const int32_t *order, const RunDev *runs,
                             const int32_t *rr, int grid, int slices, size_t lds, int std_only,
-                            hipStream_t s) {
+                            int unb, hipStream_t s) {
     if (grid <= 0) return hipSuccess;
     const dim3 blocks((unsigned)(grid * slices)), threads((unsigned)(kPassThreads / slices));
     if (std_only)
-        hipLaunchKernelGGL(k_turn_pass_std, blocks, threads, lds, s, bds, order, runs, rr);
+        hipLaunchKernelGGL(k_turn_pass_std, blocks, threads, lds, s, bds, order, runs, rr, unb);
     else
-        hipLaunchKernelGGL(k_turn_pass, blocks, threads, lds, s, bds, order, runs, rr);
+        hipLaunchKernelGGL(k_turn_pass, blocks, threads, lds, s, bds, order, runs, rr, unb);
     return hipGetLastError();
 }
 
@@ -3154,15 +3188,12 @@ hipError_t launch_hist_slabs(const BunchDev *bds, const int32_t *items, int nite
     return hipGetLastError();
 }
 
-hipError_t launch_bin_reduce(const BunchDev *bds, const int32_t *items, int nitems, hipStream_t s) {
-    if (nitems <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_bin_reduce, dim3(nitems), dim3(kRedThreads), 0, s, bds, items);
-    return hipGetLastError();
-}
-
-hipError_t launch_bin_reduce_whole(const BunchDev *bds, const int32_t *list, int nb, hipStream_t s) {
-    if (nb <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_bin_reduce_whole, dim3(nb), dim3(1024), 0, s, bds, list);
+hipError_t launch_reduce_fwd(const BunchDev *bds, const int32_t *red, int nred, const int32_t *items,
+                             int nitems, int Fmax, hipStream_t s) {
+    if (nred + nitems <= 0) return hipSuccess;
+    static_assert(kRedThreads == kConvThreads, "one launch for both");
+    hipLaunchKernelGGL(k_reduce_fwd, dim3(nred + nitems), dim3(kConvThreads),
+                       nitems > 0 ? (size_t)Fmax * 16 : 0, s, bds, red, nred, items);
     return hipGetLastError();
 }
 

@@ -71,10 +71,11 @@ hipError_t launch_init(const BunchDev *bds, const int32_t *bunch_list, int nb, h
 // `grid` workgroups over the tile order, workgroup g taking the runs
 // [rr[g], rr[g+1]); lds_bytes = the largest per-bunch histogram + potential
 // window; std_only: every bunch has (flags & kPhysMask) == kStdFlags, two bins
-// or more and (F_GHIST) hwin > 0
+// or more and (F_GHIST) hwin > 0; unb: some bunch's particles not binned are
+// counted (BunchDev::unb)
 hipError_t launch_turn_pass(const BunchDev *bds, const int32_t *order, const RunDev *runs,
                             const int32_t *rr, int grid, int slices, size_t lds, int std_only,
-                            hipStream_t s);
+                            int unb, hipStream_t s);
 // `turns` turns of bunches without a wake and without the E0 update: items
 // cover the listed bunches' pairs
 constexpr int kFreeThreads = 256;
@@ -98,12 +99,13 @@ hipError_t launch_hist_slabs(const BunchDev *bds, const int32_t *items, int nite
 // dE'-dE_init; sigma_z, current, binned count, centroid cell of a wake bunch),
 // and of the interpolation sums into the E0 update.  items holds nitems
 // (bunch, slice) pairs, red_slices(ntiles) slices per bunch.
-hipError_t launch_bin_reduce(const BunchDev *bds, const int32_t *items, int nitems, hipStream_t s);
+// launch_reduce_fwd: the pass's sums, and phase A of the convolutions of the
+// nitems (bunch, block) items
+hipError_t launch_reduce_fwd(const BunchDev *bds, const int32_t *red, int nred, const int32_t *items,
+                             int nitems, int Fmax, hipStream_t s);
 hipError_t launch_finalize(const BunchDev *bds, const int32_t *items, int nitems, hipStream_t s);
-// the same two reductions with one 1024-thread workgroup per listed bunch and
-// no cross-workgroup count: the same bits (for batches of many bunches)
-hipError_t launch_bin_reduce_whole(const BunchDev *bds, const int32_t *bunch_list, int nb,
-                                   hipStream_t s);
+// the same with one 1024-thread workgroup per listed bunch and no
+// cross-workgroup count: the same bits (for batches of many bunches)
 hipError_t launch_finalize_whole(const BunchDev *bds, const int32_t *bunch_list, int nb,
                                  hipStream_t s);
 // The whole bin phase (the reduction, the convolution and the finalize) of

@@ -89,6 +89,11 @@ constexpr int kHistRunPairs = 32767;
 constexpr int64_t kHistMaxPairs = 1 << 26;
 constexpr int kHistMinWin = 3072;
 
+// Slots of the count of a turn's particles that are not binned: one 64-byte
+// line each, so that the pass's workgroups (one addition per run at most) do
+// not queue at one address.
+constexpr int kUnbSlots = 64;
+
 // Scalars of one turn of one bunch (evolution.jl:300-304 plus the pending
 // state of the fused pass).  Written by k_init / k_finalize, read by the
 // per-particle kernels.
@@ -157,6 +162,8 @@ struct BunchDev {
     double *mon;          // device [n_turns][4] turn monitor or null
     int32_t spread;            // where counter i of hist and cic lies: spread32, spread64
     unsigned long long *cic;   // F_CIC: this turn's deposit (cic_* below; zero between turns)
+    uint32_t *unb;             // [2][kUnbSlots][16]: this turn's particles not binned, behind hist;
+                               // null where no k_reduce_fwd reads them
 };
 
 // The counters that every workgroup of the pass adds to (histogram, deposit)

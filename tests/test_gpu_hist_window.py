@@ -1,6 +1,6 @@
 """Histograms of more bins than the LDS holds: the window of 16-bit counts.
 
-Tiles of 64 chunks (32768 pairs) exceed what a 16-bit count can hold, so they
+Tiles of 32 chunks (32768 pairs) exceed what a 16-bit count can hold, so they
 take the path that adds every particle to global memory; smaller tiles take the
 window.  The counts are whole numbers, and the bunches start on a lattice with
 mean zero, so that the sums behind their sigmas are exact in any order: without
@@ -28,7 +28,7 @@ def _run(bunch, nb, tile_pairs, half, flags, turns=3):
 
 def _same(make, nb, tile_pairs, half, flags):
     out = []
-    for tp in (tile_pairs, 64):
+    for tp in (tile_pairs, 32):
         b = make()
         out.append(_run(b, nb, tp, half, flags))
         b.close()
@@ -50,23 +50,23 @@ def _gaussian(n):
 
 
 @pytest.mark.parametrize("nb", [33500, 34001, 40001, 49151, 49152, 49153, 49154, 65536, 131072])
-@pytest.mark.parametrize("n,tile_pairs,update_E0", [(50001, 63, True), (50001, 63, False), (200_003, 1, False),
+@pytest.mark.parametrize("n,tile_pairs,update_E0", [(50001, 31, True), (50001, 31, False), (200_003, 1, False),
                                                     (1, 1, False)])
 def test_window_counts(nb, n, tile_pairs, update_E0):
     _same(_gaussian(n), nb, tile_pairs, 2.5, (True, True, update_E0, True, True))
 
 
 def test_several_runs_per_workgroup():
-    _, _, counts, _ = _same(_gaussian(17_000_001), 131072, 63, 7.5, (True, True, False, True, True))
+    _, _, counts, _ = _same(_gaussian(17_000_001), 131072, 31, 7.5, (True, True, False, True, True))
     assert counts[0] > 16_900_000
 
 
 def test_one_bin_holds_a_run():
-    z0 = np.zeros(64512)
+    z0 = np.zeros(63488)
     z0[:4] = [-0.3, 0.3, -0.01, 0.01]
 
     def make():
         b = H.DeviceBunch(z0.size)
         b.upload(z0, np.zeros(z0.size))
         return b
-    _same(make, 65536, 63, 7.5, (True, True, False, False, False))
+    _same(make, 65536, 31, 7.5, (True, True, False, False, False))
