@@ -609,6 +609,11 @@ __device__ __forceinline__ double2 ldnt(const g_f64x2 *a) {
     const f64x2 v = __builtin_nontemporal_load(a);
     return make_double2(v.x, v.y);
 }
+// one or the other
+template <bool NT>
+__device__ __forceinline__ double2 ldp(const g_f64x2 *a) {
+    return NT ? ldnt(a) : ld2(a);
+}
 // streaming (nontemporal) 16-byte store
 __device__ __forceinline__ void stnt(g_f64x2 *a, double x, double y) {
     f64x2 v;
@@ -616,10 +621,27 @@ __device__ __forceinline__ void stnt(g_f64x2 *a, double x, double y) {
     v.y = y;
     __builtin_nontemporal_store(v, a);
 }
+template <bool NT>
+__device__ __forceinline__ void stp(g_f64x2 *a, double x, double y) {
+    if (NT) stnt(a, x, y);
+    else st2(a, x, y);
+}
 // P[k]*(1-w) + P[k+1]*w from the neighbour-pair table entry (P[k], P[k+1])
 __device__ __forceinline__ double gather_interp(const g_f64x2 *q, double w) {
     const f64x2 v = *q;
     return v.x * (1.0 - w) + v.y * w;
+}
+
+// The particles of a bunch with a windowed histogram are read and written
+// through the caches, by the pass and by the interpolation sums, where they fit
+// the 256 MB of the last one: many of its particles gather from the pair table,
+// and those gathers wait behind the streams (131072 bins, pass of 1e7 particles:
+// 104 -> 75 us, 4e6: 51 -> 39, 1.3e7: 139 -> 113, 2e7: 205 -> 212; one of the
+// two streaming past the caches undoes it).  With 32-bit LDS counts the same
+// costs 2 us up to 4e6 particles.
+constexpr int64_t kCachedBytes = 224ll << 20;
+__device__ __forceinline__ bool cached(const BunchDev &B) {
+    return (B.flags & F_GHIST) && B.hwin > 0 && 16 * B.n <= kCachedBytes;
 }
 
 __device__ __forceinline__ uint8_t *pass_lds() {
@@ -741,10 +763,12 @@ __device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlan
 // particles outside it gather from global memory; see the loop body).
 // CIC: the bunch's post-drift z are also deposited (cic_deposit) into the LDS
 // counters at byte cb.
+// NT: the particles are streamed past the caches, which are left to the bin
+// phase's tables.
 // With FX = kStdFlags the kick is applied from the first turn on: P is zero
 // before it, and subtracting 0 changes nothing.
 enum KickMode { kFullWindow = 0, kGatherFirst = 1, kPrefetchFirst = 2 };
-template <uint32_t FX, int HM, int KM, bool CIC>
+template <uint32_t FX, int HM, int KM, bool CIC, bool NT = true>
 __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *__restrict__ run,
                                               int cnt, unsigned t0, int hb, int cb, int unb) {
     PassCtx c;
@@ -806,8 +830,8 @@ __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *
         const unsigned b0 = (unsigned)lt * ppt, lim = min(full - b0, step);   // b0 <= full
         if (lim > 0) {
             const unsigned off = offset(lim);
-            zn = ldnt(at(zp, b0, off));
-            en = ldnt(at(ep, b0, off));
+            zn = ldp<NT>(at(zp, b0, off));
+            en = ldp<NT>(at(ep, b0, off));
         }
     }
     // the first chunk completes here (s_waitcnt vmcnt(0)), so that in the loop
@@ -840,8 +864,8 @@ __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *
                 unsigned bn = base + step < p1 ? base + step : (unsigned)ltn * ppt;
                 if (bn >= full) bn = base;
                 const unsigned off = offset(min(full - bn, step));
-                zn = ldnt(at(zp, bn, off));
-                en = ldnt(at(ep, bn, off));
+                zn = ldp<NT>(at(zp, bn, off));
+                en = ldp<NT>(at(ep, bn, off));
             };
             if (!gather_first) prefetch();
             // set and read only when kick2 (no per-pair clearing)
@@ -923,10 +947,8 @@ __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *
                 }
                 v[2] += d0;
                 v[2] += d1;
-                // streaming stores: the bunch is far larger than the caches,
-                // which are left to the bin phase's tables
-                stnt(at(zp, base, tid * 16u), z0, z1);
-                stnt(at(ep, base, tid * 16u), e0, e1);
+                stp<NT>(at(zp, base, tid * 16u), z0, z1);
+                stp<NT>(at(ep, base, tid * 16u), e0, e1);
             }
         }
         if (odd_tile && t == cnt - 1) break;   // v kept for the single particle
@@ -1059,7 +1081,10 @@ __device__ __forceinline__ void turn_pass_blocks(const BunchDev *__restrict__ bd
             else
                 turn_pass_run<FX, kHistLds, kPartial, false>(B, run, cnt, t0, hb, cb, unb);
         } else if (FX != 0 || B.hwin > 0) {
-            turn_pass_run<FX, kHistWindow, kPartial, false>(B, run, cnt, t0, hb, cb, unb);
+            if (cached(B))
+                turn_pass_run<FX, kHistWindow, kPartial, false, false>(B, run, cnt, t0, hb, cb, unb);
+            else
+                turn_pass_run<FX, kHistWindow, kPartial, false>(B, run, cnt, t0, hb, cb, unb);
         } else {
             turn_pass_run<FX, kHistGlobal, kPrefetchFirst, false>(B, run, cnt, t0, hb, cb, unb);
         }
@@ -1733,7 +1758,7 @@ __global__ __launch_bounds__(kConvThreads) void k_fft_wake(const BunchDev *__res
 // streaming loads (the next tile's first group at a tile's end) issued before
 // this group's sums; the group loop has the same trip count in every lane.
 // A tile's sums therefore depend on the tile and the block size only (not on G).
-template <int G, bool FULLW>
+template <int G, bool FULLW, bool NT>
 __device__ __forceinline__ void interp_sum_run_tiles(const BunchDev &B, const int32_t *__restrict__ run,
                                                      int nrun) {
     extern __shared__ __align__(16) double sP[];
@@ -1770,7 +1795,7 @@ __device__ __forceinline__ void interp_sum_run_tiles(const BunchDev &B, const in
 #pragma unroll
         for (int u = 0; u < G; ++u) {
             const int r = tid + u * ibs;
-            zn[u] = ldnt((u < K && r < lim0) ? zpair + (int64_t)lt * ppt + r : zpair);
+            zn[u] = ldp<NT>((u < K && r < lim0) ? zpair + (int64_t)lt * ppt + r : zpair);
         }
     }
     for (int j = 0; j < nrun; ++j) {
@@ -1800,7 +1825,7 @@ __device__ __forceinline__ void interp_sum_run_tiles(const BunchDev &B, const in
                 for (int u = 0; u < G; ++u) {
                     const double2 zz = zn[u];
                     const int r = nr + u * ibs;
-                    zn[u] = ldnt((u < nk && r < nlim) ? nbase + r : zpair);
+                    zn[u] = ldp<NT>((u < nk && r < nlim) ? nbase + r : zpair);
                     if (k + u >= K || tid + (k + u) * ibs >= lim) continue;
                     int k0, k1;
                     double w0, w1;
@@ -1838,7 +1863,7 @@ __device__ __forceinline__ void interp_sum_run_tiles(const BunchDev &B, const in
 // streaming loads in flight, so a tile of one pair per thread costs no
 // pipeline start.  A tile's sum is written when its last pair is added; it
 // depends on the tile and the block size only.
-template <bool FULLW>
+template <bool FULLW, bool NT>
 __device__ __forceinline__ void interp_sum_run_flat(const BunchDev &B, const int32_t *__restrict__ run,
                                                     int nrun) {
     extern __shared__ __align__(16) double sP[];
@@ -1893,7 +1918,7 @@ __device__ __forceinline__ void interp_sum_run_flat(const BunchDev &B, const int
         const int r = tid + lk * ibs;
         const int llt = lj < nrun ? tile_of(lj) : 0;
         const bool ok = lj < nrun && r < lim_of(llt);
-        const double2 x = ldnt(ok ? zpair + (int64_t)llt * ppt + r : zpair);
+        const double2 x = ldp<NT>(ok ? zpair + (int64_t)llt * ppt + r : zpair);
         if (++lk == K) {
             lk = 0;
             ++lj;
@@ -1946,22 +1971,24 @@ __device__ __forceinline__ void interp_sum_run_flat(const BunchDev &B, const int
 // large tiles, the run-wide ring no pipeline start per tile for small ones.
 // FULLW: the window holds the whole table (no gathers), so the compiler's
 // waits for the ring's slots count only the ring's own loads.
-template <int G, bool FULLW>
+template <int G, bool FULLW, bool NT>
 __device__ __forceinline__ void interp_sum_run_w(const BunchDev &B, const int32_t *run, int nrun) {
     if (G > 4 && B.pairs_per_tile >= G * (int64_t)kInterpThreads)
-        interp_sum_run_tiles<G, FULLW>(B, run, nrun);
+        interp_sum_run_tiles<G, FULLW, NT>(B, run, nrun);
     else if (B.pairs_per_tile >= 4 * (int64_t)kInterpThreads)
-        interp_sum_run_tiles<4, FULLW>(B, run, nrun);
+        interp_sum_run_tiles<4, FULLW, NT>(B, run, nrun);
     else
-        interp_sum_run_flat<FULLW>(B, run, nrun);
+        interp_sum_run_flat<FULLW, NT>(B, run, nrun);
 }
 
 template <int G>
 __device__ __forceinline__ void interp_sum_run(const BunchDev &B, const int32_t *run, int nrun) {
     if (B.iwin >= B.nbins)
-        interp_sum_run_w<G, true>(B, run, nrun);
+        interp_sum_run_w<G, true, true>(B, run, nrun);
+    else if (!cached(B))
+        interp_sum_run_w<G, false, true>(B, run, nrun);
     else
-        interp_sum_run_w<G, false>(B, run, nrun);
+        interp_sum_run_w<G, false, false>(B, run, nrun);
 }
 
 // The interpolation sums of the wake + update_E0 bunches over a tile table:
