@@ -3108,7 +3108,8 @@ static inline unsigned blocks_for(int64_t n, int t) { return (unsigned)((n + t -
 hipError_t configure_kernels(int lds) {
     const void *fns[] = {(const void *)k_turn_pass, (const void *)k_turn_pass_std,
                          (const void *)k_conv_fused,
-                         (const void *)k_conv_fwd, (const void *)k_conv_inv,
+                         (const void *)k_conv_fwd, (const void *)k_reduce_fwd,
+                         (const void *)k_conv_inv,
                          (const void *)k_conv_spec, (const void *)k_conv_out,
                          (const void *)k_fft_wake, (const void *)k_stage_hist,
                          (const void *)k_interp_sum, (const void *)k_interp_sum_deep,
