@@ -461,6 +461,8 @@ hm_status Batch::build_tables() {
     if (free_only_) return build_free_tables();
     std::vector<int32_t> tiles, conv[kConvKinds], red, list, bw, b64, slab;
     pass_lds_ = 0;
+    final_whole_ = true;
+    final_lds_ = 0;
     bw_lds_ = 0;
     spec_lds_ = 0;
     Fmax_ = 2;
@@ -512,6 +514,8 @@ hm_status Batch::build_tables() {
             }
         }
         list.push_back((int32_t)i);
+        if (!(q.d.flags & F_CIC) && q.d.nred > kWholeMaxSlices) final_whole_ = false;
+        if (q.d.flags & F_CIC) final_lds_ = std::max(final_lds_, (size_t)q.d.nbins * 8);
         q.d.unb = (q.d.flags & F_WAKE) && q.d.nJ > 1 ? q.d.hist + 2 * hist_half(q.d.nbins) : nullptr;
         for (int r = 0; r < q.d.nred; ++r) {
             red.push_back((int32_t)i);
@@ -554,6 +558,7 @@ hm_status Batch::build_tables() {
     ntiles_ = (int)tiles.size();
     nred_ = (int)red.size() / 2;
     nlist_ = (int)list.size();
+    if (nlist_ >= kWholeMinBunches) final_whole_ = true;
     nbw_ = (int)bw.size();
     nb64_ = (int)b64.size();
     bw.insert(bw.begin(), b64.begin(), b64.end());
@@ -1047,7 +1052,6 @@ hm_status Batch::one_turn() {
     HIP_TRY(launch_hist_slabs(d_bd_.p, d_slab_.p, nslab_, s));
     HIP_TRY(launch_bin_64(d_bd_.p, d_bw_.p, nb64_, bw_lds_, s));
     HIP_TRY(launch_bin_whole(d_bd_.p, d_bw_.p + nb64_, nbw_, bw_lds_, s));
-    const bool whole = nlist_ >= kWholeMinBunches;
     HIP_TRY(launch_reduce_fwd(d_bd_.p, d_red_.p, any_reduce_ ? nred_ : 0, d_conv_[CONV_FWD].p,
                               nconv_[CONV_FWD], Fmax_, s));
     if (any_wake_) {
@@ -1061,8 +1065,8 @@ hm_status Batch::one_turn() {
     if (any_wake_e0_)   // two workgroups per CU when both windows fit the LDS
         HIP_TRY(launch_interp_sum(d_bd_.p, d_order_.p, d_runs_.p, d_ranges_.p + pass_grid_ + 1,
                                   interp_grid_, interp_lds_, interp_deep_, s));
-    HIP_TRY(whole ? launch_finalize_whole(d_bd_.p, d_list_.p, nlist_, s)
-                  : launch_finalize(d_bd_.p, d_red_.p, nred_, s));
+    HIP_TRY(final_whole_ ? launch_finalize_whole(d_bd_.p, d_list_.p, nlist_, final_lds_, s)
+                         : launch_finalize(d_bd_.p, d_red_.p, nred_, s));
     return HM_OK;
 }
 

@@ -259,10 +259,13 @@ class Batch {
     // k_bin_whole takes a bunch whose tables fit this much LDS (up to 1024
     // bins at the tuned blocks)
     static constexpr size_t kBinWholeMaxLds = 144 * 1024;
-    // one workgroup per bunch for the reductions once the bunches alone fill
-    // the device (no cross-workgroup counts, whose device-scope fences cost
-    // more than the slices gain there)
+    // The finalize takes one workgroup per bunch where no bunch has more slices
+    // of interpolation sums than this (2 slices: 6.3 -> 4.5 us; 16: as fast
+    // either way), or the bunches alone fill the device.
+    static constexpr int kWholeMaxSlices = 8;
     static constexpr int kWholeMinBunches = 16;
+    bool final_whole_ = true;
+    size_t final_lds_ = 0;
     int nconv_[kConvKinds] = {0, 0, 0, 0, 0};
     size_t spec_lds_ = 0;   // LDS of the spectral-sum workgroups
     size_t pass_lds_ = 0;

@@ -104,9 +104,9 @@ hipError_t launch_hist_slabs(const BunchDev *bds, const int32_t *items, int nite
 hipError_t launch_reduce_fwd(const BunchDev *bds, const int32_t *red, int nred, const int32_t *items,
                              int nitems, int Fmax, hipStream_t s);
 hipError_t launch_finalize(const BunchDev *bds, const int32_t *items, int nitems, hipStream_t s);
-// the same with one 1024-thread workgroup per listed bunch and no
-// cross-workgroup count: the same bits (for batches of many bunches)
-hipError_t launch_finalize_whole(const BunchDev *bds, const int32_t *bunch_list, int nb,
+// the same bits with one 1024-thread workgroup per listed bunch and no
+// cross-workgroup count; lds: 8 bytes per bin of the largest grid with a deposit
+hipError_t launch_finalize_whole(const BunchDev *bds, const int32_t *bunch_list, int nb, size_t lds,
                                  hipStream_t s);
 // The whole bin phase (the reduction, the convolution and the finalize) of
 // each listed bunch in one 1024-thread workgroup: the same bits as the
