@@ -48,13 +48,20 @@ void *arena_take(Arena *a, size_t bytes) {
     return a->base + off;
 }
 
+// Copies up to this size go through a CopyList, larger ones by copy calls
+static constexpr size_t kListedBytes = 256 << 10;
+
 hm_status stage_begin(hm_ctx *ctx, size_t bytes) {
     Staging &g = ctx->stage;
-    g.used = 0;
+    g.n = 0;
     if (current_arena()) return HM_OK;
-    if (g.pending) {
-        HIP_TRY(hipEventSynchronize(g.done));
+    // a round follows the one before in the buffer; at its end it waits for
+    // the copies that still read the buffer and starts over
+    g.used = stage_size(g.used);
+    if (g.used + bytes > g.cap) {
+        if (g.pending) HIP_TRY(hipEventSynchronize(g.done));
         g.pending = false;
+        g.used = 0;
     }
     if (bytes > g.cap) {
         if (g.host) (void)hipHostFree(g.host);
@@ -65,6 +72,14 @@ hm_status stage_begin(hm_ctx *ctx, size_t bytes) {
         g.cap = c;
     }
     if (!g.done) HIP_TRY(hipEventCreateWithFlags(&g.done, hipEventDisableTiming));
+    return HM_OK;
+}
+
+static hm_status stage_flush(hm_ctx *ctx) {
+    Staging &g = ctx->stage;
+    const int n = g.n;
+    g.n = 0;
+    HIP_TRY(launch_copies(g.list, n, ctx->stream));
     return HM_OK;
 }
 
@@ -79,7 +94,12 @@ hm_status stage_copy(hm_ctx *ctx, void *dst, const void *src, size_t bytes) {
     if (off + bytes > g.cap) return fail(HM_ERR_LIMIT, "staging round overflows its size");
     std::memcpy(g.host + off, src, bytes);
     g.used = off + bytes;
-    HIP_TRY(hipMemcpyAsync(dst, g.host + off, bytes, hipMemcpyHostToDevice, ctx->stream));
+    if (bytes > kListedBytes || bytes % 4 != 0) {
+        HIP_TRY(hipMemcpyAsync(dst, g.host + off, bytes, hipMemcpyHostToDevice, ctx->stream));
+        return HM_OK;
+    }
+    if (g.n == kCopyList) HM_TRY(stage_flush(ctx));
+    g.list.e[g.n++] = {dst, g.host + off, (uint32_t)(bytes / 4)};
     return HM_OK;
 }
 
@@ -89,8 +109,42 @@ hm_status stage_end(hm_ctx *ctx) {
         HIP_TRY(hipStreamSynchronize(ctx->stream));
         return HM_OK;
     }
+    HM_TRY(stage_flush(ctx));
     HIP_TRY(hipEventRecord(g.done, ctx->stream));
     g.pending = true;
+    return HM_OK;
+}
+
+// Fetches pieces of device memory (sizes multiples of 4 bytes) and waits; piece k
+// is then at back[k], until the next fetch.
+static hm_status fetch(hm_ctx *ctx, const std::vector<std::pair<const void *, size_t>> &pieces,
+                       std::vector<const char *> &back) {
+    Staging &g = ctx->stage;
+    size_t bytes = 0;
+    for (auto &pc : pieces) bytes += stage_size(pc.second);
+    if (bytes > g.back_cap) {
+        if (g.back) (void)hipHostFree(g.back);
+        g.back = nullptr;
+        g.back_cap = 0;
+        const size_t c = std::max<size_t>(stage_size(bytes), size_t(1) << 16);
+        HIP_TRY(hipHostMalloc((void **)&g.back, c, hipHostMallocDefault));
+        g.back_cap = c;
+    }
+    back.clear();
+    CopyList l;
+    int n = 0;
+    size_t off = 0;
+    for (auto &pc : pieces) {
+        if (n == kCopyList) {
+            HIP_TRY(launch_copies(l, n, ctx->stream));
+            n = 0;
+        }
+        l.e[n++] = {g.back + off, pc.first, (uint32_t)(pc.second / 4)};
+        back.push_back(g.back + off);
+        off += stage_size(pc.second);
+    }
+    HIP_TRY(launch_copies(l, n, ctx->stream));
+    HIP_TRY(hipStreamSynchronize(ctx->stream));
     return HM_OK;
 }
 
@@ -749,8 +803,35 @@ hm_status Batch::add(const std::vector<RunBunch> &specs, std::vector<int> *idx) 
     return HM_OK;
 }
 
+namespace {
+// Buffers to clear, many by one launch.  Larger ones than kListedBytes by one
+// of their own.
+struct Clears {
+    hipStream_t s;
+    CopyList l;
+    int n = 0;
+    explicit Clears(hipStream_t st) : s(st) {}
+    hm_status add(void *p, size_t bytes) {
+        if (bytes > kListedBytes) {
+            HIP_TRY(launch_zero(p, bytes, s));
+            return HM_OK;
+        }
+        if (n == kCopyList) HM_TRY(flush());
+        l.e[n++] = {p, nullptr, (uint32_t)(bytes / 4)};
+        return HM_OK;
+    }
+    hm_status flush() {
+        const int k = n;
+        n = 0;
+        HIP_TRY(launch_copies(l, k, s));
+        return HM_OK;
+    }
+};
+}  // namespace
+
 hm_status Batch::add_slots(const std::vector<RunBunch> &specs, std::vector<int32_t> &fresh) {
     hipStream_t s = ctx_->stream;
+    Clears clears{s};
     for (const RunBunch &spec : specs) {
         HM_TRY(validate(&spec.p, &spec.o, spec.b->n, spec.nbins));
         int slot = -1;
@@ -811,12 +892,12 @@ hm_status Batch::add_slots(const std::vector<RunBunch> &specs, std::vector<int32
         HM_TRY(w.moments.ensure((size_t)std::max(d.ntiles, 1) * 4));
         HM_TRY(w.sc.ensure(1));
         HM_TRY(w.out.ensure(16));
-        HIP_TRY(launch_zero(w.out.p, 16 * sizeof(double), s));
+        HM_TRY(clears.add(w.out.p, 16 * sizeof(double)));
         d.spread = d.ntiles >= kSpreadTiles ? ~31 : 0;
         d.nred = red_slices(d.ntiles);
         HM_TRY(w.red.ensure((size_t)d.nred * 4));
         HM_TRY(w.cnt.ensure(1));
-        HIP_TRY(launch_zero(w.cnt.p, sizeof(uint32_t), s));
+        HM_TRY(clears.add(w.cnt.p, sizeof(uint32_t)));
         d.red = w.red.p;
         d.cnt = w.cnt.p;
         d.part = w.part.p;
@@ -833,7 +914,7 @@ hm_status Batch::add_slots(const std::vector<RunBunch> &specs, std::vector<int32
         }
         if (q.o.monitor && q.n_turns > 0) {   // copied to q.o.monitor by run_batch
             HM_TRY(w.mon.ensure((size_t)q.n_turns * 4));
-            HIP_TRY(launch_zero(w.mon.p, (size_t)q.n_turns * 4 * sizeof(double), s));
+            HM_TRY(clears.add(w.mon.p, (size_t)q.n_turns * 4 * sizeof(double)));
             d.mon = w.mon.p;
         }
         q.o.normals = nullptr;  // host memory of the caller: not kept
@@ -855,7 +936,9 @@ hm_status Batch::add_slots(const std::vector<RunBunch> &specs, std::vector<int32
     if (injected) HIP_TRY(hipStreamSynchronize(s));  // the normals' copies read the caller's memory
     // initial spreads (evolution.jl:245-253): compute_global_std, or for the
     // serial branch compute_std (two passes) into out[0..1]
+    HM_TRY(clears.flush());
     HM_TRY(run_subset_moments(fresh, 0));
+    std::vector<double> spreads(2 * fresh.size());
     for (int32_t i : fresh) {
         RunBunch &q = rb_[(size_t)i];
         if (!q.o.serial || q.b->n < 2) continue;   // n < 2: both forms give 0
@@ -865,16 +948,27 @@ hm_status Batch::add_slots(const std::vector<RunBunch> &specs, std::vector<int32
         HIP_TRY(hipMemcpyAsync(q.d.out + 1, q.d.out + 11, sizeof(double), hipMemcpyDeviceToDevice,
                                s));
     }
+    if (current_arena()) {
+        for (size_t k = 0; k < fresh.size(); ++k)
+            HIP_TRY(hipMemcpyAsync(&spreads[2 * k], rb_[(size_t)fresh[k]].d.out, 2 * sizeof(double),
+                                   hipMemcpyDeviceToHost, s));
+        HIP_TRY(hipStreamSynchronize(s));
+    } else {
+        std::vector<std::pair<const void *, size_t>> pieces;
+        std::vector<const char *> back;
+        for (int32_t i : fresh) pieces.emplace_back(rb_[(size_t)i].d.out, 2 * sizeof(double));
+        HM_TRY(fetch(ctx_, pieces, back));
+        for (size_t k = 0; k < fresh.size(); ++k)
+            std::memcpy(&spreads[2 * k], back[k], 2 * sizeof(double));
+    }
     // the callers' tables, uploaded in one staging round after the loop
     std::vector<std::pair<double *, std::vector<double>>> keep;
-    for (int32_t i : fresh) {
+    for (size_t fi = 0; fi < fresh.size(); ++fi) {
+        const int32_t i = fresh[fi];
         RunBunch &q = rb_[(size_t)i];
         BunchDev &d = q.d;
-        double o2[2];
-        HIP_TRY(hipMemcpyAsync(o2, d.out, sizeof(o2), hipMemcpyDeviceToHost, s));
-        HIP_TRY(hipStreamSynchronize(s));
-        d.sigma_E0 = o2[0];
-        const double sz0 = o2[1];
+        d.sigma_E0 = spreads[2 * fi];
+        const double sz0 = spreads[2 * fi + 1];
         if (!(d.flags & F_WAKE)) continue;
         // evolution.jl:263-281
         const int64_t nb = q.nbins;
@@ -896,7 +990,7 @@ hm_status Batch::add_slots(const std::vector<RunBunch> &specs, std::vector<int32
         const double wf = ((120.0 * kPi) * kSpeedLight) / (kPi * q.p.pipe_radius);   // evolution.jl:279
         const double ws = std::sqrt(jl_max_h(0.0, (2.0 * 30.0) / q.p.pipe_radius));  // evolution.jl:280
         const double inv_ctau = 1.0 / 4e-3;                                          // wakefield.jl:158
-        const double d_inv = dsig > 0 ? 1.0 / (std::sqrt(kTwoPi) * dsig) : 0.0;       // utils.jl:61-62
+        const double d_inv = dsig > 0 ? 1.0 / (std::sqrt(kTwoPi) * dsig) : 1.0;       // utils.jl:61-62
         const double d_ef = dsig > 0 ? -0.5 / (dsig * dsig) : 0.0;
         // the wake table: the caller's, the reference's W(c_j)
         // (k_reference_tables) or the resonators' W(j step)
@@ -961,7 +1055,7 @@ hm_status Batch::add_slots(const std::vector<RunBunch> &specs, std::vector<int32
             d.iwin = (int32_t)std::min<int64_t>(nb, ((int64_t)ctx_->lds_max - 1024) / 8);
         }
         Work &w = q.b->w;
-        HM_TRY(w.hist.ensure((size_t)hist_half((int)nb) * 2 + 2 * kUnbSlots * 16));
+        HM_TRY(w.hist.ensure(w.hist_bytes((int)nb) / 4));
         HM_TRY(w.P.ensure((size_t)nb));
         HM_TRY(w.P2.ensure((size_t)nb * 2));
         HM_TRY(w.lam.ensure((size_t)nb));
@@ -977,21 +1071,21 @@ hm_status Batch::add_slots(const std::vector<RunBunch> &specs, std::vector<int32
             }
         }
         // (centres beyond 1e300 or NaN: the tables are those of 1e300, finite as ever)
-        HIP_TRY(launch_reference_tables(ref_table ? w.Wtmp.p : nullptr, dsig > 0 ? w.lam.p : nullptr,
+        HIP_TRY(launch_reference_tables(ref_table ? w.Wtmp.p : nullptr, w.lam.p,
                                         (int)nb, zw <= 1e300 ? zw : 1e300, wf, ws, inv_ctau, d_inv, d_ef,
                                         s));
-        if (!(dsig > 0)) HIP_TRY(launch_fill(w.lam.p, (size_t)nb, 1.0, s));
         if (rset.n > 0)
             HIP_TRY(launch_resonator_table(w.Wtmp.p, (int)nb, step, rset, s));
         else if (!ref_table)
             keep.emplace_back(w.Wtmp.p, std::move(W));
-        HIP_TRY(launch_zero(w.P.p, (size_t)nb * 8, s));
-        HIP_TRY(launch_zero(w.P2.p, (size_t)nb * 16, s));
+        HM_TRY(clears.add(w.P.p, (size_t)nb * 8));
+        HM_TRY(clears.add(w.P2.p, (size_t)nb * 16));
+        HM_TRY(clears.add(w.hist.p, w.hist_bytes((int)nb)));
         d.cic = nullptr;
         if (d.flags & F_CIC) {   // cleared again by each turn's finalize
             const size_t words = cic_words((int)nb);
             HM_TRY(w.cic.ensure(words));
-            HIP_TRY(launch_zero(w.cic.p, words * 8, s));
+            HM_TRY(clears.add(w.cic.p, words * 8));
             d.cic = w.cic.p;
         }
         d.P2 = w.P2.p;
@@ -1003,6 +1097,7 @@ hm_status Batch::add_slots(const std::vector<RunBunch> &specs, std::vector<int32
         HM_TRY(twiddles(ctx_, d.F, &tw));
         d.tw = tw;
     }
+    HM_TRY(clears.flush());
     {   // the callers' tables, the descriptors and the new bunches' list: one round
         HM_TRY(d_tmp_list_.ensure(fresh.size()));
         size_t bytes = stage_size(rb_.size() * sizeof(BunchDev)) + stage_size(fresh.size() * 4);
@@ -1119,7 +1214,7 @@ hm_status Batch::capture_graph() {
     return HM_OK;
 }
 
-hm_status Batch::advance(int64_t turns) {
+hm_status Batch::advance(int64_t turns, bool wait) {
     int64_t step = 0;
     for (;;) {
         std::vector<int32_t> retiring;
@@ -1161,7 +1256,7 @@ hm_status Batch::advance(int64_t turns) {
             if (used_[i] && rb_[i].active) rb_[i].turns_done += did;
     }
     HM_TRY(flush_timing());
-    HIP_TRY(hipStreamSynchronize(ctx_->stream));
+    if (wait) HIP_TRY(hipStreamSynchronize(ctx_->stream));
     return HM_OK;
 }
 
@@ -1174,10 +1269,45 @@ hm_status Batch::finish_now(int i) {
 
 hm_status Batch::result(int i, hm_result *r, double *cz, double *cE) {
     if (i < 0 || (size_t)i >= rb_.size() || !used_[(size_t)i]) return fail(HM_ERR_ARG, "bad slot");
-    RunBunch &q = rb_[(size_t)i];
     double o[16];
-    HIP_TRY(hipMemcpyAsync(o, q.d.out, sizeof(o), hipMemcpyDeviceToHost, ctx_->stream));
-    HIP_TRY(hipStreamSynchronize(ctx_->stream));
+    if (current_arena()) {
+        HIP_TRY(hipMemcpyAsync(o, rb_[(size_t)i].d.out, sizeof(o), hipMemcpyDeviceToHost, ctx_->stream));
+        HIP_TRY(hipStreamSynchronize(ctx_->stream));
+    } else {
+        std::vector<const char *> back;
+        HM_TRY(fetch(ctx_, {{rb_[(size_t)i].d.out, sizeof(o)}}, back));
+        std::memcpy(o, back[0], sizeof(o));
+    }
+    read_result(i, o, r, cz, cE);
+    return HM_OK;
+}
+
+hm_status Batch::results(const std::vector<int> &idx, std::vector<hm_result> &r, hm_bunch *b, double *z,
+                         double *dE) {
+    std::vector<std::pair<const void *, size_t>> pieces;
+    std::vector<const char *> back;
+    double o[16];
+    for (int i : idx) pieces.emplace_back(rb_[(size_t)i].d.out, sizeof(o));
+    if (z) {
+        pieces.emplace_back(b->z, (size_t)b->n * 8);
+        pieces.emplace_back(b->dE, (size_t)b->n * 8);
+    }
+    HM_TRY(fetch(ctx_, pieces, back));
+    r.resize(idx.size());
+    for (size_t k = 0; k < idx.size(); ++k) {
+        std::memcpy(o, back[k], sizeof(o));
+        read_result(idx[k], o, &r[k], nullptr, nullptr);
+    }
+    if (z) {
+        std::memcpy(z, back[idx.size()], (size_t)b->n * 8);
+        std::memcpy(dE, back[idx.size() + 1], (size_t)b->n * 8);
+    }
+    return HM_OK;
+}
+
+// a slot's result from its 16 output doubles
+void Batch::read_result(int i, const double *o, hm_result *r, double *cz, double *cE) const {
+    const RunBunch &q = rb_[(size_t)i];
     std::memset(r, 0, sizeof(*r));
     r->sigma_E0 = o[0];
     r->sigma_z0 = o[1];
@@ -1200,7 +1330,6 @@ hm_status Batch::result(int i, hm_result *r, double *cz, double *cE) {
     r->corr_z_dE = (q.o.fom_stats && q.b->n >= 2) ? o[13] : NAN;
     if (cz) *cz = o[7];
     if (cE) *cE = o[8];
-    return HM_OK;
 }
 
 void Batch::remove(int i) {
@@ -1219,7 +1348,8 @@ using namespace hm;
 // ---------------------------------------------------------------------------
 
 static hm_status run_batch(hm_ctx *ctx, int32_t nb, hm_bunch *const *bunches, const int64_t *nbins,
-                           const hm_params *params, const hm_options *opts, hm_result *results) {
+                           const hm_params *params, const hm_options *opts, hm_result *results,
+                           double *host_z = nullptr, double *host_dE = nullptr) {
     if (!ctx || nb <= 0 || !bunches || !params || !results) return fail(HM_ERR_ARG, "bad batch arguments");
     HM_TRY(set_device(ctx));
     bool timing = false;
@@ -1259,23 +1389,27 @@ static hm_status run_batch(hm_ctx *ctx, int32_t nb, hm_bunch *const *bunches, co
     HM_TRY(B.add(specs, &idx));
     int64_t max_turns = 0;
     for (auto &q : specs) max_turns = std::max<int64_t>(max_turns, q.p.n_turns);
-    HM_TRY(B.advance(max_turns));
+    HM_TRY(B.advance(max_turns, false));
     HIP_TRY(hipEventRecord(t1, ctx->stream));
-    HIP_TRY(hipEventSynchronize(t1));
+    std::vector<hm_result> r;
+    HM_TRY(B.results(idx, r, specs[0].b, host_z, host_dE));
     float total_ms = 0.f;
     HIP_TRY(hipEventElapsedTime(&total_ms, t0, t1));
     (void)hipEventDestroy(t0);
     (void)hipEventDestroy(t1);
+    bool monitor = false;
     for (size_t k = 0; k < idx.size(); ++k) {
-        HM_TRY(B.result(idx[k], &results[orig[k]], nullptr, nullptr));
+        results[orig[k]] = r[k];
         results[orig[k]].ms_total = total_ms;
         const RunBunch &q = specs[k];
-        if (q.o.monitor && q.p.n_turns > 0)
+        if (q.o.monitor && q.p.n_turns > 0) {
             HIP_TRY(hipMemcpyAsync(q.o.monitor, q.b->w.mon.p,
                                    (size_t)q.p.n_turns * 4 * sizeof(double), hipMemcpyDeviceToHost,
                                    ctx->stream));
+            monitor = true;
+        }
     }
-    HIP_TRY(hipStreamSynchronize(ctx->stream));
+    if (monitor) HIP_TRY(hipStreamSynchronize(ctx->stream));
     return HM_OK;
 }
 
@@ -1321,6 +1455,7 @@ hm_status hm_destroy(hm_ctx *ctx) {
     ctx->ssc.release();
     ctx->sbd.release();
     if (ctx->stage.host) (void)hipHostFree(ctx->stage.host);
+    if (ctx->stage.back) (void)hipHostFree(ctx->stage.back);
     if (ctx->stage.done) (void)hipEventDestroy(ctx->stage.done);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
@@ -1459,8 +1594,17 @@ hm_status hm_evolve(hm_ctx *ctx, double *z, double *dE, int64_t n, int64_t nbins
         ctx->tmp = nullptr;
     }
     if (!ctx->tmp) HM_TRY(hm_bunch_create(ctx, n, &ctx->tmp));
-    HM_TRY(hm_bunch_upload(ctx->tmp, z, dE));
     hm_bunch *arr[1] = {ctx->tmp};
+    const size_t bytes = (size_t)n * 8;
+    if (n > 0 && bytes <= kListedBytes) {   // with the tables' and the results' copies
+        HM_TRY(set_device(ctx));
+        HM_TRY(stage_begin(ctx, 2 * stage_size(bytes)));
+        HM_TRY(stage_copy(ctx, ctx->tmp->z, z, bytes));
+        HM_TRY(stage_copy(ctx, ctx->tmp->dE, dE, bytes));
+        HM_TRY(stage_end(ctx));
+        return run_batch(ctx, 1, arr, &nbins, params, opts, result, z, dE);
+    }
+    HM_TRY(hm_bunch_upload(ctx->tmp, z, dE));
     HM_TRY(run_batch(ctx, 1, arr, &nbins, params, opts, result));
     return hm_bunch_download(ctx->tmp, z, dE);
 }

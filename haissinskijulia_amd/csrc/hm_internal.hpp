@@ -93,6 +93,10 @@ struct Work {
     DevBuf<double> red, Y;
     DevBuf<uint32_t> cnt;
     DevBuf<unsigned long long> cic;
+    // both halves, and the counts of particles not binned behind them
+    static size_t hist_bytes(int nbins) {
+        return ((size_t)hist_half(nbins) * 2 + 2 * kUnbSlots * 16) * 4;
+    }
     void release() {
         hist.release(); slabs.release(); P.release(); P2.release(); lam.release(); What.release(); X.release();
         Wtmp.release(); part.release(); ipart.release(); moments.release(); normals.release();
@@ -117,6 +121,11 @@ struct Staging {
     size_t cap = 0, used = 0;
     hipEvent_t done = nullptr;
     bool pending = false;
+    CopyList list;        // the round's copies that no launch has taken yet
+    int n = 0;
+    // the other way: device memory fetched into pinned memory in one launch
+    char *back = nullptr;
+    size_t back_cap = 0;
 };
 
 }  // namespace hm
@@ -195,11 +204,16 @@ class Batch {
     // slot this call took is released again and idx is left as it was.
     hm_status add(const std::vector<RunBunch> &specs, std::vector<int> *idx);
     // run up to `turns` turns of every active bunch; bunches that reach their
-    // n_turns run the epilogue and become finished
-    hm_status advance(int64_t turns);
+    // n_turns run the epilogue and become finished.  wait: returns with the
+    // turns done, else with them enqueued
+    hm_status advance(int64_t turns, bool wait = true);
     // stop a bunch now (epilogue included), e.g. a failed or cancelled job
     hm_status finish_now(int i);
     hm_status result(int i, hm_result *r, double *centroid_z, double *centroid_E);
+    // the results of the slots idx, and where z is given the particles of
+    // bunch b (the only slot), with one wait
+    hm_status results(const std::vector<int> &idx, std::vector<hm_result> &r, hm_bunch *b, double *z,
+                      double *dE);
     void remove(int i);   // forget a finished slot (the bunch itself is the caller's)
     int active_count() const;
     size_t size() const { return rb_.size(); }
@@ -211,6 +225,8 @@ class Batch {
     int64_t pass_count() const { return pass_count_; }
 
   private:
+    void read_result(int i, const double *o, hm_result *r, double *centroid_z,
+                     double *centroid_E) const;
     hm_status add_slots(const std::vector<RunBunch> &specs, std::vector<int32_t> &fresh);
     hm_status build_tables();
     hm_status build_free_tables();

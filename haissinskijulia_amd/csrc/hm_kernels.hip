@@ -1706,7 +1706,7 @@ __global__ void k_resonator_table(double *__restrict__ W, int nb, double step, R
 
 // The reference's tables of the bin centres (set-up of an evolve call): its
 // wake W(c) (wakefield.jl:115-118) and the delta kernel (utils.jl:58-66), each
-// where asked for.  The centre is the correctly rounded zw num / nb: with
+// where asked for (ef = 0: the constant s_inv).  The centre is the correctly rounded zw num / nb: with
 // zw num = p + e and the quotient q of p, the remainder p + e - q nb is exact
 // (both parts are multiples of q's last place, less than nb of them), and
 // q plus the remainder's quotient rounds once: that quotient's own rounding is
@@ -1725,7 +1725,7 @@ __global__ void k_reference_tables(double *__restrict__ W, double *__restrict__ 
     const double q = p / den;
     const double c = q + (__builtin_fma(-q, den, p) + e) / den;
     if (W) W[i] = c > 0.0 ? 0.0 : (wf * exp(c * inv_ctau)) * cos(ws * c);
-    if (lam) lam[i] = s_inv * exp((c * c) * ef);
+    if (lam) lam[i] = ef == 0.0 ? s_inv : s_inv * exp((c * c) * ef);
 }
 
 // FFT of one wake block per workgroup (set-up of an evolve call)
@@ -2151,9 +2151,6 @@ __global__ __launch_bounds__(kFinalThreads) void k_moments_final(const BunchDev 
 __global__ __launch_bounds__(kFinalThreads) void k_init(const BunchDev *__restrict__ bds,
                                                         const int32_t *__restrict__ list) {
     const BunchDev &B = bds[list[blockIdx.x]];
-    if (B.flags & F_WAKE)
-        for (int b = threadIdx.x; b < 2 * hist_half(B.nbins) + 2 * kUnbSlots * 16; b += blockDim.x)
-            B.hist[b] = 0u;   // and the counts of particles not binned behind it
     if (threadIdx.x == 0) {
         TurnScalars s = {};
         turn_scalars(B, B.E0_init, s);
@@ -3308,6 +3305,33 @@ hipError_t launch_finalize(const BunchDev *bds, const int32_t *items, int nitems
     return hipGetLastError();
 }
 
+__global__ __launch_bounds__(256) void k_copies(CopyList l) {
+    const uint32_t n = l.e[blockIdx.x].words, st = gridDim.y * 256u;
+    g_u32 *d = (g_u32 *)l.e[blockIdx.x].dst;
+    const g_u32 *s = (const g_u32 *)l.e[blockIdx.x].src;
+    if (!l.e[blockIdx.x].src) {
+        for (uint32_t i = blockIdx.y * 256u + threadIdx.x; i < n; i += st) d[i] = 0u;
+        return;
+    }
+    for (uint32_t i = blockIdx.y * 256u + threadIdx.x; i < n; i += 4 * st) {
+        uint32_t x[4];
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) x[u] = s[min(i + u * st, n - 1)];
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u)
+            if (i + u * st < n) d[i + u * st] = x[u];
+    }
+}
+
+hipError_t launch_copies(const CopyList &l, int n, hipStream_t s) {
+    if (n <= 0) return hipSuccess;
+    uint32_t words = 0;
+    for (int k = 0; k < n; ++k) words = std::max(words, l.e[k].words);
+    const uint32_t gy = std::min<uint32_t>(64, (words + 1023) / 1024);
+    hipLaunchKernelGGL(k_copies, dim3((unsigned)n, std::max<uint32_t>(gy, 1)), dim3(256), 0, s, l);
+    return hipGetLastError();
+}
+
 hipError_t launch_hist_slabs(const BunchDev *bds, const int32_t *items, int nitems, hipStream_t s) {
     if (nitems <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_hist_slabs, dim3(nitems), dim3(1024), 0, s, bds, items);
@@ -3348,20 +3372,6 @@ __global__ void k_zero(uint32_t *__restrict__ p, int64_t words) {
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < words;
          i += (int64_t)gridDim.x * blockDim.x)
         p[i] = 0u;
-}
-
-__global__ void k_fill(double *__restrict__ p, int64_t n, double v) {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (int64_t)gridDim.x * blockDim.x)
-        p[i] = v;
-}
-
-hipError_t launch_fill(double *p, size_t n, double v, hipStream_t s) {
-    if (n == 0) return hipSuccess;
-    const int64_t b = ((int64_t)n + 255) / 256;
-    hipLaunchKernelGGL(k_fill, dim3((unsigned)(b < 1024 ? b : 1024)), dim3(256), 0, s, p,
-                       (int64_t)n, v);
-    return hipGetLastError();
 }
 
 hipError_t launch_zero(void *p, size_t bytes, hipStream_t s) {

@@ -55,8 +55,21 @@ inline bool conv_spec_fits(int nA, int nJ, int F, int lds_max) {
 // zero `bytes` (a multiple of 4) at p by a kernel (no memset node: callers may
 // capture the stream)
 hipError_t launch_zero(void *p, size_t bytes, hipStream_t s);
-// p[0..n) = v by a kernel
-hipError_t launch_fill(double *p, size_t n, double v, hipStream_t s);
+// Up to kCopyList copies of 4-byte words between pinned host and device memory
+// by one kernel, which reads and writes the host's memory itself; a piece
+// without a source is cleared.  A copy call or a launch each took about 4 us of
+// the host and 2 to 3 of the stream, a pageable copy 15 to 25: a call of 4000
+// particles and 10 turns took 476 us with them, 370 so.
+constexpr int kCopyList = 32;
+struct CopyList {
+    struct {
+        void *dst;
+        const void *src;
+        uint32_t words;
+    } e[kCopyList];
+};
+hipError_t launch_copies(const CopyList &l, int n, hipStream_t s);
+
 // allow the dynamic-LDS kernels the device's LDS per block (best effort)
 hipError_t configure_kernels(int max_dynamic_lds);
 
