@@ -655,6 +655,17 @@ __device__ __forceinline__ uint32_t &pass_unbinned() {
     return s_unb;
 }
 
+// the next unit of the workgroup's run, and the single particle of an odd
+// bunch: z, its energy change, and 1 if it is not binned
+__device__ __forceinline__ int &pass_next() {
+    __shared__ int s_next;
+    return s_next;
+}
+__device__ __forceinline__ double (&pass_odd())[3] {
+    __shared__ double s_odd[3];
+    return s_odd;
+}
+
 // Copies the w entries from P to LDS, both 16-byte aligned, by 16-byte loads,
 // kStageLoads in flight per thread (eight spend registers and gain nothing).  In
 // 8-byte loads a window of 97 KB took 3 us of a pass and 128 KB 3 us of an
@@ -748,11 +759,16 @@ __device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlan
 // by several workgroups has its tiles dealt to them in turn).  Tiles are whole
 // multiples of the block size, so thread t's pairs in tile lt are
 // lt*ppt + t + k*kPassThreads in ascending k, exactly as for a tile taken
-// alone.  The loop over them is uniform: one chunk of kPassThreads pairs per
-// step, its addresses a scalar base plus the thread's constant offset, the
-// next chunk (the next tile's first at a tile's end) prefetched; only the last
-// chunk of a bunch may be shorter, and its lanes past the end re-read its last
-// pair and skip the rest.  Each tile's per-wave sums are written at its end.
+// alone; the 64 consecutive t of a tile are a unit, with sums of its own.  The
+// waves take the run's units one by one from a counter in LDS, the next one
+// while they work on the last: with every wave bound to the same 64 threads of
+// each tile, the older waves of a SIMD ran ahead, and the last of the younger
+// ones ran alone (1e7 particles: a pass of 69.7 -> 68.3 us; 28 bunches: 165.7 ->
+// 159.4; 24 served jobs: 30.2 -> 29.2).  The loop over a unit is uniform: one chunk of
+// kPassThreads pairs per step, its addresses a scalar base plus the lane's
+// offset, the next chunk (the next unit's first at a unit's end) prefetched;
+// only the last chunk of a bunch may be shorter, and its lanes past the end
+// re-read its last pair and skip the rest.  A unit's sums are written at its end.
 // The pass is bound by vector instructions below about 1e8 particles: with
 // per-thread 64-bit positions and bounds the same loop spent 16 of them per
 // pair on addresses, and 130 per tile on spilled scalars (a turn of a scan of 28
@@ -799,37 +815,65 @@ __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *
     const int spread = HM == kHistLds ? 0 : B.spread, hwin = B.hwin;
     const int hlo = HM == kHistWindow ? uni(window_lo(sc.centre_bin, hwin, c.nb)) : 0;
     g_u32 *n_bad = CIC ? cic_n(B) + hist_half(c.nb) : nullptr;
-    const unsigned tid = t0 + threadIdx.x;
-    const int wave = uni((int)(tid >> 6));
+    const int lane = (int)threadIdx.x & 63;
+    const int lw = 31 - __builtin_clz(blockDim.x >> 6);   // log2 of the waves
+    const int units = cnt << lw;
     constexpr unsigned step = kPassThreads;
 
     // pair `base` + (byte offset / 16) of the z or dE array
     auto at = [](g_f64 *a, unsigned base, unsigned off) -> g_f64x2 * {
         return (g_f64x2 *)((g_u8 *)a + (int64_t)base * 16 + off);
     };
-    // per-wave partial sums of a tile: no workgroup barrier per tile, so a wave
-    // never waits for the others of its workgroup between tiles
-    auto flush = [&](const double (&v)[4], int lt) {
+    // a unit's partial sums: no workgroup barrier per tile, so a wave never
+    // waits for the others of its workgroup between tiles
+    auto flush = [&](const double (&v)[4], int lt, int slot) {
         const double tot = wave_total4(v);
-        const int lane = (int)tid & 63;
-        g_f64 *o = (g_f64 *)B.part + 4 * ((int64_t)lt * kTileWaves + wave);
+        g_f64 *o = (g_f64 *)B.part + 4 * ((int64_t)lt * kTileWaves + slot);
         if (lane >= 60) o[lane - 60] = tot;
         if (unb && lane == 63 && tot != 0.0) atomicAdd(&pass_unbinned(), (uint32_t)tot);
     };
-    // the single particle of an odd bunch sits in the bunch's last tile, the
-    // last of this run if the run has it: that tile is flushed after the loop
+    // The single particle of an odd bunch sits in the bunch's last tile, the
+    // last of this run if the run has it, and belongs to that tile's first
+    // thread, whose unit adds it last.  Its turn is out of the loop over the
+    // units, so that it does not add to the loop's register pressure.
     const int lt_last = run[cnt - 1] - tb;
-    const bool odd_tile = (n & 1) && (int64_t)full >= (int64_t)lt_last * ppt &&
-                          (int64_t)full < min((int64_t)(lt_last + 1) * ppt, B.npairs);
-    double v[4] = {0.0, 0.0, 0.0, 0.0};   // sum z, sum z^2, sum (dE'-dE_init), not binned
-    // a chunk's byte offset for this thread; lanes past the end take its last pair
-    auto offset = [&](unsigned lim) -> unsigned { return min(tid, lim - 1) * 16u; };
+    const bool odd = (n & 1) && t0 == 0 && (int64_t)full >= (int64_t)lt_last * ppt &&
+                     (int64_t)full < min((int64_t)(lt_last + 1) * ppt, B.npairs);
+    if (odd) {
+        if (threadIdx.x == 0) {
+            const int64_t i = n - 1;
+            double z0 = zp[i], e0 = ep[i], r0 = 0.0, r1 = 0.0;
+            if (qe) {
+                if (inj) r0 = nrm[i];
+                else qe_pair_normals32(seed, full, tabs, r0, r1);
+            }
+            e0 = apply_pending(c, z0, e0);
+            double d0, v[4] = {0.0, 0.0, 0.0, 0.0};
+            advance(c, fl, z0, e0, r0, d0);
+            if (wake) bin_and_sum<HM, CIC>(c, ghist, spread, hlo, hwin, n_bad, z0, v);
+            if (CIC) cic_deposit(c, cb, z0);
+            zp[i] = z0;
+            ep[i] = e0;
+            pass_odd()[0] = z0;
+            pass_odd()[1] = d0;
+            pass_odd()[2] = v[3];
+        }
+        __syncthreads();
+    }
+    double v[4];   // sum z, sum z^2, sum (dE'-dE_init), not binned
+    // a chunk's byte offset for a thread; lanes past the end take its last pair
+    auto offset = [&](unsigned tid, unsigned lim) -> unsigned { return min(tid, lim - 1) * 16u; };
+    // unit u: its tile, and its lanes' threads of the tile
+    auto tile_of = [&](int u) { return run[u >> lw] - tb; };
+    auto tid_of = [&](int u) { return t0 + (unsigned)((u & ((1 << lw) - 1)) << 6) + (unsigned)lane; };
     double2 zn = make_double2(0.0, 0.0), en = make_double2(0.0, 0.0);
-    int lt = run[0] - tb;
+    int u = uni((int)(threadIdx.x >> 6));
+    int lt = tile_of(u);
+    unsigned tid = tid_of(u);
     {
         const unsigned b0 = (unsigned)lt * ppt, lim = min(full - b0, step);   // b0 <= full
         if (lim > 0) {
-            const unsigned off = offset(lim);
+            const unsigned off = offset(tid, lim);
             zn = ldp<NT>(at(zp, b0, off));
             en = ldp<NT>(at(ep, b0, off));
         }
@@ -838,10 +882,16 @@ __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *
     // the pair in hand is never taken for an outstanding load and the waits
     // there count only the loads issued in the loop
     __builtin_amdgcn_s_waitcnt(0x0F70);
-    for (int t = 0; t < cnt; ++t) {
+    while (u < units) {
         const unsigned p0 = (unsigned)lt * ppt;
         const unsigned p1 = min(p0 + ppt, full);
-        const int ltn = t + 1 < cnt ? run[t + 1] - tb : lt;
+        int un = units;   // the next unit; a single tile has one for each wave
+        if (cnt > 1) {
+            if (lane == 0) un = atomicAdd(&pass_next(), 1);
+            un = uni(un);
+        }
+        const int ltn = un < units ? tile_of(un) : lt;
+        const unsigned tidn = un < units ? tid_of(un) : tid;
 #pragma unroll
         for (int k = 0; k < 4; ++k) v[k] = 0.0;
         for (unsigned base = p0; base < p1; base += step) {
@@ -856,14 +906,16 @@ __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *
             // first.  The order of the loads changes no result.
             constexpr bool gather = KM != kFullWindow;
             constexpr bool gather_first = KM == kGatherFirst;
-            // the next chunk (the next tile's first at a tile's end); past the
+            // the next chunk (the next unit's first at a unit's end); past the
             // end of the run, or where that tile has no pair of two particles,
-            // this chunk is read again and not used, so the load is
-            // unconditional and zn, en need no copy of their old value
+            // the tile's first chunk or this one is read again and not used,
+            // so the load is unconditional and zn, en need no copy of their
+            // old value
             auto prefetch = [&]() {
-                unsigned bn = base + step < p1 ? base + step : (unsigned)ltn * ppt;
+                const bool more = base + step < p1;
+                unsigned bn = more ? base + step : (unsigned)ltn * ppt;
                 if (bn >= full) bn = base;
-                const unsigned off = offset(min(full - bn, step));
+                const unsigned off = offset(more ? tid : tidn, min(full - bn, step));
                 zn = ldp<NT>(at(zp, bn, off));
                 en = ldp<NT>(at(ep, bn, off));
             };
@@ -951,32 +1003,17 @@ __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *
                 stp<NT>(at(ep, base, tid * 16u), e0, e1);
             }
         }
-        if (odd_tile && t == cnt - 1) break;   // v kept for the single particle
-        if (!wake) { v[0] = 0.0; v[1] = 0.0; }
-        flush(v, lt);
-        lt = ltn;
-    }
-    // the single particle of an odd bunch (last pair), out of the tile loop so
-    // that its inlined turn does not add to the loop's register pressure
-    if (odd_tile) {
-        if (tid == 0) {
-            const int64_t i = n - 1;
-            double z0 = zp[i], e0 = ep[i], r0 = 0.0, r1 = 0.0;
-            if (qe) {
-                if (inj) r0 = nrm[i];
-                else qe_pair_normals32(seed, full, tabs, r0, r1);
-            }
-            e0 = apply_pending(c, z0, e0);
-            double d0;
-            advance(c, fl, z0, e0, r0, d0);
-            if (wake) bin_and_sum<HM, CIC>(c, ghist, spread, hlo, hwin, n_bad, z0, v);
-            if (CIC) cic_deposit(c, cb, z0);
-            v[2] += d0;
-            zp[i] = z0;
-            ep[i] = e0;
+        if (odd && lt == lt_last && tid == (unsigned)lane && lane == 0) {   // the unit of slot 0
+            v[0] += pass_odd()[0];
+            v[1] = __builtin_fma(pass_odd()[0], pass_odd()[0], v[1]);
+            v[3] += pass_odd()[2];
+            v[2] += pass_odd()[1];
         }
         if (!wake) { v[0] = 0.0; v[1] = 0.0; }
-        flush(v, lt_last);
+        flush(v, lt, uni((int)(tid >> 6)));
+        u = un;
+        lt = ltn;
+        tid = tidn;
     }
 }
 
@@ -1031,7 +1068,10 @@ __device__ inline void flush_hist(const BunchDev &B, int slab, int unb) {
 template <uint32_t FX>
 __device__ inline void stage_bunch(const BunchDev &B, int unb) {
     __syncthreads();   // the previous bunch's LDS is no longer read
-    if (unb && threadIdx.x == 0) pass_unbinned() = 0u;
+    if (threadIdx.x == 0) {
+        if (unb) pass_unbinned() = 0u;
+        pass_next() = (int)(blockDim.x >> 6);   // each wave starts with the unit of its number
+    }
     const int hb = pass_hist_bytes(B);
     clear_lds(pass_lds(), hb);
     if (B.flags & F_CIC) clear_lds(pass_lds() + B.cic_off, cic_bytes(B.nbins));
