@@ -2693,20 +2693,23 @@ __global__ __launch_bounds__(1024) void k_bin_64(const BunchDev *__restrict__ bd
     const int tid = (int)threadIdx.x, lane = tid & 63;
     const int sp = B.spread;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int64_t turn = ((const TurnScalars *)B.sc)->turn;
-    // the binned count, from both halves' counts (this turn's is known a load later)
+    // The first loads, all in flight together: the twiddles for LDS, s_tw[tid] =
+    // w1, wa or wb (c = 0, 1, 2) of stage pair r at butterfly index k, by waves 0
+    // and 1; the turn; both halves' counts (this turn's is known a load later).
+    // Without branches: the compiler waited for all of them before the first
+    // one's, and loaded the twiddles after (1024 bins: 9.6 -> 9.4 us).
+    double2 twv = make_double2(0.0, 0.0);
+    if (wave < 2) {
+        const int r = (tid >= 6) + (tid >= 30), q = tid - 6 * r - 18 * (r >> 1);
+        const int k = q & ((2 << (2 * r)) - 1), c = q >> (2 * r + 1), m = max(c - 1, 0);
+        twv = ld2((const g_f64x2 *)B.tw + min((k + (m << (2 * r + 1))) << (5 - 2 * r - min(c, 1)), 63));
+    }
+    const int64_t turn = *(const __attribute__((address_space(1))) int64_t *)&B.sc->turn;
     const g_u32 *hist = (const g_u32 *)B.hist;
     const int bin = min(tid, nb - 1);
     const uint32_t h0 = hist[spread32(sp, bin)], h1 = hist[hist_half(nb) + spread32(sp, bin)];
     const double lam = ((const g_f64 *)B.lam)[bin];
-    {
-        int r = 0, c = tid;   // s_tw[tid] = w1, wa or wb (c) of stage pair r at butterfly index k
-        if (c >= 30) { r = 2; c -= 30; } else if (c >= 6) { r = 1; c -= 6; }
-        const int hh = 2 << (2 * r), k = c & (hh - 1), sh = 5 - 2 * r;
-        c >>= 2 * r + 1;
-        if (tid < 126)
-            s_tw[tid] = ld2((const g_f64x2 *)B.tw + (c == 0 ? k << sh : (c == 1 ? k : k + hh) << (sh - 1)));
-    }
+    if (tid < 126) s_tw[tid] = twv;
     const uint32_t hc = tid < nb ? ((turn & 1) ? h1 : h0) : 0u;
     {
         uint32_t c = hc;
