@@ -609,6 +609,10 @@ hm_status Batch::build_tables() {
             Fmax_ = std::max(Fmax_, q.d.F);
         }
     }
+    int64_t zbytes = 0;
+    for (size_t i = 0; i < rb_.size(); ++i)
+        if (used_[i] && rb_[i].active) zbytes += 8 * rb_[i].d.n;
+    keep_z_ = zbytes > kKeepMinBytes && zbytes <= kKeepMaxBytes;
     ntiles_ = (int)tiles.size();
     nred_ = (int)red.size() / 2;
     nlist_ = (int)list.size();
@@ -1142,7 +1146,7 @@ hm_status Batch::one_turn() {
         HIP_TRY(hipEventRecord(e0, s));
     }
     HIP_TRY(launch_turn_pass(d_bd_.p, d_order_.p, d_runs_.p, d_ranges_.p, pass_grid_, pass_slices_, pass_lds_,
-                             std_only_ ? 1 : 0, nconv_[CONV_FWD] > 0 ? 1 : 0, s));
+                             std_only_ ? 1 : 0, nconv_[CONV_FWD] > 0 ? 1 : 0, keep_z_, s));
     if (timing_) HIP_TRY(hipEventRecord(e1, s));
     HIP_TRY(launch_hist_slabs(d_bd_.p, d_slab_.p, nslab_, s));
     HIP_TRY(launch_bin_64(d_bd_.p, d_bw_.p, nb64_, bw_lds_, s));
@@ -1159,7 +1163,7 @@ hm_status Batch::one_turn() {
     if (timing_) HIP_TRY(hipEventRecord(e2, s));
     if (any_wake_e0_)   // two workgroups per CU when both windows fit the LDS
         HIP_TRY(launch_interp_sum(d_bd_.p, d_order_.p, d_runs_.p, d_ranges_.p + pass_grid_ + 1,
-                                  interp_grid_, interp_lds_, interp_deep_, s));
+                                  interp_grid_, interp_lds_, interp_deep_, keep_z_, s));
     HIP_TRY(final_whole_ ? launch_finalize_whole(d_bd_.p, d_list_.p, nlist_, final_lds_, s)
                          : launch_finalize(d_bd_.p, d_red_.p, nred_, s));
     return HM_OK;

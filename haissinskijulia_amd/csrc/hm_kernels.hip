@@ -779,12 +779,12 @@ __device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlan
 // particles outside it gather from global memory; see the loop body).
 // CIC: the bunch's post-drift z are also deposited (cic_deposit) into the LDS
 // counters at byte cb.
-// NT: the particles are streamed past the caches, which are left to the bin
+// NTZ, NTE: z, dE are streamed past the caches, which are left to the bin
 // phase's tables.
 // With FX = kStdFlags the kick is applied from the first turn on: P is zero
 // before it, and subtracting 0 changes nothing.
 enum KickMode { kFullWindow = 0, kGatherFirst = 1, kPrefetchFirst = 2 };
-template <uint32_t FX, int HM, int KM, bool CIC, bool NT = true>
+template <uint32_t FX, int HM, int KM, bool CIC, bool NTZ, bool NTE = true>
 __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *__restrict__ run,
                                               int cnt, unsigned t0, int hb, int cb, int unb) {
     PassCtx c;
@@ -874,8 +874,8 @@ __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *
         const unsigned b0 = (unsigned)lt * ppt, lim = min(full - b0, step);   // b0 <= full
         if (lim > 0) {
             const unsigned off = offset(tid, lim);
-            zn = ldp<NT>(at(zp, b0, off));
-            en = ldp<NT>(at(ep, b0, off));
+            zn = ldp<NTZ>(at(zp, b0, off));
+            en = ldp<NTE>(at(ep, b0, off));
         }
     }
     // the first chunk completes here (s_waitcnt vmcnt(0)), so that in the loop
@@ -916,8 +916,8 @@ __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *
                 unsigned bn = more ? base + step : (unsigned)ltn * ppt;
                 if (bn >= full) bn = base;
                 const unsigned off = offset(more ? tid : tidn, min(full - bn, step));
-                zn = ldp<NT>(at(zp, bn, off));
-                en = ldp<NT>(at(ep, bn, off));
+                zn = ldp<NTZ>(at(zp, bn, off));
+                en = ldp<NTE>(at(ep, bn, off));
             };
             if (!gather_first) prefetch();
             // set and read only when kick2 (no per-pair clearing)
@@ -999,8 +999,8 @@ __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *
                 }
                 v[2] += d0;
                 v[2] += d1;
-                stp<NT>(at(zp, base, tid * 16u), z0, z1);
-                stp<NT>(at(ep, base, tid * 16u), e0, e1);
+                stp<NTZ>(at(zp, base, tid * 16u), z0, z1);
+                stp<NTE>(at(ep, base, tid * 16u), e0, e1);
             }
         }
         if (odd && lt == lt_last && tid == (unsigned)lane && lane == 0) {   // the unit of slot 0
@@ -1092,7 +1092,7 @@ __device__ inline void stage_bunch(const BunchDev &B, int unb) {
 // scalar loads per tile before the first byte was streamed.  Launched with half
 // the threads, two consecutive workgroups share a range, each with the tiles'
 // lower or upper eight waves and LDS tables of its own.
-template <uint32_t FX>
+template <uint32_t FX, bool NTZ>
 __device__ __forceinline__ void turn_pass_blocks(const BunchDev *__restrict__ bds,
                                                  const int32_t *__restrict__ order,
                                                  const RunDev *__restrict__ runs,
@@ -1114,38 +1114,40 @@ __device__ __forceinline__ void turn_pass_blocks(const BunchDev *__restrict__ bd
         const bool full = B.win >= B.nbins;
         const int cb = B.cic_off;
         if (B.flags & F_CIC) {   // the deposit comes with the whole table
-            turn_pass_run<FX, kHistLds, kFullWindow, true>(B, run, cnt, t0, hb, cb, unb);
+            turn_pass_run<FX, kHistLds, kFullWindow, true, NTZ>(B, run, cnt, t0, hb, cb, unb);
         } else if (!(B.flags & F_GHIST)) {   // a bunch without a wake among them
             if (full)
-                turn_pass_run<FX, kHistLds, kFullWindow, false>(B, run, cnt, t0, hb, cb, unb);
+                turn_pass_run<FX, kHistLds, kFullWindow, false, NTZ>(B, run, cnt, t0, hb, cb, unb);
             else
-                turn_pass_run<FX, kHistLds, kPartial, false>(B, run, cnt, t0, hb, cb, unb);
+                turn_pass_run<FX, kHistLds, kPartial, false, NTZ>(B, run, cnt, t0, hb, cb, unb);
         } else if (FX != 0 || B.hwin > 0) {
             if (cached(B))
-                turn_pass_run<FX, kHistWindow, kPartial, false, false>(B, run, cnt, t0, hb, cb, unb);
+                turn_pass_run<FX, kHistWindow, kPartial, false, false, false>(B, run, cnt, t0, hb, cb, unb);
             else
-                turn_pass_run<FX, kHistWindow, kPartial, false>(B, run, cnt, t0, hb, cb, unb);
+                turn_pass_run<FX, kHistWindow, kPartial, false, NTZ>(B, run, cnt, t0, hb, cb, unb);
         } else {
-            turn_pass_run<FX, kHistGlobal, kPrefetchFirst, false>(B, run, cnt, t0, hb, cb, unb);
+            turn_pass_run<FX, kHistGlobal, kPrefetchFirst, false, NTZ>(B, run, cnt, t0, hb, cb, unb);
         }
         flush_hist(B, rd.slab + (int)slice, unb);
     }
 }
 
+template <bool NTZ>
 __global__ __launch_bounds__(kPassThreads) void k_turn_pass(const BunchDev *__restrict__ bds,
                                                             const int32_t *__restrict__ order,
                                                             const RunDev *__restrict__ runs,
                                                             const int32_t *__restrict__ rr, int unb) {
-    turn_pass_blocks<0>(bds, order, runs, rr, unb);
+    turn_pass_blocks<0, NTZ>(bds, order, runs, rr, unb);
 }
 
 // the same for tables whose bunches all have exactly kStdFlags, two bins or more
 // and some of their histogram in LDS
+template <bool NTZ>
 __global__ __launch_bounds__(kPassThreads) void k_turn_pass_std(const BunchDev *__restrict__ bds,
                                                                 const int32_t *__restrict__ order,
                                                                 const RunDev *__restrict__ runs,
                                                                 const int32_t *__restrict__ rr, int unb) {
-    turn_pass_blocks<kStdFlags>(bds, order, runs, rr, unb);
+    turn_pass_blocks<kStdFlags, NTZ>(bds, order, runs, rr, unb);
 }
 
 // ---------------------------------------------------------------------------
@@ -2021,12 +2023,12 @@ __device__ __forceinline__ void interp_sum_run_w(const BunchDev &B, const int32_
         interp_sum_run_flat<FULLW, NT>(B, run, nrun);
 }
 
-template <int G>
+template <int G, bool NTZ>
 __device__ __forceinline__ void interp_sum_run(const BunchDev &B, const int32_t *run, int nrun) {
     if (B.iwin >= B.nbins)
-        interp_sum_run_w<G, true, true>(B, run, nrun);
+        interp_sum_run_w<G, true, NTZ>(B, run, nrun);
     else if (!cached(B))
-        interp_sum_run_w<G, false, true>(B, run, nrun);
+        interp_sum_run_w<G, false, NTZ>(B, run, nrun);
     else
         interp_sum_run_w<G, false, false>(B, run, nrun);
 }
@@ -2034,7 +2036,7 @@ __device__ __forceinline__ void interp_sum_run(const BunchDev &B, const int32_t 
 // The interpolation sums of the wake + update_E0 bunches over a tile table:
 // each workgroup walks its runs of the sums' tile order (a bunch shared by
 // several workgroups has its tiles dealt to them in turn, as in the pass).
-template <int G>
+template <int G, bool NTZ>
 __device__ __forceinline__ void interp_sum_blocks(const BunchDev *__restrict__ bds,
                                                   const int32_t *__restrict__ order,
                                                   const RunDev *__restrict__ runs,
@@ -2044,24 +2046,26 @@ __device__ __forceinline__ void interp_sum_blocks(const BunchDev *__restrict__ b
         const RunDev rd = runs[r];
         const BunchDev &B = bds[rd.bunch];
         if ((B.flags & F_WAKE) && (B.flags & F_E0) && !(B.flags & F_CIC))
-            interp_sum_run<G>(B, order + rd.begin, rd.count);
+            interp_sum_run<G, NTZ>(B, order + rd.begin, rd.count);
     }
 }
 
 // At most 64 VGPRs, so that two workgroups fit a CU when both windows fit its
 // LDS; rings of four loads.
+template <bool NTZ>
 __global__ __launch_bounds__(kInterpThreads) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_interp_sum(
     const BunchDev *__restrict__ bds, const int32_t *__restrict__ order,
     const RunDev *__restrict__ runs, const int32_t *__restrict__ rr) {
-    interp_sum_blocks<4>(bds, order, runs, rr);
+    interp_sum_blocks<4, NTZ>(bds, order, runs, rr);
 }
 
 // One workgroup per CU (a window of P larger than half the LDS): the
 // registers of four waves per SIMD allow rings of eight loads.
+template <bool NTZ>
 __global__ __launch_bounds__(kInterpThreads) void k_interp_sum_deep(
     const BunchDev *__restrict__ bds, const int32_t *__restrict__ order,
     const RunDev *__restrict__ runs, const int32_t *__restrict__ rr) {
-    interp_sum_blocks<8>(bds, order, runs, rr);
+    interp_sum_blocks<8, NTZ>(bds, order, runs, rr);
 }
 
 // Per-tile sums of z, z^2, dE, dE^2 (the initial and final spreads,
@@ -3244,13 +3248,15 @@ __global__ __launch_bounds__(1024) void k_stream_copy(const f64x2 *__restrict__ 
 static inline unsigned blocks_for(int64_t n, int t) { return (unsigned)((n + t - 1) / t); }
 
 hipError_t configure_kernels(int lds) {
-    const void *fns[] = {(const void *)k_turn_pass, (const void *)k_turn_pass_std,
+    const void *fns[] = {(const void *)k_turn_pass<true>, (const void *)k_turn_pass<false>,
+                         (const void *)k_turn_pass_std<true>, (const void *)k_turn_pass_std<false>,
                          (const void *)k_conv_fused,
                          (const void *)k_conv_fwd, (const void *)k_reduce_fwd,
                          (const void *)k_conv_inv,
                          (const void *)k_conv_spec, (const void *)k_conv_out,
                          (const void *)k_fft_wake, (const void *)k_stage_hist,
-                         (const void *)k_interp_sum, (const void *)k_interp_sum_deep,
+                         (const void *)k_interp_sum<true>, (const void *)k_interp_sum<false>,
+                         (const void *)k_interp_sum_deep<true>, (const void *)k_interp_sum_deep<false>,
                          (const void *)k_bin_whole, (const void *)k_bin_64};
     hipError_t last = hipSuccess;
     for (const void *f : fns) {
@@ -3291,13 +3297,12 @@ hipError_t launch_init(const BunchDev *bds, const int32_t *list, int nb, hipStre
 
 hipError_t launch_turn_pass(const BunchDev *bds, const int32_t *order, const RunDev *runs,
                             const int32_t *rr, int grid, int slices, size_t lds, int std_only,
-                            int unb, hipStream_t s) {
+                            int unb, bool keep_z, hipStream_t s) {
     if (grid <= 0) return hipSuccess;
     const dim3 blocks((unsigned)(grid * slices)), threads((unsigned)(kPassThreads / slices));
-    if (std_only)
-        hipLaunchKernelGGL(k_turn_pass_std, blocks, threads, lds, s, bds, order, runs, rr, unb);
-    else
-        hipLaunchKernelGGL(k_turn_pass, blocks, threads, lds, s, bds, order, runs, rr, unb);
+    auto *k = std_only ? (keep_z ? k_turn_pass_std<false> : k_turn_pass_std<true>)
+                       : (keep_z ? k_turn_pass<false> : k_turn_pass<true>);
+    hipLaunchKernelGGL(k, blocks, threads, lds, s, bds, order, runs, rr, unb);
     return hipGetLastError();
 }
 
@@ -3331,14 +3336,12 @@ hipError_t launch_conv(int kind, const BunchDev *bds, const int32_t *items, int 
 
 hipError_t launch_interp_sum(const BunchDev *bds, const int32_t *order, const RunDev *runs,
                              const int32_t *rr, int grid, size_t lds_bytes, bool deep,
-                             hipStream_t s) {
+                             bool keep_z, hipStream_t s) {
     if (grid <= 0) return hipSuccess;
-    if (deep)
-        hipLaunchKernelGGL(k_interp_sum_deep, dim3((unsigned)grid), dim3(kInterpThreads), lds_bytes,
-                           s, bds, order, runs, rr);
-    else
-        hipLaunchKernelGGL(k_interp_sum, dim3((unsigned)grid), dim3(kInterpThreads), lds_bytes, s,
-                           bds, order, runs, rr);
+    auto *k = deep ? (keep_z ? k_interp_sum_deep<false> : k_interp_sum_deep<true>)
+                   : (keep_z ? k_interp_sum<false> : k_interp_sum<true>);
+    hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(kInterpThreads), lds_bytes, s, bds, order, runs,
+                       rr);
     return hipGetLastError();
 }
 

@@ -85,10 +85,10 @@ hipError_t launch_init(const BunchDev *bds, const int32_t *bunch_list, int nb, h
 // [rr[g], rr[g+1]); lds_bytes = the largest per-bunch histogram + potential
 // window; std_only: every bunch has (flags & kPhysMask) == kStdFlags, two bins
 // or more and (F_GHIST) hwin > 0; unb: some bunch's particles not binned are
-// counted (BunchDev::unb)
+// counted (BunchDev::unb); keep_z: z stays in the caches (Batch::keep_z_)
 hipError_t launch_turn_pass(const BunchDev *bds, const int32_t *order, const RunDev *runs,
                             const int32_t *rr, int grid, int slices, size_t lds, int std_only,
-                            int unb, hipStream_t s);
+                            int unb, bool keep_z, hipStream_t s);
 // `turns` turns of bunches without a wake and without the E0 update: items
 // cover the listed bunches' pairs
 constexpr int kFreeThreads = 256;
@@ -104,7 +104,7 @@ hipError_t launch_conv(int kind, const BunchDev *bds, const int32_t *items, int 
 // deep: one workgroup per CU, eight streaming loads in flight per thread
 hipError_t launch_interp_sum(const BunchDev *bds, const int32_t *order, const RunDev *runs,
                              const int32_t *rr, int grid, size_t lds_bytes, bool deep,
-                             hipStream_t s);
+                             bool keep_z, hipStream_t s);
 // the slabs of the windowed histograms added up: items are (bunch, group of 512
 // bins of its window) pairs
 hipError_t launch_hist_slabs(const BunchDev *bds, const int32_t *items, int nitems, hipStream_t s);
