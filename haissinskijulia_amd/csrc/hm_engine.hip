@@ -519,6 +519,7 @@ hm_status Batch::build_tables() {
     final_lds_ = 0;
     bw_lds_ = 0;
     spec_lds_ = 0;
+    spec_threads_ = kConvThreads;
     Fmax_ = 2;
     any_wake_ = any_wake_e0_ = any_reduce_ = false;
     std_only_ = true;
@@ -605,6 +606,8 @@ hm_status Batch::build_tables() {
                     conv[CONV_SPEC].push_back(c);
                 }
                 spec_lds_ = std::max(spec_lds_, conv_spec_lds(q.d.nA, q.d.nJ, q.d.F));
+                spec_threads_ = std::min(kConvMaxThreads,
+                                         std::max(spec_threads_, (q.d.nA * spec_chunk(q.d.nA, q.d.F) + 63) & ~63));
             }
             Fmax_ = std::max(Fmax_, q.d.F);
         }
@@ -1156,7 +1159,7 @@ hm_status Batch::one_turn() {
     if (any_wake_) {
         HIP_TRY(launch_conv(CONV_FUSED, d_bd_.p, d_conv_[CONV_FUSED].p, nconv_[CONV_FUSED], Fmax_, s));
         HIP_TRY(launch_conv(CONV_SPEC, d_bd_.p, d_conv_[CONV_SPEC].p, nconv_[CONV_SPEC],
-                            (int)spec_lds_, s));
+                            (int)spec_lds_, s, spec_threads_));
         HIP_TRY(launch_conv(CONV_OUT, d_bd_.p, d_conv_[CONV_OUT].p, nconv_[CONV_OUT], Fmax_, s));
         HIP_TRY(launch_conv(CONV_INV, d_bd_.p, d_conv_[CONV_INV].p, nconv_[CONV_INV], Fmax_, s));
     }

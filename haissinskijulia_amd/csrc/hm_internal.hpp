@@ -292,6 +292,7 @@ class Batch {
     size_t final_lds_ = 0;
     int nconv_[kConvKinds] = {0, 0, 0, 0, 0};
     size_t spec_lds_ = 0;   // LDS of the spectral-sum workgroups
+    int spec_threads_ = kConvThreads;   // and their threads
     size_t pass_lds_ = 0;
     int Fmax_ = 2;
     bool any_wake_ = false, any_wake_e0_ = false;   // some bunch with wake / wake + update_E0

@@ -298,10 +298,10 @@ __device__ __forceinline__ double butterfly(double v) {
 // Deterministic block sum of NV values: wave butterflies, then the waves in
 // order.  The result is valid in thread 0.  s_red holds NV * 16 doubles.
 template <int NV>
-__device__ inline void block_sum(double (&v)[NV], double *s_red) {
+__device__ inline void block_sum(double (&v)[NV], double *s_red, int nw = (int)(blockDim.x >> 6)) {
 #pragma unroll
     for (int k = 0; k < NV; ++k) v[k] = butterfly(v[k]);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     if (lane == 0) {
 #pragma unroll
         for (int k = 0; k < NV; ++k) s_red[k * 16 + wave] = v[k];
@@ -1275,7 +1275,7 @@ __device__ inline void slice_sum(const double *a, int n, int r, double (&v)[NV],
     for (int k = 0; k < kRedPer; ++k)
 #pragma unroll
         for (int j = 0; j < NV; ++j) v[j] += x[k][j];
-    block_sum<NV>(v, s_red);
+    block_sum<NV>(v, s_red, kRedThreads / 64);
 }
 
 // Counts slice r of bunch B in, its NV sums (thread 0's v) first stored at
@@ -1593,10 +1593,11 @@ __global__ __launch_bounds__(kConvThreads) void k_conv_fwd(const BunchDev *__res
 // 5 to 7 us each, one after the other: 1e6 particles, 16384 bins: 56.5 -> 52.4 us a
 // turn; 1e7, 8192 bins: 120 -> 117; 28 bunches of 4096 bins, which had one
 // workgroup per bunch for the reductions: 212 -> 210.
-__global__ __launch_bounds__(kConvThreads) void k_reduce_fwd(const BunchDev *__restrict__ bds,
+__global__ __launch_bounds__(kConvMaxThreads) void k_reduce_fwd(const BunchDev *__restrict__ bds,
                                                              const int32_t *__restrict__ red, int nred,
                                                              const int32_t *__restrict__ items) {
     if ((int)blockIdx.x < nred) {
+        if ((int)threadIdx.x >= kRedThreads) return;   // whole waves, before any barrier
         bin_reduce(bds[red[2 * blockIdx.x]], red[2 * blockIdx.x + 1]);
         return;
     }
@@ -1617,7 +1618,7 @@ __global__ __launch_bounds__(kConvThreads) void k_reduce_fwd(const BunchDev *__r
 // once per output block as in k_conv_inv); a thread takes one (frequency,
 // output block) pair.  The products are added in ascending j from zero, as in
 // k_conv_inv, so Y_o and the potential are the same bits on either path.
-__global__ __launch_bounds__(kConvThreads) void k_conv_spec(const BunchDev *__restrict__ bds,
+__global__ __launch_bounds__(kConvMaxThreads) void k_conv_spec(const BunchDev *__restrict__ bds,
                                                             const int32_t *__restrict__ items) {
     extern __shared__ double2 sS[];
     const BunchDev &B = bds[items[2 * blockIdx.x]];
@@ -1653,7 +1654,7 @@ __global__ __launch_bounds__(kConvThreads) void k_conv_spec(const BunchDev *__re
 }
 
 // phase B2: inverse FFT of Y_o, P block o
-__global__ __launch_bounds__(kConvThreads) void k_conv_out(const BunchDev *__restrict__ bds,
+__global__ __launch_bounds__(kConvMaxThreads) void k_conv_out(const BunchDev *__restrict__ bds,
                                                            const int32_t *__restrict__ items) {
     extern __shared__ double2 sX[];
     const BunchDev &B = bds[items[2 * blockIdx.x]];
@@ -3316,8 +3317,14 @@ hipError_t launch_free_turns(const BunchDev *bds, const RunDev *items, int nitem
     return hipGetLastError();
 }
 
+// A butterfly per thread and stage of the longest transform (2048 points, 131072
+// bins: k_reduce_fwd 13.1 -> 11.3 us, k_conv_out 11.2 -> 9.6 by 1024 threads)
+static unsigned fft_threads(int Fmax) {
+    return (unsigned)std::min(std::max(Fmax / 2, kConvThreads), kConvMaxThreads);
+}
+
 hipError_t launch_conv(int kind, const BunchDev *bds, const int32_t *items, int nitems, int Fmax,
-                       hipStream_t s) {
+                       hipStream_t s, int threads) {
     if (nitems <= 0) return hipSuccess;
     const size_t lds = (size_t)Fmax * 16;
     if (kind == CONV_FUSED)
@@ -3327,10 +3334,10 @@ hipError_t launch_conv(int kind, const BunchDev *bds, const int32_t *items, int 
     else if (kind == CONV_INV)
         hipLaunchKernelGGL(k_conv_inv, dim3(nitems), dim3(kConvInvThreads), lds, s, bds, items);
     else if (kind == CONV_SPEC)
-        hipLaunchKernelGGL(k_conv_spec, dim3(nitems), dim3(kConvThreads), (size_t)Fmax, s, bds,
+        hipLaunchKernelGGL(k_conv_spec, dim3(nitems), dim3((unsigned)threads), (size_t)Fmax, s, bds,
                            items);
     else
-        hipLaunchKernelGGL(k_conv_out, dim3(nitems), dim3(kConvThreads), lds, s, bds, items);
+        hipLaunchKernelGGL(k_conv_out, dim3(nitems), dim3(fft_threads(Fmax)), lds, s, bds, items);
     return hipGetLastError();
 }
 
@@ -3387,8 +3394,8 @@ hipError_t launch_hist_slabs(const BunchDev *bds, const int32_t *items, int nite
 hipError_t launch_reduce_fwd(const BunchDev *bds, const int32_t *red, int nred, const int32_t *items,
                              int nitems, int Fmax, hipStream_t s) {
     if (nred + nitems <= 0) return hipSuccess;
-    static_assert(kRedThreads == kConvThreads, "one launch for both");
-    hipLaunchKernelGGL(k_reduce_fwd, dim3(nred + nitems), dim3(kConvThreads),
+    static_assert(kRedThreads <= kConvThreads, "one launch for both");
+    hipLaunchKernelGGL(k_reduce_fwd, dim3(nred + nitems), dim3(nitems > 0 ? fft_threads(Fmax) : kRedThreads),
                        nitems > 0 ? (size_t)Fmax * 16 : 0, s, bds, red, nred, items);
     return hipGetLastError();
 }
