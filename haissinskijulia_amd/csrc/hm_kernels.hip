@@ -2675,7 +2675,7 @@ __device__ __forceinline__ double2 dpp_swap1(double2 v) {   // the neighbouring 
 //   reduce meanwhile; one of their lanes (kScalarThread) does the scalars.
 // It is bound by LDS bandwidth: 264 KB for the forward transforms and 320 KB for
 // the spectral sums of 1024 bins, at 128 B a cycle.  Measured in a turn: 1024
-// bins 17.7 us (k_bin_whole) -> 9.5 us, 512 bins 12.7 -> 7.4 us.
+// bins 17.7 us (k_bin_whole) -> 9.4 us, 512 bins 12.7 -> 7.7 us.
 constexpr int kScalarThread = 512;
 // A point's place in its block in LDS: the stages' strides (2, 8 and 32 points of
 // 16 bytes) and the contiguous reads then spread over all banks.

@@ -157,8 +157,8 @@ hipError_t launch_bin_whole(const BunchDev *bds, const int32_t *bunch_list, int 
 // (what the tuned table gives 256 to 1024 bins), at most 16 of them, a wake of
 // more than one block (one block has nothing to sum), at most four reduction
 // slices, and the whole potential in the pass's window `win` (k_bin_64 leaves
-// the neighbour-pair table out).  Same bits; in a turn 9.5 us against 17.7 us
-// at 1024 bins, 7.4 against 12.7 us at 512.  Its LDS fits in
+// the neighbour-pair table out).  Same bits; in a turn 9.4 us against 17.7 us
+// at 1024 bins, 7.7 against 12.7 us at 512.  Its LDS fits in
 // bin_whole_layout(...).bytes.
 inline bool fits_bin_64(bool wake, int nbins, int win, int nA, int nJ, int F, int nred) {
     return wake && F == 128 && nbins >= 2 && nA <= 16 && nJ > 1 && nJ <= 16 && nred <= 4 && win >= nbins;
