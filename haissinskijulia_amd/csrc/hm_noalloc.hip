@@ -25,11 +25,15 @@
 
 namespace {
 
-// 8 MiB: the work set of a bunch of up to 32768 bins (about 32 B per bin for
+// 9 MiB: the work set of a bunch of up to 32768 bins (about 32 B per bin for
 // each of the three spectra tables, 48 B per bin for the histogram halves and
 // the potential tables, ~0.7 MB of per-tile sums for the at most 1025 tiles of
-// any bunch size)
-constexpr size_t kScratchBytes = size_t(8) << 20;
+// any bunch size) in 5 MB; the rest is for the sums of a caller's smaller tiles
+// (672 B each; 1.09e7 particles of 1024-pair tiles on 32768 bins).  1 MiB of it
+// pays for the counters that leave every other 128 bytes out (8 B per bin, 28
+// with the deposit) and the items of k_free_turns: in 8 MiB such a bunch ended
+// at 1.01e7 particles.
+constexpr size_t kScratchBytes = size_t(9) << 20;
 constexpr int64_t kMaxBins = 32768;
 
 __device__ __align__(256) unsigned char scratch[kScratchBytes];

@@ -165,7 +165,7 @@ hm_status hm_bunch_device_ptrs(hm_bunch *b, double **z_device, double **dE_devic
 /* No counterpart in the reference: hm_bunch_evolve on the caller's device
  * arrays z_device, dE_device (mutated in place) with no device allocation, for
  * callers that cannot allocate (code under stream capture, serving loops,
- * harnesses that forbid hipMalloc).  Every work buffer comes from an 8 MiB
+ * harnesses that forbid hipMalloc).  Every work buffer comes from a 9 MiB
  * per-GPU scratch array held until the process ends: at most 32768 bins
  * (HM_ERR_LIMIT beyond); no injected normals, turn monitor or timing
  * (HM_ERR_ARG).  The same kernels as hm_bunch_evolve, so the same results.
