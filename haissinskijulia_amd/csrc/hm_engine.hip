@@ -687,12 +687,10 @@ hm_status Batch::build_tables() {
     if (pass_grid_ > 0) find_runs(0, pass_grid_, 0, true);
     if (interp_grid_ > 0) find_runs((size_t)pass_grid_ + 1, interp_grid_, (size_t)ntiles_, false);
     nslab_ = (int)slab.size() / 2;
-    for (size_t i = 0; i < rb_.size(); ++i)
-        if (used_[i] && rb_[i].active && rb_[i].d.nslabs > 0) {
-            BunchDev &d = rb_[i].d;
-            HM_TRY(rb_[i].b->w.slabs.ensure((size_t)d.nslabs * (size_t)(d.hwin / 2)));
-            d.slabs = rb_[i].b->w.slabs.p;
-        }
+    for (size_t i = 0; i < rb_.size(); ++i)   // max_slabs of them were taken at set-up
+        if (used_[i] && rb_[i].active && rb_[i].d.nslabs > 0 &&
+            (size_t)rb_[i].d.nslabs * (size_t)(rb_[i].d.hwin / 2) > rb_[i].b->w.slabs.cap)
+            return fail(HM_ERR_LIMIT, "bunch %zu has more runs than slabs", i);
     // one staging round for every table and the descriptors
     size_t bytes = stage_size(ranges.size() * 4) + stage_size(list.size() * 4) +
                    stage_size(bw.size() * 4) +
@@ -1103,6 +1101,16 @@ hm_status Batch::add_slots(const std::vector<RunBunch> &specs, std::vector<int32
         const double *tw;
         HM_TRY(twiddles(ctx_, d.F, &tw));
         d.tw = tw;
+    }
+    // The slabs, last: a bunch they do not fit beside counts in global memory
+    // (the same counts), as a histogram without a window does.
+    for (int32_t i : fresh) {
+        BunchDev &d = rb_[(size_t)i].d;
+        if (d.hwin == 0) continue;
+        DevBuf<uint32_t> &slabs = rb_[(size_t)i].b->w.slabs;
+        if (slabs.ensure((size_t)max_slabs(d.ntiles, d.pairs_per_tile, ctx_->cus) * (size_t)(d.hwin / 2)) != HM_OK)
+            d.hwin = 0;
+        d.slabs = slabs.p;
     }
     HM_TRY(clears.flush());
     {   // the callers' tables, the descriptors and the new bunches' list: one round

@@ -71,6 +71,7 @@ struct DevBuf {
         hipError_t e = hipMalloc(&p, bytes);
         if (e != hipSuccess) {
             p = nullptr;
+            (void)hipGetLastError();   // reported here, not by the next launch
             return fail(HM_ERR_OOM, "hipMalloc(%zu bytes) failed: %s", bytes, hipGetErrorString(e));
         }
         cap = std::max<size_t>(n, 1);

@@ -1,0 +1,44 @@
+// hm_rules.hpp -- choices of the engine that depend on sizes alone: no device
+// code, so that the CPU can check them.
+#pragma once
+#include <stdint.h>
+
+#include <algorithm>
+
+namespace hm {
+
+// Histograms of more bins than the LDS holds 32-bit counts for (F_GHIST).  An
+// addition to global memory per particle was bound by the crowded lines: 1e7
+// particles, 131072 bins: a pass of 0.40 ms; 45056 bins 0.54 ms.  So the pass
+// counts a window of kHistWin bins around the centroid in LDS, in 16 bits (a run
+// has at most kHistRunPairs pairs, so they cannot overflow), stores each run's
+// window to a slab of its own without atomics, and k_hist_slabs adds the slabs
+// up; only particles outside the window add to global memory: 0.108 ms and
+// 0.083 ms.  49152 bins are +-2.8 sigma of a bunch on 131072 bins over +-7.5
+// sigma (one particle in 200 outside) and leave 8000 entries for the window of
+// P, which the kick reads; 32768, 40960 and 57344 bins: 0.084, 0.085 and 0.098
+// ms against 0.089 at 65536 bins, 0.105, 0.105 and 0.111 at 131072, but 0.173,
+// 0.153 and 0.138 against 0.145 at 262144.  Slabs cost a launch of 8 us a turn
+// (25 MB written and read), so 32-bit counts of all bins stay as long as they
+// leave kHistMinWin entries of P: 1e7 particles, 34000 bins 95 + 35 us of pass
+// and bin phase, 36000 bins by the window 80 + 43, 40000 bins 118 + 35 before and
+// 81 + 43 after.  Tiles of more than kHistRunPairs pairs cannot use 16 bits;
+// kHistMaxPairs bounds the slabs of one bunch to a few hundred MB.
+constexpr int kHistWin = 49152;
+constexpr int kHistRunPairs = 32767;
+constexpr int64_t kHistMaxPairs = 1 << 26;
+constexpr int kHistMinWin = 3072;
+
+// The most slabs the windowed histogram of a bunch of ntiles tiles of ppt pairs
+// can fill, alone or in any batch, on a device of cus CUs.  The pass has at most
+// a workgroup per CU, each with one stretch of the bunch's tiles, and a run of it
+// per kHistRunPairs pairs: a stretch of t tiles makes at most (t + per - 1) / per
+// runs.  A slab per run, two where tiles are split over two workgroups, which
+// takes at most cus / 2 tiles.  1e6 particles 263, 1e7 376 (alone both fill 256).
+inline int64_t max_slabs(int64_t ntiles, int64_t ppt, int cus) {
+    const int64_t per = std::max<int64_t>(1, kHistRunPairs / ppt);
+    const int64_t runs = std::min(ntiles, (ntiles + std::min<int64_t>(ntiles, cus) * (per - 1)) / per);
+    return 2 * ntiles <= cus ? 2 * ntiles : runs;
+}
+
+}  // namespace hm

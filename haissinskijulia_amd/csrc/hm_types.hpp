@@ -25,6 +25,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "hm_rules.hpp"
+
 namespace hm {
 
 constexpr double kTwoPi = 6.283185307179586;   // Julia's 2π as Float64
@@ -66,28 +68,6 @@ constexpr int64_t kCicRunPairs = (int64_t)1 << 20;
 // flags that select the pass's code path
 constexpr uint32_t kStdFlags = F_WAKE | F_ETA | F_E0 | F_SR | F_QE;
 constexpr uint32_t kPhysMask = F_WAKE | F_ETA | F_E0 | F_SR | F_QE | F_INJ;
-
-// Histograms of more bins than the LDS holds 32-bit counts for (F_GHIST).  An
-// addition to global memory per particle was bound by the crowded lines: 1e7
-// particles, 131072 bins: a pass of 0.40 ms; 45056 bins 0.54 ms.  So the pass
-// counts a window of kHistWin bins around the centroid in LDS, in 16 bits (a run
-// has at most kHistRunPairs pairs, so they cannot overflow), stores each run's
-// window to a slab of its own without atomics, and k_hist_slabs adds the slabs
-// up; only particles outside the window add to global memory: 0.108 ms and
-// 0.083 ms.  49152 bins are +-2.8 sigma of a bunch on 131072 bins over +-7.5
-// sigma (one particle in 200 outside) and leave 8000 entries for the window of
-// P, which the kick reads; 32768, 40960 and 57344 bins: 0.084, 0.085 and 0.098
-// ms against 0.089 at 65536 bins, 0.105, 0.105 and 0.111 at 131072, but 0.173,
-// 0.153 and 0.138 against 0.145 at 262144.  Slabs cost a launch of 8 us a turn
-// (25 MB written and read), so 32-bit counts of all bins stay as long as they
-// leave kHistMinWin entries of P: 1e7 particles, 34000 bins 95 + 35 us of pass
-// and bin phase, 36000 bins by the window 80 + 43, 40000 bins 118 + 35 before and
-// 81 + 43 after.  Tiles of more than kHistRunPairs pairs cannot use 16 bits;
-// kHistMaxPairs bounds the slabs of one bunch to a few hundred MB.
-constexpr int kHistWin = 49152;
-constexpr int kHistRunPairs = 32767;
-constexpr int64_t kHistMaxPairs = 1 << 26;
-constexpr int kHistMinWin = 3072;
 
 // Slots of the count of a turn's particles that are not binned: one 64-byte
 // line each, so that the pass's workgroups (one addition per run at most) do

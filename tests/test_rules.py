@@ -1,0 +1,46 @@
+"""The engine's choices by size (haissinskijulia_amd/csrc/hm_rules.hpp), compiled
+for the CPU from the same source (CPU)."""
+import ctypes as C
+import os
+import random
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+CUS = 256
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    out = tmp_path_factory.mktemp("rules") / "libhmrules.so"
+    subprocess.run(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", os.path.join(HERE, "rules_host_shim.cpp"),
+                    "-o", str(out)], check=True)
+    L = C.CDLL(str(out))
+    L.t_max_slabs.restype = C.c_int64
+    L.t_max_slabs.argtypes = [C.c_int64, C.c_int64, C.c_int]
+    return L
+
+
+def test_max_slabs_bounds_every_split(rules):
+    """Any split of a bunch's tiles over the pass's workgroups, beside any number
+    of other tiles: a run takes up to 32767 pairs, and each tile is split in two
+    where the workgroups, one per tile, number at most half the CUs."""
+    rng = random.Random(1)
+    for _ in range(20_000):
+        ppt = 1024 * rng.randint(1, 31)
+        ntiles = int(round(2 ** rng.uniform(0, 12)))
+        grid = min(ntiles + rng.choice((0, 0, 1, 7, 100, 1000)), CUS)
+        slices = 2 if 2 * grid <= CUS else 1
+        groups = rng.randint(1, min(ntiles, grid))
+        cuts = [0] + sorted(rng.sample(range(1, ntiles), groups - 1)) + [ntiles]
+        per = 32767 // ppt
+        runs = sum(-(-(b - a) // per) for a, b in zip(cuts, cuts[1:]))
+        assert slices * runs <= rules.t_max_slabs(ntiles, ppt, CUS)
+
+
+def test_max_slabs_of_a_lone_bunch_is_near_what_it_fills(rules):
+    assert rules.t_max_slabs(1, 1024, CUS) == 2
+    assert rules.t_max_slabs(128, 1024, CUS) == 256
+    assert rules.t_max_slabs(489, 1024, CUS) == 263      # 1e6 particles
+    assert rules.t_max_slabs(977, 5120, CUS) == 376      # 1e7
