@@ -322,19 +322,6 @@ hm_status validate(const hm_params *p, const hm_options *o, int64_t n, int64_t n
 // Batch
 // ---------------------------------------------------------------------------
 
-static int64_t pairs_per_tile_for(int64_t npairs, int threads, int32_t tile_pairs) {
-    // tiling depends on the bunch size (and the option) alone, so a bunch is
-    // reduced in the same order alone and in any batch: by default about 1024
-    // tiles of a large bunch (four per CU), at least one pair per thread.  A
-    // workgroup streams its run of consecutive tiles of a bunch as one loop,
-    // so small tiles cost no extra pipeline start.
-    if (tile_pairs > 0) return (int64_t)tile_pairs * threads;
-    const int64_t target_tiles = 1024;
-    int64_t ppt = (npairs + target_tiles - 1) / target_tiles;
-    ppt = ((ppt + threads - 1) / threads) * threads;
-    return std::max<int64_t>(ppt, (int64_t)threads);
-}
-
 // The turn pass's order of the tile table.  The balanced ranges give each
 // workgroup a contiguous block of entries; a bunch whose tiles fall in the
 // blocks of several workgroups has its tiles dealt to them in turn instead
@@ -1031,14 +1018,10 @@ hm_status Batch::add_slots(const std::vector<RunBunch> &specs, std::vector<int32
         d.logF = ilog2(d.F);
         d.nA = (int32_t)((nb + Bk - 1) / Bk);
         d.nJ = (int32_t)((nw + Bk - 1) / Bk);
-        // The whole histogram in LDS only with room for a window of at least
-        // two entries of P beside it (the all-flags pass relies on that), or,
-        // where a window of 16-bit counts can take its place (a tile's counts
-        // fit them), of kHistMinWin.
-        const bool hwin = d.pairs_per_tile <= kHistRunPairs && d.npairs <= kHistMaxPairs;
-        if ((size_t)nb * 4 + 8 * (size_t)(hwin ? kHistMinWin : 2) > (size_t)ctx_->lds_max - 1024) {
+        const int hwin = hist_window(nb, d.npairs, d.pairs_per_tile, ctx_->lds_max);
+        if (hwin >= 0) {
             d.flags |= F_GHIST;
-            d.hwin = hwin ? (int32_t)std::min<int64_t>(nb, kHistWin) & ~1 : 0;
+            d.hwin = hwin;
         }
         // With update_E0 the pass deposits the interpolation weights of its
         // post-drift z (cloud in cell) where its LDS holds the counters beside

@@ -83,7 +83,6 @@ struct DevBuf {
         cap = 0;
         from_arena = false;
     }
-    size_t bytes() const { return cap * sizeof(T); }
 };
 
 // per-bunch work buffers of an evolve call (kept between calls)
@@ -103,12 +102,6 @@ struct Work {
         Wtmp.release(); part.release(); ipart.release(); moments.release(); normals.release();
         out.release(); stats.release(); mon.release(); sc.release(); red.release(); cnt.release();
         Y.release(); cic.release();
-    }
-    size_t bytes() const {
-        return hist.bytes() + slabs.bytes() + P.bytes() + P2.bytes() + lam.bytes() + What.bytes() + X.bytes() +
-               Wtmp.bytes() + part.bytes() + ipart.bytes() + moments.bytes() + normals.bytes() +
-               out.bytes() + stats.bytes() + mon.bytes() + sc.bytes() + red.bytes() + cnt.bytes() +
-               Y.bytes() + cic.bytes();
     }
 };
 

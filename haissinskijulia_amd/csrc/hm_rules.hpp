@@ -7,6 +7,20 @@
 
 namespace hm {
 
+// Pairs per tile of a bunch.
+inline int64_t pairs_per_tile_for(int64_t npairs, int threads, int32_t tile_pairs) {
+    // tiling depends on the bunch size (and the option) alone, so a bunch is
+    // reduced in the same order alone and in any batch: by default about 1024
+    // tiles of a large bunch (four per CU), at least one pair per thread.  A
+    // workgroup streams its run of consecutive tiles of a bunch as one loop,
+    // so small tiles cost no extra pipeline start.
+    if (tile_pairs > 0) return (int64_t)tile_pairs * threads;
+    const int64_t target_tiles = 1024;
+    int64_t ppt = (npairs + target_tiles - 1) / target_tiles;
+    ppt = ((ppt + threads - 1) / threads) * threads;
+    return std::max<int64_t>(ppt, (int64_t)threads);
+}
+
 // Histograms of more bins than the LDS holds 32-bit counts for (F_GHIST).  An
 // addition to global memory per particle was bound by the crowded lines: 1e7
 // particles, 131072 bins: a pass of 0.40 ms; 45056 bins 0.54 ms.  So the pass
@@ -29,6 +43,16 @@ constexpr int kHistRunPairs = 32767;
 constexpr int64_t kHistMaxPairs = 1 << 26;
 constexpr int kHistMinWin = 3072;
 
+// Where a bunch of nb bins counts its histogram: -1 in LDS, 0 in global memory, else
+// the bins of its window in LDS.  The whole histogram in LDS only with room for a
+// window of at least two entries of P beside it (the all-flags pass relies on
+// that), or, where a window of 16-bit counts can take its place (a tile's counts
+// fit them), of kHistMinWin.
+inline int hist_window(int64_t nb, int64_t npairs, int64_t ppt, int lds_max) {
+    const bool window = ppt <= kHistRunPairs && npairs <= kHistMaxPairs;
+    if (4 * nb + 8 * (window ? kHistMinWin : 2) <= (int64_t)lds_max - 1024) return -1;
+    return window ? (int)std::min<int64_t>(nb, kHistWin) & ~1 : 0;
+}
 // The most slabs the windowed histogram of a bunch of ntiles tiles of ppt pairs
 // can fill, alone or in any batch, on a device of cus CUs.  The pass has at most
 // a workgroup per CU, each with one stretch of the bunch's tiles, and a run of it

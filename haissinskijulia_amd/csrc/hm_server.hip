@@ -30,10 +30,25 @@ struct Job {
     bool cancelled = false, failed_by_request = false;
 };
 
-size_t job_bytes(const hm_job &j) {
-    const size_t n = (size_t)std::max<int64_t>(j.n, 1);
-    const size_t nb = (size_t)std::max<int64_t>(j.nbins, 1);
-    return 16 * n + 104 * nb + (size_t)(1 << 16) + 2 * (size_t)kMaxFFT * 16;
+// What a job holds in device memory, at most: its particles, and the buffers of
+// Work as its set-up and its tables take them.  The wake's support is not known
+// before the bunch is, so the spectra count with as many blocks as the grid has.
+size_t job_bytes(const hm_ctx *ctx, const hm_job &j) {
+    const int64_t n = std::max<int64_t>(j.n, 1), npairs = (n + 1) / 2;
+    const int64_t ppt = pairs_per_tile_for(npairs, kPassThreads, j.opts.tile_pairs);
+    const int64_t tiles = (npairs + ppt - 1) / ppt;
+    // the particles; sums per wave of a tile (5) and per tile (4), per slice (4); the pairs' statistics
+    size_t bytes = 16 * (size_t)n + (size_t)tiles * (5 * kTileWaves + 4) * 8 +
+                   (size_t)red_slices((int)tiles) * 32 + 24 * kStatBlocks;
+    if (j.params.use_wakefield) {
+        const size_t nb = (size_t)j.nbins, block = (size_t)(j.opts.fft_block ? j.opts.fft_block : kAutoFFTBlock);
+        // P, its pairs, lambda, the wake; three tables of spectra; the counters
+        bytes += 40 * nb + 96 * (nb + block) + Work::hist_bytes((int)nb);
+        if (j.params.update_E0 && cic_bytes((int)nb) <= ctx->lds_max) bytes += cic_words((int)nb) * 8;
+        const int hwin = hist_window(j.nbins, npairs, ppt, ctx->lds_max);
+        if (hwin > 0) bytes += (size_t)max_slabs(tiles, ppt, ctx->cus) * (size_t)hwin * 2;
+    }
+    return bytes + (size_t)(1 << 16) + 2 * (size_t)kMaxFFT * 16;
 }
 
 }  // namespace
@@ -193,7 +208,7 @@ hm_status hm_server_submit(hm_server *s, const hm_job *job, int64_t *job_id) {
         j.res.assign(job->opts.resonators, job->opts.resonators + 3 * job->opts.n_resonators);
     j.spec.opts.wake_table = nullptr;
     j.spec.opts.resonators = nullptr;
-    j.bytes = job_bytes(*job);
+    j.bytes = job_bytes(s->ctx, *job);
     j.t_submit = s->now();
     if (job_id) *job_id = j.id;
     s->queue.push_back(std::move(j));

@@ -38,3 +38,22 @@ def test_a_jobs_buffers_are_taken_at_admission(n, nbins):
     res = {r.job_id: r for r in srv.run(10)}
     srv.close()
     assert res[job].status == 0
+
+
+@pytest.mark.parametrize("n,nbins,options", [(524_288, 65536, dict(tile_pairs=1)), (40_000, 131072, {}),
+                                             (200_000, 5000, dict(tile_pairs=1))])
+def test_admitted_jobs_stay_within_the_budget(n, nbins, options):
+    # 64 MiB; launch tables, and what the runtime rounds sizes up to, 8
+    srv = H.Server(budget_bytes=64 * MB, max_slots=32)
+    srv.submit(_job(n, nbins, 2, **options))
+    srv.run(10)
+    before = _free()
+    jobs = [srv.submit(_job(n, nbins, 4, **options)) for _ in range(12)]
+    most, left = 0, 1
+    while left:
+        left = srv.tick(1)
+        most = max(most, before - _free())
+        print(f"{left} jobs left, {most / MB:.1f} MiB at most", flush=True)
+    assert most <= 72 * MB
+    assert all(r.status == 0 for r in srv.poll()) and len(jobs) == 12
+    srv.close()
