@@ -1018,7 +1018,7 @@ hm_status Batch::add_slots(const std::vector<RunBunch> &specs, std::vector<int32
         d.logF = ilog2(d.F);
         d.nA = (int32_t)((nb + Bk - 1) / Bk);
         d.nJ = (int32_t)((nw + Bk - 1) / Bk);
-        const int hwin = hist_window(nb, d.npairs, d.pairs_per_tile, ctx_->lds_max);
+        const int hwin = hist_window(nb, d.ntiles, d.npairs, d.pairs_per_tile, ctx_->lds_max);
         if (hwin >= 0) {
             d.flags |= F_GHIST;
             d.hwin = hwin;

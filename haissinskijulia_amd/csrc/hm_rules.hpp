@@ -32,26 +32,38 @@ inline int64_t pairs_per_tile_for(int64_t npairs, int threads, int32_t tile_pair
 // sigma (one particle in 200 outside) and leave 8000 entries for the window of
 // P, which the kick reads; 32768, 40960 and 57344 bins: 0.084, 0.085 and 0.098
 // ms against 0.089 at 65536 bins, 0.105, 0.105 and 0.111 at 131072, but 0.173,
-// 0.153 and 0.138 against 0.145 at 262144.  Slabs cost a launch of 8 us a turn
-// (25 MB written and read), so 32-bit counts of all bins stay as long as they
-// leave kHistMinWin entries of P: 1e7 particles, 34000 bins 95 + 35 us of pass
-// and bin phase, 36000 bins by the window 80 + 43, 40000 bins 118 + 35 before and
-// 81 + 43 after.  Tiles of more than kHistRunPairs pairs cannot use 16 bits;
-// kHistMaxPairs bounds the slabs of one bunch to a few hundred MB.
+// 0.153 and 0.138 against 0.145 at 262144.  Tiles of more than kHistRunPairs pairs
+// cannot use 16 bits; kHistMaxPairs bounds the slabs of one bunch to a few
+// hundred MB.
 constexpr int kHistWin = 49152;
 constexpr int kHistRunPairs = 32767;
 constexpr int64_t kHistMaxPairs = 1 << 26;
 constexpr int kHistMinWin = 3072;
 
-// Where a bunch of nb bins counts its histogram: -1 in LDS, 0 in global memory, else
-// the bins of its window in LDS.  The whole histogram in LDS only with room for a
-// window of at least two entries of P beside it (the all-flags pass relies on
-// that), or, where a window of 16-bit counts can take its place (a tile's counts
-// fit them), of kHistMinWin.
-inline int hist_window(int64_t nb, int64_t npairs, int64_t ppt, int lds_max) {
-    const bool window = ppt <= kHistRunPairs && npairs <= kHistMaxPairs;
+// Where a bunch of nb bins counts its histogram: -1 in LDS by 32 bits, 0 in global
+// memory, else the bins of its window in LDS by 16 bits.  32 bits need room for two
+// entries of P beside them (the all-flags pass relies on that): 40700 bins.  From
+// 34561 on, where they leave less than kHistMinWin entries of P, the window is an
+// alternative: its pass gathers less of P from global memory, for a launch and
+// slabs that grow to 25 MB (one per workgroup) between 1e4 and 5e5 particles and no
+// further.  A turn by 32 bits and by the window, the energy update on (reference
+// lattice, off), in us:
+//   particles     34600 bins                 38000 bins                 40600 bins
+//   2e4       46.8, 45.6  (37.4, 38.0)   47.8, 45.8  (38.1, 38.5)   48.4, 46.4  (38.6, 38.6)
+//   5e4       46.8, 46.7  (37.2, 39.0)   47.8, 47.4  (38.0, 39.3)   48.7, 47.9  (38.5, 39.6)
+//   1e5       47.0, 49.5  (37.4, 41.6)   48.0, 50.2  (38.2, 42.3)   48.9, 51.4  (38.6, 43.1)
+//   1e6       57.4, 64.1  (46.3, 55.0)   60.1, 64.7  (47.1, 55.0)   60.6, 65.0  (48.0, 54.9)
+//   2e6       64.7, 68.7  (53.9, 58.0)   68.7, 69.8  (55.5, 58.6)   69.9, 69.5  (55.7, 59.6)
+//   2.5e6     76.5, 80.3  (63.2, 68.4)   82.3, 81.2  (66.3, 68.8)   86.3, 81.0  (70.3, 69.1)
+//   3e6       78.8, 81.3  (65.5, 69.8)   85.7, 82.4  (70.2, 70.1)   90.3, 82.7  (74.3, 70.2)
+//   1e7        138,  123  ( 113,  104)    155,  125  ( 130,  107)    164,  125  ( 136,  106)
+constexpr int64_t kHistMinPairs = 1250000;   // the window from here on,
+constexpr int kHistFewTiles = 24;            // and up to here
+inline int hist_window(int64_t nb, int64_t ntiles, int64_t npairs, int64_t ppt, int lds_max) {
+    const bool can = ppt <= kHistRunPairs && npairs <= kHistMaxPairs;
+    const bool window = can && (npairs >= kHistMinPairs || ntiles <= kHistFewTiles);
     if (4 * nb + 8 * (window ? kHistMinWin : 2) <= (int64_t)lds_max - 1024) return -1;
-    return window ? (int)std::min<int64_t>(nb, kHistWin) & ~1 : 0;
+    return can ? (int)std::min<int64_t>(nb, kHistWin) & ~1 : 0;
 }
 // The most slabs the windowed histogram of a bunch of ntiles tiles of ppt pairs
 // can fill, alone or in any batch, on a device of cus CUs.  The pass has at most

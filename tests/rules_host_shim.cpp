@@ -3,4 +3,8 @@
 
 extern "C" {
 int64_t t_max_slabs(int64_t ntiles, int64_t ppt, int cus) { return hm::max_slabs(ntiles, ppt, cus); }
+int t_hist_window(int64_t nb, int64_t ntiles, int64_t npairs, int64_t ppt, int lds) {
+    return hm::hist_window(nb, ntiles, npairs, ppt, lds);
+}
+int64_t t_pairs_per_tile(int64_t npairs, int tile_pairs) { return hm::pairs_per_tile_for(npairs, 1024, tile_pairs); }
 }

@@ -19,6 +19,9 @@ def rules(tmp_path_factory):
     L = C.CDLL(str(out))
     L.t_max_slabs.restype = C.c_int64
     L.t_max_slabs.argtypes = [C.c_int64, C.c_int64, C.c_int]
+    L.t_hist_window.argtypes = [C.c_int64] * 4 + [C.c_int]
+    L.t_pairs_per_tile.restype = C.c_int64
+    L.t_pairs_per_tile.argtypes = [C.c_int64, C.c_int]
     return L
 
 
@@ -44,3 +47,20 @@ def test_max_slabs_of_a_lone_bunch_is_near_what_it_fills(rules):
     assert rules.t_max_slabs(128, 1024, CUS) == 256
     assert rules.t_max_slabs(489, 1024, CUS) == 263      # 1e6 particles
     assert rules.t_max_slabs(977, 5120, CUS) == 376      # 1e7
+
+
+@pytest.mark.parametrize("n,tile_pairs,windowed", [
+    (1, 0, True), (49_152, 0, True), (49_153, 0, False), (1_000_000, 0, False), (2_499_998, 0, False),
+    (2_499_999, 0, True), (10_000_000, 0, True), (50_001, 31, True), (50_001, 32, False), (10_000_000, 32, False)])
+def test_histogram_form(rules, n, tile_pairs, windowed):
+    """Up to 34560 bins 32-bit counts of all bins; from 40701 on, which they do not
+    fit, the window; in between the window where it is the faster one."""
+    npairs = (n + 1) // 2
+    ppt = rules.t_pairs_per_tile(npairs, tile_pairs)
+
+    def form(nb):
+        return rules.t_hist_window(nb, -(-npairs // ppt), npairs, ppt, 163840)
+    assert form(34560) == -1
+    assert [form(nb) for nb in (34561, 40700)] == ([34560, 40700] if windowed else [-1, -1])
+    can = ppt <= 32767
+    assert [form(nb) for nb in (40701, 49152, 131073)] == ([40700, 49152, 49152] if can else [0, 0, 0])
