@@ -603,6 +603,17 @@ hm_status Batch::build_tables() {
     for (size_t i = 0; i < rb_.size(); ++i)
         if (used_[i] && rb_[i].active) zbytes += 8 * rb_[i].d.n;
     keep_z_ = zbytes > kKeepMinBytes && zbytes <= kKeepMaxBytes;
+    int64_t through = 0;   // bytes that would go through the caches with the windowed bunches
+    for (size_t i = 0; i < rb_.size(); ++i)
+        if (used_[i] && rb_[i].active) {
+            const BunchDev &d = rb_[i].d;
+            through += d.hwin > 0 ? cached_bytes(d.n) : (keep_z_ ? 8 * d.n : 0);
+        }
+    for (size_t i = 0; i < rb_.size(); ++i) {
+        BunchDev &d = rb_[i].d;
+        d.flags &= ~F_CACHED;
+        if (used_[i] && rb_[i].active && d.hwin > 0 && through <= kCachedBytes) d.flags |= F_CACHED;
+    }
     ntiles_ = (int)tiles.size();
     nred_ = (int)red.size() / 2;
     nlist_ = (int)list.size();

@@ -632,17 +632,8 @@ __device__ __forceinline__ double gather_interp(const g_f64x2 *q, double w) {
     return v.x * (1.0 - w) + v.y * w;
 }
 
-// The particles of a bunch with a windowed histogram are read and written
-// through the caches, by the pass and by the interpolation sums, where they fit
-// the 256 MB of the last one: many of its particles gather from the pair table,
-// and those gathers wait behind the streams (131072 bins, pass of 1e7 particles:
-// 104 -> 75 us, 4e6: 51 -> 39, 1.3e7: 139 -> 113, 2e7: 205 -> 212; one of the
-// two streaming past the caches undoes it).  With 32-bit LDS counts the same
-// costs 2 us up to 4e6 particles.
-constexpr int64_t kCachedBytes = 224ll << 20;
-__device__ __forceinline__ bool cached(const BunchDev &B) {
-    return (B.flags & F_GHIST) && B.hwin > 0 && 16 * B.n <= kCachedBytes;
-}
+// whether the bunch's particles are read and written through the caches
+__device__ __forceinline__ bool cached(const BunchDev &B) { return (B.flags & F_CACHED) != 0; }
 
 __device__ __forceinline__ uint8_t *pass_lds() {
     extern __shared__ __align__(16) uint8_t s_lds[];

@@ -77,4 +77,17 @@ inline int64_t max_slabs(int64_t ntiles, int64_t ppt, int cus) {
     return 2 * ntiles <= cus ? 2 * ntiles : runs;
 }
 
+// The particles of bunches with a windowed histogram are read and written
+// through the caches, by the pass and by the interpolation sums, where all of them
+// and 10 MB of tables a bunch fit the 256 MB of the last one: many particles
+// gather from the pair table, and those gathers wait behind the streams (131072
+// bins, pass of 1e7 particles: 104 -> 75 us, 4e6: 51 -> 39, 1.3e7: 139 -> 113, 2e7:
+// 205 -> 212; one of the two streaming past the caches undoes it).  A turn through
+// them and past them, us: 65536 bins, 1.3e7 particles (218 MB) 156, 173; two bunches
+// of 6e6 (212 MB) 152, 166, of 7e6 (244 MB) 190, 180, of 1e7 265, 242; three of 4e6
+// (222 MB) 156, 172; six of 2e6 (252 MB) 203, 194; ten of 1e6 (260 MB) 217, 205; with
+// 36000 and 262144 bins the line lies at the same particles.
+constexpr int64_t kCachedBytes = 224ll << 20;
+inline int64_t cached_bytes(int64_t n) { return 16 * n + 10000000; }
+
 }  // namespace hm

@@ -44,6 +44,7 @@ enum BunchFlags : uint32_t {
     F_GHIST = 128u,    // too many bins for a histogram in LDS: hwin of them there, or none
     F_LAG = 256u,      // wake table by lag behind the source: bin k feels bins k+j (causal)
     F_CIC = 512u,      // the pass deposits the interpolation weights of the new z (cic)
+    F_CACHED = 1024u,  // z and dE of a windowed histogram's bunch go through the caches
 };
 
 // Cloud-in-cell deposit (F_CIC).  The E0 update needs sum_i interp(P_t, z_i)

@@ -7,4 +7,9 @@ int t_hist_window(int64_t nb, int64_t ntiles, int64_t npairs, int64_t ppt, int l
     return hm::hist_window(nb, ntiles, npairs, ppt, lds);
 }
 int64_t t_pairs_per_tile(int64_t npairs, int tile_pairs) { return hm::pairs_per_tile_for(npairs, 1024, tile_pairs); }
+int t_cached(const int64_t *n, int count) {
+    int64_t bytes = 0;
+    for (int i = 0; i < count; ++i) bytes += hm::cached_bytes(n[i]);
+    return bytes <= hm::kCachedBytes;
+}
 }

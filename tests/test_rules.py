@@ -64,3 +64,12 @@ def test_histogram_form(rules, n, tile_pairs, windowed):
     assert [form(nb) for nb in (34561, 40700)] == ([34560, 40700] if windowed else [-1, -1])
     can = ppt <= 32767
     assert [form(nb) for nb in (40701, 49152, 131073)] == ([40700, 49152, 49152] if can else [0, 0, 0])
+
+
+def test_cached_particles_fit_the_last_cache_together(rules):
+    def cached(*n):
+        return bool(rules.t_cached((C.c_int64 * len(n))(*n), len(n)))
+    assert cached(10_000_000) and cached(13_000_000) and not cached(15_000_000)
+    assert cached(6_000_000, 6_000_000) and not cached(7_000_000, 7_000_000)
+    assert not cached(10_000_000, 10_000_000)
+    assert cached(*[1_000_000] * 5) and not cached(*[1_000_000] * 10)
