@@ -495,11 +495,39 @@ hm_status Batch::free_turns(int64_t turns) {
     return HM_OK;
 }
 
+// the pass's LDS window of P: what the histogram (and deposit) leave of the LDS
+static void set_pass_window(BunchDev &d, int lds_max) {
+    const int64_t cap = ((int64_t)lds_max - 1024 - (int64_t)pass_hist_bytes(d) - (int64_t)pass_cic_bytes(d)) / 8;
+    d.win = cap >= 2 ? (int32_t)std::min<int64_t>(d.nbins, cap) : 0;
+    d.cic_off = (d.flags & F_CIC) ? pass_hist_bytes(d) + ((d.win * 8 + 15) & ~15) : 0;
+}
+
+// Where the active bunches with more than 34560 bins count: a window, all bins by
+// 32 bits, or global memory.
+void Batch::place_histograms() {
+    int64_t pairs = 0, tiles = 0;
+    for (size_t i = 0; i < rb_.size(); ++i)
+        if (used_[i] && rb_[i].active && (rb_[i].d.flags & F_WAKE) && rb_[i].hwin > 0) {
+            pairs += rb_[i].d.npairs;
+            tiles += rb_[i].d.ntiles;
+        }
+    for (size_t i = 0; i < rb_.size(); ++i) {
+        BunchDev &d = rb_[i].d;
+        if (!used_[i] || !rb_[i].active || !(d.flags & F_WAKE) || rb_[i].hwin < 0) continue;
+        const bool fits = hist_fits(d.nbins, ctx_->lds_max);
+        const bool window = rb_[i].hwin > 0 && (!fits || hist_window_pays(pairs, tiles));
+        d.hwin = window ? rb_[i].hwin : 0;
+        d.flags = window || !fits ? d.flags | F_GHIST : d.flags & ~F_GHIST;
+        set_pass_window(d, ctx_->lds_max);
+    }
+}
+
 hm_status Batch::build_tables() {
     free_only_ = !timing_;   // timing asks for one launch of the pass per turn
     for (size_t i = 0; i < rb_.size(); ++i)
         if (used_[i] && rb_[i].active && (rb_[i].d.flags & (F_WAKE | F_E0))) free_only_ = false;
     if (free_only_) return build_free_tables();
+    place_histograms();
     std::vector<int32_t> tiles, conv[kConvKinds], red, list, bw, b64, slab;
     pass_lds_ = 0;
     final_whole_ = true;
@@ -1029,11 +1057,8 @@ hm_status Batch::add_slots(const std::vector<RunBunch> &specs, std::vector<int32
         d.logF = ilog2(d.F);
         d.nA = (int32_t)((nb + Bk - 1) / Bk);
         d.nJ = (int32_t)((nw + Bk - 1) / Bk);
-        const int hwin = hist_window(nb, d.ntiles, d.npairs, d.pairs_per_tile, ctx_->lds_max);
-        if (hwin >= 0) {
-            d.flags |= F_GHIST;
-            d.hwin = hwin;
-        }
+        q.hwin = hist_window(nb, d.npairs, d.pairs_per_tile, ctx_->lds_max);
+        if (q.hwin >= 0 && !hist_fits(nb, ctx_->lds_max)) d.flags |= F_GHIST;
         // With update_E0 the pass deposits the interpolation weights of its
         // post-drift z (cloud in cell) where its LDS holds the counters beside
         // the histogram and the whole table of P, instead of the interpolation
@@ -1045,11 +1070,8 @@ hm_status Batch::add_slots(const std::vector<RunBunch> &specs, std::vector<int32
             (int64_t)pass_hist_bytes(d) + 8 * nb + cic_bytes((int)nb) <=
                 (int64_t)ctx_->lds_max - 1024)
             d.flags |= F_CIC;
-        {   // the pass's LDS window of P: what the histogram (and deposit) leave of the LDS
-            const int64_t cap = ((int64_t)ctx_->lds_max - 1024 - (int64_t)pass_hist_bytes(d) -
-                                 (int64_t)pass_cic_bytes(d)) / 8;
-            d.win = cap >= 2 ? (int32_t)std::min<int64_t>(nb, cap) : 0;
-            d.cic_off = (d.flags & F_CIC) ? pass_hist_bytes(d) + ((d.win * 8 + 15) & ~15) : 0;
+        {
+            set_pass_window(d, ctx_->lds_max);
             // the interpolation sums' window: the whole table when it fits
             d.iwin = (int32_t)std::min<int64_t>(nb, ((int64_t)ctx_->lds_max - 1024) / 8);
         }
@@ -1096,15 +1118,15 @@ hm_status Batch::add_slots(const std::vector<RunBunch> &specs, std::vector<int32
         HM_TRY(twiddles(ctx_, d.F, &tw));
         d.tw = tw;
     }
-    // The slabs, last: a bunch they do not fit beside counts in global memory
-    // (the same counts), as a histogram without a window does.
+    // The slabs, last: a bunch they do not fit beside goes without a window (the
+    // same counts).
     for (int32_t i : fresh) {
-        BunchDev &d = rb_[(size_t)i].d;
-        if (d.hwin == 0) continue;
-        DevBuf<uint32_t> &slabs = rb_[(size_t)i].b->w.slabs;
-        if (slabs.ensure((size_t)max_slabs(d.ntiles, d.pairs_per_tile, ctx_->cus) * (size_t)(d.hwin / 2)) != HM_OK)
-            d.hwin = 0;
-        d.slabs = slabs.p;
+        RunBunch &q = rb_[(size_t)i];
+        if (q.hwin <= 0) continue;
+        DevBuf<uint32_t> &slabs = q.b->w.slabs;
+        if (slabs.ensure((size_t)max_slabs(q.d.ntiles, q.d.pairs_per_tile, ctx_->cus) * (size_t)(q.hwin / 2)) != HM_OK)
+            q.hwin = 0;
+        q.d.slabs = slabs.p;
     }
     HM_TRY(clears.flush());
     {   // the callers' tables, the descriptors and the new bunches' list: one round

@@ -180,6 +180,7 @@ struct RunBunch {
     int64_t n_turns = 0;      // turns to run
     int64_t turns_done = 0;
     BunchDev d{};
+    int hwin = -1;            // what hist_window allows (d.hwin: what build_tables chose)
     bool active = false;      // still turning
     bool finished = false;    // epilogue done, results valid
     bool fail_setup = false;  // test hook: the set-up fails by request after the slot is taken
@@ -224,6 +225,7 @@ class Batch {
     hm_status add_slots(const std::vector<RunBunch> &specs, std::vector<int32_t> &fresh);
     hm_status build_tables();
     hm_status build_free_tables();
+    void place_histograms();
     hm_status upload_descriptors();
     hm_status stage_descriptors();
     hm_status run_subset_moments(const std::vector<int32_t> &which, int mode);

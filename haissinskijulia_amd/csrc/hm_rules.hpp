@@ -40,14 +40,23 @@ constexpr int kHistRunPairs = 32767;
 constexpr int64_t kHistMaxPairs = 1 << 26;
 constexpr int kHistMinWin = 3072;
 
-// Where a bunch of nb bins counts its histogram: -1 in LDS by 32 bits, 0 in global
-// memory, else the bins of its window in LDS by 16 bits.  32 bits need room for two
-// entries of P beside them (the all-flags pass relies on that): 40700 bins.  From
-// 34561 on, where they leave less than kHistMinWin entries of P, the window is an
-// alternative: its pass gathers less of P from global memory, for a launch and
-// slabs that grow to 25 MB (one per workgroup) between 1e4 and 5e5 particles and no
-// further.  A turn by 32 bits and by the window, the energy update on (reference
-// lattice, off), in us:
+// 32-bit counts of nb bins in LDS, beside two entries of P at least (the
+// all-flags pass relies on that): up to 40700 bins.
+inline bool hist_fits(int64_t nb, int lds_max) { return 4 * nb + 16 <= (int64_t)lds_max - 1024; }
+
+// The bins of a bunch's window, 0 where it cannot have one, or -1 where it needs
+// none: 32-bit counts leave kHistMinWin entries of P (up to 34560 bins).
+inline int hist_window(int64_t nb, int64_t npairs, int64_t ppt, int lds_max) {
+    if (hist_fits(nb + 2 * kHistMinWin - 4, lds_max)) return -1;
+    return ppt <= kHistRunPairs && npairs <= kHistMaxPairs ? (int)std::min<int64_t>(nb, kHistWin) & ~1 : 0;
+}
+
+// Whether the bunches of a launch that can have either, 34561 to 40700 bins, take
+// the window, from the pairs and tiles of all its windowed bunches.  Its pass
+// gathers less of P from global memory, for a launch and slabs that grow to 25 MB
+// (one per workgroup) between 1e4 and 5e5 particles and no further.  The counts,
+// and with them the results, are the same.  A turn by 32 bits and by the window, the
+// energy update on (reference lattice, off), in us:
 //   particles     34600 bins                 38000 bins                 40600 bins
 //   2e4       46.8, 45.6  (37.4, 38.0)   47.8, 45.8  (38.1, 38.5)   48.4, 46.4  (38.6, 38.6)
 //   5e4       46.8, 46.7  (37.2, 39.0)   47.8, 47.4  (38.0, 39.3)   48.7, 47.9  (38.5, 39.6)
@@ -57,13 +66,13 @@ constexpr int kHistMinWin = 3072;
 //   2.5e6     76.5, 80.3  (63.2, 68.4)   82.3, 81.2  (66.3, 68.8)   86.3, 81.0  (70.3, 69.1)
 //   3e6       78.8, 81.3  (65.5, 69.8)   85.7, 82.4  (70.2, 70.1)   90.3, 82.7  (74.3, 70.2)
 //   1e7        138,  123  ( 113,  104)    155,  125  ( 130,  107)    164,  125  ( 136,  106)
+// Several bunches at 36000 bins: two of 1e5 58, 67 (46, 57), sixteen of 1e5 120, 123
+// (100, 107), two of 1e6 77, 80 (62, 67), two of 2e6 94, 86 (72, 70), five of 1e6 114,
+// 100 (92, 82), twenty of 5e5 215, 200 (174, 170), 1.2e7 and 1e6 202, 157 (171, 133).
 constexpr int64_t kHistMinPairs = 1250000;   // the window from here on,
-constexpr int kHistFewTiles = 24;            // and up to here
-inline int hist_window(int64_t nb, int64_t ntiles, int64_t npairs, int64_t ppt, int lds_max) {
-    const bool can = ppt <= kHistRunPairs && npairs <= kHistMaxPairs;
-    const bool window = can && (npairs >= kHistMinPairs || ntiles <= kHistFewTiles);
-    if (4 * nb + 8 * (window ? kHistMinWin : 2) <= (int64_t)lds_max - 1024) return -1;
-    return can ? (int)std::min<int64_t>(nb, kHistWin) & ~1 : 0;
+constexpr int64_t kHistFewTiles = 24;        // and up to here
+inline bool hist_window_pays(int64_t pairs, int64_t tiles) {
+    return pairs >= kHistMinPairs || tiles <= kHistFewTiles;
 }
 // The most slabs the windowed histogram of a bunch of ntiles tiles of ppt pairs
 // can fill, alone or in any batch, on a device of cus CUs.  The pass has at most

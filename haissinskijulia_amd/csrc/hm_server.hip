@@ -45,7 +45,7 @@ size_t job_bytes(const hm_ctx *ctx, const hm_job &j) {
         // P, its pairs, lambda, the wake; three tables of spectra; the counters
         bytes += 40 * nb + 96 * (nb + block) + Work::hist_bytes((int)nb);
         if (j.params.update_E0 && cic_bytes((int)nb) <= ctx->lds_max) bytes += cic_words((int)nb) * 8;
-        const int hwin = hist_window(j.nbins, tiles, npairs, ppt, ctx->lds_max);
+        const int hwin = hist_window(j.nbins, npairs, ppt, ctx->lds_max);
         if (hwin > 0) bytes += (size_t)max_slabs(tiles, ppt, ctx->cus) * (size_t)hwin * 2;
     }
     return bytes + (size_t)(1 << 16) + 2 * (size_t)kMaxFFT * 16;

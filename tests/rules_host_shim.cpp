@@ -3,8 +3,12 @@
 
 extern "C" {
 int64_t t_max_slabs(int64_t ntiles, int64_t ppt, int cus) { return hm::max_slabs(ntiles, ppt, cus); }
-int t_hist_window(int64_t nb, int64_t ntiles, int64_t npairs, int64_t ppt, int lds) {
-    return hm::hist_window(nb, ntiles, npairs, ppt, lds);
+// the form of a lone bunch: -1 32-bit counts, 0 global memory, else the window
+int t_hist_form(int64_t nb, int64_t ntiles, int64_t npairs, int64_t ppt, int lds) {
+    const int w = hm::hist_window(nb, npairs, ppt, lds);
+    if (w < 0) return -1;
+    if (w > 0 && (!hm::hist_fits(nb, lds) || hm::hist_window_pays(npairs, ntiles))) return w;
+    return hm::hist_fits(nb, lds) ? -1 : 0;
 }
 int64_t t_pairs_per_tile(int64_t npairs, int tile_pairs) { return hm::pairs_per_tile_for(npairs, 1024, tile_pairs); }
 int t_cached(const int64_t *n, int count) {

@@ -19,7 +19,7 @@ def rules(tmp_path_factory):
     L = C.CDLL(str(out))
     L.t_max_slabs.restype = C.c_int64
     L.t_max_slabs.argtypes = [C.c_int64, C.c_int64, C.c_int]
-    L.t_hist_window.argtypes = [C.c_int64] * 4 + [C.c_int]
+    L.t_hist_form.argtypes = [C.c_int64] * 4 + [C.c_int]
     L.t_pairs_per_tile.restype = C.c_int64
     L.t_pairs_per_tile.argtypes = [C.c_int64, C.c_int]
     return L
@@ -59,7 +59,7 @@ def test_histogram_form(rules, n, tile_pairs, windowed):
     ppt = rules.t_pairs_per_tile(npairs, tile_pairs)
 
     def form(nb):
-        return rules.t_hist_window(nb, -(-npairs // ppt), npairs, ppt, 163840)
+        return rules.t_hist_form(nb, -(-npairs // ppt), npairs, ppt, 163840)
     assert form(34560) == -1
     assert [form(nb) for nb in (34561, 40700)] == ([34560, 40700] if windowed else [-1, -1])
     can = ppt <= 32767
