@@ -630,7 +630,7 @@ hm_status Batch::build_tables() {
     int64_t zbytes = 0;
     for (size_t i = 0; i < rb_.size(); ++i)
         if (used_[i] && rb_[i].active) zbytes += 8 * rb_[i].d.n;
-    keep_z_ = zbytes > kKeepMinBytes && zbytes <= kKeepMaxBytes;
+    keep_z_ = keeps_z(zbytes, any_wake_e0_);
     int64_t through = 0;   // bytes that would go through the caches with the windowed bunches
     for (size_t i = 0; i < rb_.size(); ++i)
         if (used_[i] && rb_[i].active) {

@@ -253,13 +253,7 @@ class Batch {
     DevBuf<RunDev> d_runs_;
     DevBuf<int32_t> d_ranges_;
     int pass_grid_ = 0, pass_slices_ = 1, interp_grid_ = 0;
-    // z of the active bunches goes through the caches, dE past them, where z
-    // fits the 256 MB of the last one and is not small: the pass and the
-    // interpolation sums read it again.  28 bunches, 176 MB of z: 188 -> 170 us a
-    // turn; one bunch of 1e7 particles (80 MB) and 8192 bins 119 -> 116, of 2.8e7
-    // (224 MB) 257 -> 239; of 4e7 346 -> 358; of 4e6 (32 MB) 69 -> 71, where z
-    // drives the bin phase's tables from the caches nearer to the CUs.
-    static constexpr int64_t kKeepMinBytes = 76ll << 20, kKeepMaxBytes = 224ll << 20;
+    // z of the active bunches goes through the caches, dE past them (keeps_z)
     bool keep_z_ = false;
     bool interp_deep_ = false;   // one interpolation workgroup per CU: deeper rings
     // no active bunch needs a sum over its particles between turns: the items

@@ -99,4 +99,23 @@ inline int64_t max_slabs(int64_t ntiles, int64_t ppt, int cus) {
 constexpr int64_t kCachedBytes = 224ll << 20;
 inline int64_t cached_bytes(int64_t n) { return 16 * n + 10000000; }
 
+// Whether z of the active bunches (zbytes in all) goes through the caches, dE past
+// them: where z fits the 256 MB of the last one and is not small, the pass and the
+// interpolation sums (interp: some bunch has them) find it there again.  28
+// bunches, 176 MB of z: 188 -> 170 us a turn; one bunch of 2.8e7 particles (224 MB)
+// and 8192 bins 257 -> 239; of 4e7 346 -> 358; of 4e6 (32 MB) 62 -> 66, where z
+// drives the bin phase's tables from the caches nearer to the CUs.  Where that
+// turns, one bunch, past the caches and through them (three runs of each, 0.5 us):
+//   particles     8.5e6         9e6           9.5e6         1e7           1.04e7        1.2e7
+//   1024 bins     76.6, 78.3    78.0, 78.7    80.4, 81.1    82.7, 81.8    83.7, 83.6    92.5, 88.0
+//   4096 bins     84.4, 87.2    85.5, 88.2    87.8, 89.9    90.8, 91.0    92.5, 93.2    101,  97.4
+//   8192 bins     102,  105     105,  106     107,  105     111,  109     112,  110     122,  117
+//   16384 bins    103,  107     106,  107     110,  108     112,  111     113,  112     126,  119
+//   8192, E0 off  82.4, 86.7    83.8, 87.2    86.4, 87.6    88.2, 88.9    88.6, 89.5    99.7, 99.8
+// so from 75 MB with the sums (8192 and 16384 bins), from 84 MB without.
+constexpr int64_t kKeepMinInterp = 75000000, kKeepMin = 84000000, kKeepMax = 224ll << 20;
+inline bool keeps_z(int64_t zbytes, bool interp) {
+    return zbytes > (interp ? kKeepMinInterp : kKeepMin) && zbytes <= kKeepMax;
+}
+
 }  // namespace hm

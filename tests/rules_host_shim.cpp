@@ -16,4 +16,5 @@ int t_cached(const int64_t *n, int count) {
     for (int i = 0; i < count; ++i) bytes += hm::cached_bytes(n[i]);
     return bytes <= hm::kCachedBytes;
 }
+int t_keeps_z(int64_t zbytes, int interp) { return hm::keeps_z(zbytes, interp != 0); }
 }

@@ -19,6 +19,7 @@ def rules(tmp_path_factory):
     L = C.CDLL(str(out))
     L.t_max_slabs.restype = C.c_int64
     L.t_max_slabs.argtypes = [C.c_int64, C.c_int64, C.c_int]
+    L.t_keeps_z.argtypes = [C.c_int64, C.c_int]
     L.t_hist_form.argtypes = [C.c_int64] * 4 + [C.c_int]
     L.t_pairs_per_tile.restype = C.c_int64
     L.t_pairs_per_tile.argtypes = [C.c_int64, C.c_int]
@@ -73,3 +74,9 @@ def test_cached_particles_fit_the_last_cache_together(rules):
     assert cached(6_000_000, 6_000_000) and not cached(7_000_000, 7_000_000)
     assert not cached(10_000_000, 10_000_000)
     assert cached(*[1_000_000] * 5) and not cached(*[1_000_000] * 10)
+
+
+@pytest.mark.parametrize("n,with_sums,without", [(9_000_000, 0, 0), (9_500_000, 1, 0), (10_400_000, 1, 0),
+                                                 (11_000_000, 1, 1), (29_000_000, 1, 1), (30_000_000, 0, 0)])
+def test_where_z_goes_through_the_caches(rules, n, with_sums, without):
+    assert (rules.t_keeps_z(8 * n, 1), rules.t_keeps_z(8 * n, 0)) == (with_sums, without)
