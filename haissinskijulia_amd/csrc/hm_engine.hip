@@ -485,10 +485,9 @@ hm_status Batch::build_free_tables() {
     return HM_OK;
 }
 
-// turns of the free bunches, at most about 4e9 pair-turns (40 ms) per launch
+// turns of the free bunches, several launches of up to about 40 ms each
 hm_status Batch::free_turns(int64_t turns) {
-    const int64_t most = std::min<int64_t>(
-        1 << 20, std::max<int64_t>(1, (int64_t)4e9 / std::max<int64_t>(1, free_pairs_)));
+    const int64_t most = free_turns_per_launch(free_pairs_);
     for (int64_t t = 0; t < turns; t += most)
         HIP_TRY(launch_free_turns(d_bd_.p, d_free_.p, nfree_, d_list_.p, nlist_,
                                   (int)std::min(most, turns - t), ctx_->stream));

@@ -118,4 +118,13 @@ inline bool keeps_z(int64_t zbytes, bool interp) {
     return zbytes > (interp ? kKeepMinInterp : kKeepMin) && zbytes <= kKeepMax;
 }
 
+// Turns of one launch of k_free_turns over `pairs` pairs, for about 40 ms: 4e9
+// pair-turns fill the device (27 ms for 1e7 particles), and below 8e4 pairs a
+// turn takes the 0.8 us of a thread's own chain however few there are.  Bounded
+// by the pair-turns alone, a launch of a few thousand particles ran for 2^20
+// turns, 0.8 s.
+inline int64_t free_turns_per_launch(int64_t pairs) {
+    return std::min<int64_t>(50000, std::max<int64_t>(1, (int64_t)4e9 / std::max<int64_t>(1, pairs)));
+}
+
 }  // namespace hm

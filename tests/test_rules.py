@@ -19,6 +19,8 @@ def rules(tmp_path_factory):
     L = C.CDLL(str(out))
     L.t_max_slabs.restype = C.c_int64
     L.t_max_slabs.argtypes = [C.c_int64, C.c_int64, C.c_int]
+    L.t_free_turns.restype = C.c_int64
+    L.t_free_turns.argtypes = [C.c_int64]
     L.t_keeps_z.argtypes = [C.c_int64, C.c_int]
     L.t_hist_form.argtypes = [C.c_int64] * 4 + [C.c_int]
     L.t_pairs_per_tile.restype = C.c_int64
@@ -80,3 +82,11 @@ def test_cached_particles_fit_the_last_cache_together(rules):
                                                  (11_000_000, 1, 1), (29_000_000, 1, 1), (30_000_000, 0, 0)])
 def test_where_z_goes_through_the_caches(rules, n, with_sums, without):
     assert (rules.t_keeps_z(8 * n, 1), rules.t_keeps_z(8 * n, 0)) == (with_sums, without)
+
+
+@pytest.mark.parametrize("pairs", [0, 1, 500, 50_000, 500_000, 5_000_000, 50_000_000, 2 ** 31])
+def test_free_turns_of_a_launch_stay_near_40_ms(rules, pairs):
+    """0.8 us a turn for a thread's chain, or 6.8e-12 s per pair-turn of a full device."""
+    turns = rules.t_free_turns(pairs)
+    assert turns >= 1
+    assert turns == 1 or turns * max(0.8e-6, 6.8e-12 * pairs) <= 0.045
