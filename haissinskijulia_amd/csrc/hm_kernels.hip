@@ -20,10 +20,12 @@
 //                 evolution.jl:404-435 needs before the next turn.
 //   k_finalize    E0 update and the scalars of the next turn.
 //
-// All floating-point work is FP64.  Multiplies and adds are never contracted
-// (-ffp-contract=off) except inside the elementary functions of hm_math.hpp;
-// divides by per-turn constants are multiplies by their reciprocals.  Sums
-// are reduced in a fixed order, so a run is bitwise reproducible.
+// All floating-point work is FP64.  Multiplies and adds of the per-particle path
+// are never contracted (-ffp-contract=off); fused ones are written out in the
+// elementary functions (hm_math.hpp, bm_radius) and in steps that are exact or
+// round once by them (the uniforms, the deposit's weights, the bin centres).
+// Divides by per-turn constants are multiplies by their reciprocals.  Sums are
+// reduced in a fixed order, so a run is bitwise reproducible.
 #include <hip/hip_runtime.h>
 #include <math.h>
 
@@ -697,7 +699,7 @@ template <int HM, bool CIC>
 __device__ __forceinline__ void bin_and_sum(const PassCtx &c, g_u32 *ghist, int spread, int hlo,
                                             int hwin, g_u32 *n_bad, double z, double (&v)[4]) {
     v[0] += z;
-    v[1] = __builtin_fma(z, z, v[1]);
+    v[1] += z * z;
     // hist_bin with its range test as the branch: in range, u = (z - e0) * inv
     // is >= 0, and its conversion to int (truncation) is floor(u)
     if ((z >= c.e0) & (z <= c.e1)) {
@@ -996,7 +998,7 @@ __device__ __forceinline__ void turn_pass_run(const BunchDev &B, const int32_t *
         }
         if (odd && lt == lt_last && tid == (unsigned)lane && lane == 0) {   // the unit of slot 0
             v[0] += pass_odd()[0];
-            v[1] = __builtin_fma(pass_odd()[0], pass_odd()[0], v[1]);
+            v[1] += pass_odd()[0] * pass_odd()[0];
             v[3] += pass_odd()[2];
             v[2] += pass_odd()[1];
         }
