@@ -105,11 +105,12 @@ struct Work {
     }
 };
 
-// Uploads of small host tables through one pinned staging buffer per
-// context: a round packs its pieces into the buffer, enqueues their copies
-// without waiting and records an event; the next round waits for that event
-// before it packs again.  In an allocation-free call the copies come from the
-// caller's pageable memory and the round ends with a stream synchronisation.
+// Uploads of small host tables through one pinned staging buffer per context: a
+// round packs its pieces behind those of the round before, enqueues their
+// copies without waiting and records an event; the round that reaches the
+// buffer's end waits for that event and starts over.  In an allocation-free
+// call the copies come from the caller's pageable memory and the round ends
+// with a stream synchronisation.
 struct Staging {
     char *host = nullptr;
     size_t cap = 0, used = 0;

@@ -232,11 +232,11 @@ __device__ __forceinline__ double interp_pot(const double *__restrict__ P, doubl
     return P[k] * (1.0 - w) + P[k + 1] * w;
 }
 
-// this turn's half of the two-turn histogram buffer
 // the slots of `turn`'s count of particles that are not binned
 __device__ __forceinline__ uint32_t *unb_of(const BunchDev &B, int64_t turn) {
     return B.unb + (int)(turn & 1) * (kUnbSlots * 16);
 }
+// `turn`'s half of the two-turn histogram buffer
 __device__ __forceinline__ uint32_t *hist_of(const BunchDev &B, int64_t turn) {
     return B.hist + (int)(turn & 1) * hist_half(B.nbins);
 }
@@ -1354,14 +1354,14 @@ __device__ inline void bin_scalars(const BunchDev &B, const double (&t)[4]) {
     bin_scalars_on(B, t, *B.sc);
 }
 
-// The sum over the nred slices of a per-wave partial array by one 1024-thread
-// workgroup, with the arithmetic of slice_sum (256 threads) and slices_done:
-// the workgroup's four groups of four waves take four slices at a time, each
-// group exactly as a 256-thread slice workgroup, and thread 0 adds the slice
-// sums in slice order.  Same bits as the sliced form, no cross-workgroup
-// count (for batches of many bunches, where the bunches fill the device).
-template <int NV>
-__device__ inline void whole_sum(const BunchDev &B, const double *a, double (&t)[NV]) {
+// The sums t over the nred slices of the pass's per-wave sums by one 1024-thread
+// workgroup (k_bin_whole), with the arithmetic of slice_sum (256 threads) and
+// slices_done: the workgroup's four groups of four waves take four slices at a
+// time, each group exactly as a 256-thread slice workgroup, and thread 0 adds
+// the slice sums in slice order.  Same bits as the sliced form, without its count
+// across workgroups.
+__device__ inline void whole_sum(const BunchDev &B, double (&t)[4]) {
+    constexpr int NV = 4;
     __shared__ double s_red[4][NV * 16];
     __shared__ double s_slice[4][NV];
     const int n = B.ntiles * kTileWaves, nred = B.nred;
@@ -1380,20 +1380,16 @@ __device__ inline void whole_sum(const BunchDev &B, const double *a, double (&t)
 #pragma unroll
             for (int k = 0; k < kRedPer; ++k) {
                 const int e = e0 + k * kRedThreads;
-                if constexpr (NV == 4) {
-                    double2 lo = make_double2(0.0, 0.0), hi = make_double2(0.0, 0.0);
-                    if (e < n) {
-                        const g_f64x2 *q = (const g_f64x2 *)a + 2 * (int64_t)e;
-                        lo = ld2(q);
-                        hi = ld2(q + 1);
-                    }
-                    x[k][0] = lo.x;
-                    x[k][1] = lo.y;
-                    x[k][2] = hi.x;
-                    x[k][3] = hi.y;
-                } else {
-                    x[k][0] = e < n ? ((const g_f64 *)a)[e] : 0.0;
+                double2 lo = make_double2(0.0, 0.0), hi = make_double2(0.0, 0.0);
+                if (e < n) {
+                    const g_f64x2 *q = (const g_f64x2 *)B.part + 2 * (int64_t)e;
+                    lo = ld2(q);
+                    hi = ld2(q + 1);
                 }
+                x[k][0] = lo.x;
+                x[k][1] = lo.y;
+                x[k][2] = hi.x;
+                x[k][3] = hi.y;
             }
 #pragma unroll
             for (int k = 0; k < kRedPer; ++k)
@@ -2202,8 +2198,6 @@ __global__ __launch_bounds__(kFinalThreads) void k_init(const BunchDev *__restri
     }
 }
 
-// The E0 update (evolution.jl:419-429) from this turn's sums, and the scalars
-// of the next turn.  One workgroup per slice of the interpolation sums.
 // The E0 update (evolution.jl:419-429) from this turn's sums (psum: the sum of
 // the interpolated potential over the bunch), and the scalars of the next turn.
 // finish_on updates the turn scalars s in place.
@@ -2528,7 +2522,7 @@ __device__ inline void bin_phase_whole(const BunchDev &B) {
     }
     if (fl & (F_WAKE | F_E0)) {
         double t[4];
-        whole_sum<4>(B, B.part, t);   // its barriers also publish the staged LDS
+        whole_sum(B, t);   // its barriers also publish the staged LDS
         if (threadIdx.x == 0) {
             bin_scalars_on(B, t, sc);
             s_nh = sc.n_h;

@@ -41,7 +41,7 @@ enum BunchFlags : uint32_t {
     F_QE = 16u,        // use_excitation
     F_INJ = 32u,       // injected normals instead of Philox
     F_CHARGE = 64u,    // fixed wake current (charge extension / stage entry)
-    F_GHIST = 128u,    // too many bins for a histogram in LDS: hwin of them there, or none
+    F_GHIST = 128u,    // the histogram is not whole in LDS: hwin of its bins are, or none
     F_LAG = 256u,      // wake table by lag behind the source: bin k feels bins k+j (causal)
     F_CIC = 512u,      // the pass deposits the interpolation weights of the new z (cic)
     F_CACHED = 1024u,  // z and dE of a windowed histogram's bunch go through the caches
