@@ -458,11 +458,7 @@ hm_status Batch::build_free_tables() {
     free_pairs_ = 0;
     for (size_t i = 0; i < rb_.size(); ++i)
         if (used_[i] && rb_[i].active) free_pairs_ += rb_[i].d.npairs;
-    // one pair per thread until that fills the SIMDs several times over, then
-    // four in turn (3e6 particles: 6 rounds of waves either way), and at most
-    // about 65536 items
-    int64_t per_thread = free_pairs_ > (int64_t)kFreeThreads * 32 * ctx_->cus ? 4 : 1;
-    per_thread = std::max(per_thread, free_pairs_ / ((int64_t)kFreeThreads << 16) + 1);
+    const int64_t per_thread = free_pairs_per_thread(free_pairs_, kFreeThreads, ctx_->cus);
     const int64_t chunk = kFreeThreads * per_thread;
     for (size_t i = 0; i < rb_.size(); ++i) {
         if (!used_[i] || !rb_[i].active) continue;

@@ -1168,22 +1168,27 @@ __global__ __launch_bounds__(kFreeThreads) void k_free_turns(const BunchDev *__r
     const int64_t n = B.n, turn = B.sc->turn;
     const uint32_t t0 = (uint32_t)uni((int)(uint32_t)(B.turn_offset + turn));
     const unsigned end = (unsigned)it.begin + (unsigned)it.count;
+    const unsigned full = (unsigned)(n >> 1);   // pairs with two particles
     g_f64 *zp = (g_f64 *)B.z;
     g_f64 *ep = (g_f64 *)B.dE;
+    double2 zn = make_double2(0.0, 0.0), en = make_double2(0.0, 0.0);
+    // pair q of the item, where it has two particles
+    auto prefetch = [&](unsigned q) {
+        if (q >= min(end, full)) return;
+        zn = ldnt((const g_f64x2 *)zp + q);
+        en = ldnt((const g_f64x2 *)ep + q);
+    };
+    prefetch((unsigned)it.begin + threadIdx.x);
     for (unsigned p = (unsigned)it.begin + threadIdx.x; p < end; p += kFreeThreads) {
         const int64_t i = 2 * (int64_t)p;
-        const bool two = i + 1 < n;   // else the single particle of an odd bunch
-        double z0, z1 = 0.0, e0, e1 = 0.0;
-        if (two) {
-            const double2 zz = ldnt((const g_f64x2 *)(zp + i)), ee = ldnt((const g_f64x2 *)(ep + i));
-            z0 = zz.x;
-            z1 = zz.y;
-            e0 = ee.x;
-            e1 = ee.y;
-        } else {
+        const bool two = p < full;   // else the single particle of an odd bunch
+        double z0 = zn.x, z1 = zn.y, e0 = en.x, e1 = en.y;
+        if (!two) {
             z0 = zp[i];
             e0 = ep[i];
+            z1 = e1 = 0.0;
         }
+        prefetch(p + kFreeThreads);   // on its way during this pair's turns
         for (int t = 0; t < turns; ++t) {
             double r0 = 0.0, r1 = 0.0, d;
             if (qe) {

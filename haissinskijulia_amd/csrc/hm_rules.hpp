@@ -118,6 +118,20 @@ inline bool keeps_z(int64_t zbytes, bool interp) {
     return zbytes > (interp ? kKeepMinInterp : kKeepMin) && zbytes <= kKeepMax;
 }
 
+// Pairs per thread of k_free_turns: one until that fills the SIMDs several times
+// over, then four in turn (3e6 particles: 6 rounds of waves either way), sixteen
+// where a launch still has 32 workgroups per CU of them, and at most about 65536
+// items.  A thread's next pair is on its way during the turns of the one before:
+// a call of one turn of 1e8 particles takes 1180 to 1200 us (1257 to 1316 by a launch
+// of the pass; with four pairs per thread, each loaded when its turn came, 1200 or,
+// by the addresses of the two arrays, up to 1445); 3e7 particles, 40 turns, 4.17 ms with
+// four, 4.45 with sixteen.
+inline int64_t free_pairs_per_thread(int64_t pairs, int threads, int cus) {
+    const int64_t wave = (int64_t)threads * cus;
+    const int64_t per = pairs > 512 * wave ? 16 : pairs > 32 * wave ? 4 : 1;
+    return std::max(per, pairs / ((int64_t)threads << 16) + 1);
+}
+
 // Turns of one launch of k_free_turns over `pairs` pairs, for about 40 ms: 4e9
 // pair-turns fill the device (27 ms for 1e7 particles), and below 8e4 pairs a
 // turn takes the 0.8 us of a thread's own chain however few there are.  Bounded

@@ -18,4 +18,5 @@ int t_cached(const int64_t *n, int count) {
 }
 int t_keeps_z(int64_t zbytes, int interp) { return hm::keeps_z(zbytes, interp != 0); }
 int64_t t_free_turns(int64_t pairs) { return hm::free_turns_per_launch(pairs); }
+int64_t t_free_pairs(int64_t pairs) { return hm::free_pairs_per_thread(pairs, 256, 256); }
 }

@@ -19,6 +19,8 @@ def rules(tmp_path_factory):
     L = C.CDLL(str(out))
     L.t_max_slabs.restype = C.c_int64
     L.t_max_slabs.argtypes = [C.c_int64, C.c_int64, C.c_int]
+    L.t_free_pairs.restype = C.c_int64
+    L.t_free_pairs.argtypes = [C.c_int64]
     L.t_free_turns.restype = C.c_int64
     L.t_free_turns.argtypes = [C.c_int64]
     L.t_keeps_z.argtypes = [C.c_int64, C.c_int]
@@ -90,3 +92,12 @@ def test_free_turns_of_a_launch_stay_near_40_ms(rules, pairs):
     turns = rules.t_free_turns(pairs)
     assert turns >= 1
     assert turns == 1 or turns * max(0.8e-6, 6.8e-12 * pairs) <= 0.045
+
+
+@pytest.mark.parametrize("pairs", [1, 2_097_152, 2_097_153, 15_000_000, 33_554_432, 33_554_433, 50_000_000, 2 ** 31])
+def test_free_items(rules, pairs):
+    per = rules.t_free_pairs(pairs)
+    items = -(-pairs // (256 * per))
+    assert per == (1 if pairs <= 2_097_152 else 4 if pairs <= 33_554_432 else max(16, pairs // (256 << 16) + 1))
+    assert items <= 65536
+    assert per < 16 or items >= 32 * 256
