@@ -919,7 +919,9 @@ hm_status Batch::add_slots(const std::vector<RunBunch> &specs, std::vector<int32
         HM_TRY(w.sc.ensure(1));
         HM_TRY(w.out.ensure(16));
         HM_TRY(clears.add(w.out.p, 16 * sizeof(double)));
-        d.spread = d.ntiles >= kSpreadTiles ? ~31 : 0;
+        const int lds = ctx_->lds_max;
+        const bool global = !hist_fits(q.nbins, lds) && hist_window(q.nbins, d.npairs, d.pairs_per_tile, lds) == 0;
+        d.spread = spreads_counters(d.ntiles, q.nbins, (d.flags & F_WAKE) && global) ? ~31 : 0;
         d.nred = red_slices(d.ntiles);
         HM_TRY(w.red.ensure((size_t)d.nred * 4));
         HM_TRY(w.cnt.ensure(1));

@@ -86,6 +86,24 @@ inline int64_t max_slabs(int64_t ntiles, int64_t ppt, int cus) {
     return 2 * ntiles <= cus ? 2 * ntiles : runs;
 }
 
+// Whether the counters of a bunch leave every other 128 bytes out: additions of
+// many workgroups to few consecutive counters queue at few memory channels.  98
+// workgroups adding to 1024 counters of 8 bytes: 3.8 us back to back, 2.8 us so (an
+// empty kernel 1.6); 246 workgroups and 512 counters of 4 bytes: 6.0 and 4.2 us; no
+// difference from 16384 counters on, nor for 49 workgroups, where the bin phase,
+// which reads twice the range, loses 0.2 us.  So from kSpreadTiles tiles on; but
+// where every particle adds to global memory (global: neither form above fits), the
+// gain turns with the bins.  Pass of 3e7 particles, back to back and so, us:
+//   45000 bins 1384, 1142     65536  1194, 1139     98304  1191, 1153    104000  1322, 1146
+//   112000     1163, 1167    125000  1164, 1222    131072  1171, 1236    138000  1151, 1204
+//   150000     1160, 1169    155000  1228, 1160    160000  1216, 1162    262144  1224, 1171
+// and of 1e8, 131072 bins 3831, 4081: back to back from 110000 to 150000 bins.
+constexpr int kSpreadTiles = 32;
+constexpr int64_t kPackedMin = 110000, kPackedMax = 150000;
+inline bool spreads_counters(int64_t tiles, int64_t nb, bool global) {
+    return tiles >= kSpreadTiles && !(global && nb >= kPackedMin && nb <= kPackedMax);
+}
+
 // The particles of bunches with a windowed histogram are read and written
 // through the caches, by the pass and by the interpolation sums, where all of them
 // and 10 MB of tables a bunch fit the 256 MB of the last one: many particles

@@ -148,14 +148,8 @@ struct BunchDev {
 };
 
 // The counters that every workgroup of the pass adds to (histogram, deposit)
-// use the first 128 of every 256 bytes where the bunch has kSpreadTiles tiles or
-// more (BunchDev::spread is ~31, else 0): additions of many workgroups to few
-// consecutive counters queue at few memory channels.  98 workgroups adding to
-// 1024 counters of 8 bytes: 3.8 us back to back, 2.8 us so (an empty kernel 1.6);
-// 246 workgroups and 512 counters of 4 bytes: 6.0 and 4.2 us; no difference from
-// 16384 counters on, nor for 49 workgroups, where the bin phase, which reads
-// twice the range, loses 0.2 us.
-constexpr int kSpreadTiles = 32;
+// use the first 128 of every 256 bytes where spreads_counters says so
+// (BunchDev::spread is ~31, else 0).
 __host__ __device__ inline int spread32(int spread, int i) { return i + (i & spread); }
 __host__ __device__ inline int spread64(int spread, int i) { return i + (i & (spread >> 1)); }
 // 32-bit words of one half of a histogram, 64-bit words of a deposit's hi or lo

@@ -11,6 +11,7 @@ int t_hist_form(int64_t nb, int64_t ntiles, int64_t npairs, int64_t ppt, int lds
     return hm::hist_fits(nb, lds) ? -1 : 0;
 }
 int64_t t_pairs_per_tile(int64_t npairs, int tile_pairs) { return hm::pairs_per_tile_for(npairs, 1024, tile_pairs); }
+int t_spreads(int64_t tiles, int64_t nb, int global) { return hm::spreads_counters(tiles, nb, global != 0); }
 int t_cached(const int64_t *n, int count) {
     int64_t bytes = 0;
     for (int i = 0; i < count; ++i) bytes += hm::cached_bytes(n[i]);

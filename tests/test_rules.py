@@ -71,6 +71,15 @@ def test_histogram_form(rules, n, tile_pairs, windowed):
     assert [form(nb) for nb in (40701, 49152, 131073)] == ([40700, 49152, 49152] if can else [0, 0, 0])
 
 
+@pytest.mark.parametrize("tiles,nb,everywhere,in_lds", [
+    (31, 1024, 0, 0), (32, 1024, 1, 1), (100, 109_999, 1, 1), (100, 110_000, 0, 1), (100, 131_072, 0, 1),
+    (100, 150_000, 0, 1), (100, 150_001, 1, 1), (31, 150_001, 0, 0)])
+def test_where_counters_leave_gaps(rules, tiles, nb, everywhere, in_lds):
+    L = rules.t_spreads
+    L.argtypes = [C.c_int64, C.c_int64, C.c_int]
+    assert (L(tiles, nb, 1), L(tiles, nb, 0)) == (everywhere, in_lds)
+
+
 def test_cached_particles_fit_the_last_cache_together(rules):
     def cached(*n):
         return bool(rules.t_cached((C.c_int64 * len(n))(*n), len(n)))
